@@ -133,12 +133,21 @@ size_t fa_decode_workspace_bytes(int batch, int heads_q, int seqlen_q, int head_
   return fa::decode_workspace_bytes(batch, heads_q, seqlen_q, head_dim, num_splits);
 }
 
-int fa_fwd(const fa_fwd_params* params, void* stream) {
+size_t fa_fwd_workspace_bytes(const fa_fwd_params* params) {
+  if (!params) return 0;
+  return fa::fwd_workspace_bytes(*params);
+}
+
+int fa_fwd_ws(const fa_fwd_params* params, void* workspace, size_t workspace_bytes, void* stream) {
   if (!params) return fail(FA_ERR_INVALID, "fa_fwd: params is NULL");
   int rc = check_fwd(*params, "fa_fwd");
   if (rc) return rc;
-  return from_hip(fa::launch_fwd(*params, (hipStream_t)stream), "fa_fwd");
+  if (workspace && !aligned16(workspace)) return fail(FA_ERR_INVALID, "fa_fwd: workspace must be 16-byte aligned");
+  const fa::FwdScratch w{workspace, (int64_t)workspace_bytes};
+  return from_hip(fa::launch_fwd(*params, w, (hipStream_t)stream), "fa_fwd");
 }
+
+int fa_fwd(const fa_fwd_params* params, void* stream) { return fa_fwd_ws(params, nullptr, 0, stream); }
 
 static int bwd_common(const fa_bwd_params* params, int phases, void* stream) {
   if (!params) return fail(FA_ERR_INVALID, "fa_bwd: params is NULL");

@@ -1,4 +1,4 @@
-// fa_fwd16.hpp - forward kernel specialised for 16-bit inputs and D <= 128.
+// fa_fwd16.hpp - forward kernel specialised for 16-bit inputs.
 //
 // Same algorithm and results as fwd_kernel (exp2 online softmax,
 // LSE = m*ln2 + ln l; reference kernels/forward.py:28-164 and
@@ -32,6 +32,11 @@ namespace fa {
 // a heavy causal block runs at full CU throughput instead of sharing the CU
 // with a light one and then running alone.
 //
+// D > 128 runs NH = 1 only, one workgroup per CU: O^T, Q and the scores of 32
+// rows take up to 400 registers, so a SIMD holds one wave.  What bounds it is
+// LDS operand reads, one per MFMA as in the narrower forms, and the softmax
+// that no second wave covers.
+//
 // NH = 1 is the same kernel with one key half: 4 waves walk all key tiles of
 // the 128 rows and no merge is needed.  Its 64 KiB of LDS and 4 waves let two
 // workgroups share a CU, so one workgroup's prologue (Q and first tiles) and
@@ -46,29 +51,50 @@ struct Fwd16Cfg {
   static constexpr int NT = 64 * NW;
   static constexpr int NTH = 64 * NQ;          // threads per key half
   static constexpr int BM = 32 * NQ;
-  static constexpr int BN = 64;
-  static constexpr int KTILE = BN * D;  // elements (K), then V
-  static constexpr int STAGE = 2 * KTILE;
+  static constexpr int BN = D <= 128 ? 64 : 32;  // D = 256: a 64-key stage pair would exceed the LDS
+  // Output columns per workgroup: D = 512 splits O^T in two over the grid.
+  static constexpr int DO = D <= 256 ? D : 256;
+  static constexpr int NDC = D / DO;
+  static constexpr int KTILE = BN * D;   // elements (K), then V
+  static constexpr int VTILE = BN * DO;
+  static constexpr int STAGE = KTILE + VTILE;
   static constexpr int HALF = 2 * STAGE;       // two stages per key half
-  static constexpr int MERGE_BYTES = NH == 1 ? 0 : NQ * (D / 32) * 16 * 64 * 4 + 2 * NQ * 64 * 4;
+  static constexpr int MERGE_BYTES = NH == 1 ? 0 : NQ * (DO / 32) * 16 * 64 * 4 + 2 * NQ * 64 * 4;
   static constexpr int LOOP_BYTES = NH * HALF * 2;
-  static constexpr int LDS_BYTES = LOOP_BYTES > MERGE_BYTES ? LOOP_BYTES : MERGE_BYTES;
+  // A wave's rows on their way out (store_rows_staged): NH = 1 packs the four
+  // waves' areas, NH = 2 uses the block its merge partner parked into.
+  static constexpr int OUT_WAVE_BYTES = NH == 1 ? 32 * (DO + 8) * 2 : (DO / 32) * 4096;
+  static constexpr int OUT_BYTES = NQ * OUT_WAVE_BYTES;
+  static constexpr int LDS_BYTES = LOOP_BYTES > MERGE_BYTES ? (LOOP_BYTES > OUT_BYTES ? LOOP_BYTES : OUT_BYTES)
+                                                            : (MERGE_BYTES > OUT_BYTES ? MERGE_BYTES : OUT_BYTES);
   static constexpr int NSTEP = D / 16;
   static constexpr int NKB = BN / 32;
   static constexpr int NPV = BN / 16;
-  static constexpr int NDB = D / 32;
+  static constexpr int NDB = DO / 32;
+  // One partial of the key-split form: the four waves' O^T accumulators as
+  // park_acc leaves them, then m and l of the 128 rows (floats).
+  static constexpr int PART_O = NQ * NDB * 1024;
+  static constexpr int PART = PART_O + 2 * BM;
 };
 
 // Largest growth of the running max (log2 domain) absorbed without rescaling.
-constexpr float kLazyRescale = 8.0f;
+// Wide heads follow the max exactly: the largest weights are then 1 or just
+// below it, where a 16-bit float rounds least (measured output error at
+// D = 512 fp16: 2.85e-4 of the norm against 2.93e-4 with a lazy max).
+template <int D>
+constexpr float kLazyRescale = D <= 128 ? 8.0f : 0.0f;
 
 // One work item: the 128 query rows of row block (num_m_blocks - 1 - mb_rev)
-// of (batch, head) bh, item = mb_rev * B * Hq + bh.  `end_barrier`: the
+// of (batch, head) bh, output columns [dc * DO, (dc + 1) * DO),
+// item = (mb_rev * B * Hq + bh) * NDC + dc.  `end_barrier`: the
 // workgroup runs another item after this one, so every wave passes a
 // barrier once this item's LDS use (merge, staged stores) is over.
-template <typename Tag, int D, int MODE, int NH>
+// SPLIT: the item covers share `split` of `nsplit` of the block's key tiles
+// and leaves its unnormalised state in `part` for fwd16_merge_kernel.
+template <typename Tag, int D, int MODE, int NH, bool SPLIT = false>
 __device__ __forceinline__ void fwd16_item(const fa_fwd_params& p, int num_m_blocks, int item,
-                                           unsigned char* smem_raw, bool end_barrier) {
+                                           unsigned char* smem_raw, bool end_barrier, int split = 0,
+                                           int nsplit = 1, float* part = nullptr) {
   using C = Fwd16Cfg<D, NH>;
   using EL = Elem<Tag>;
   using S = uint16_t;
@@ -82,8 +108,9 @@ __device__ __forceinline__ void fwd16_item(const fa_fwd_params& p, int num_m_blo
   const int h = lane >> 5, l32 = lane & 31;
 
   const int bh_count = p.batch * p.heads_q;
-  const int mb_rev = item / bh_count;
-  const int bh = item - mb_rev * bh_count;
+  const int dc = item % C::NDC;
+  const int mb_rev = item / C::NDC / bh_count;
+  const int bh = item / C::NDC - mb_rev * bh_count;
   const int b = bh / p.heads_q, hq = bh - b * p.heads_q;
   const int hk = hq / (p.heads_q / p.heads_kv);
   const int mblk = num_m_blocks - 1 - mb_rev;  // heaviest causal blocks first
@@ -101,7 +128,7 @@ __device__ __forceinline__ void fwd16_item(const fa_fwd_params& p, int num_m_blo
   const S* kb = reinterpret_cast<const S*>(p.k) + b * p.k_stride[0] + hk * p.k_stride[1] +
                 (int64_t)k_start * p.k_stride[2];
   const S* vb = reinterpret_cast<const S*>(p.v) + b * p.v_stride[0] + hk * p.v_stride[1] +
-                (int64_t)k_start * p.v_stride[2];
+                (int64_t)k_start * p.v_stride[2] + dc * C::DO;
   const int64_t qs = p.q_stride[2], ks = p.k_stride[2], vs = p.v_stride[2];
   const Mods md = make_mods(p, b, hq, sq, sk);
   const float c = md.scale_log2;
@@ -112,7 +139,12 @@ __device__ __forceinline__ void fwd16_item(const fa_fwd_params& p, int num_m_blo
   if (p.window_right >= 0) hi = min(hi, mlast + md.off + p.window_right + 1);
   if (p.window_left >= 0) lo = max(0, m0 + md.off - p.window_left);
   lo = lo / C::BN * C::BN;
-  const int ntiles = hi > lo ? (hi - lo + C::BN - 1) / C::BN : 0;
+  int ntiles = hi > lo ? (hi - lo + C::BN - 1) / C::BN : 0;
+  if constexpr (SPLIT) {
+    const int t0 = ntiles * split / nsplit;
+    ntiles = ntiles * (split + 1) / nsplit - t0;
+    lo += t0 * C::BN;
+  }
 
   const int m0w = m0 + 32 * wave;
   const int mrows = min(32, sq - m0w);
@@ -126,7 +158,8 @@ __device__ __forceinline__ void fwd16_item(const fa_fwd_params& p, int num_m_blo
 #pragma unroll
   for (int i = 0; i < C::NDB; ++i) acc[i] = zero16();
 
-  DmaSwzTile<C::BN, D, C::NTH> kt, vt;
+  DmaSwzTile<C::BN, D, C::NTH> kt;
+  DmaSwzTile<C::BN, C::DO, C::NTH> vt;
   kt.init(ks, htid);
   vt.init(vs, htid);
   // Both halves run nh0 steps so their barriers line up.
@@ -146,7 +179,7 @@ __device__ __forceinline__ void fwd16_item(const fa_fwd_params& p, int num_m_blo
     const int rows = min(C::BN, sk - n_next);
     const uint32_t base = lds0 + (uint32_t)(stage * C::STAGE) * 2u;
     kt.load(rows_rsrc_words<D>(k_next, ks, rows), base, wave);
-    vt.load(rows_rsrc_words<D>(v_next, vs, rows), base + C::KTILE * 2u, wave);
+    vt.load(rows_rsrc_words<C::DO>(v_next, vs, rows), base + C::KTILE * 2u, wave);
     n_next += TSTEP * C::BN;
     k_next += (int64_t)(TSTEP * C::BN) * ks;
     v_next += (int64_t)(TSTEP * C::BN) * vs;
@@ -251,7 +284,7 @@ __device__ __forceinline__ void fwd16_item(const fa_fwd_params& p, int num_m_blo
       }
       tmax = half_max(tmax);
       // Lazy rescale, decided for the whole wave.
-      if (__builtin_amdgcn_ballot_w64(tmax > m_i + kLazyRescale)) {
+      if (__builtin_amdgcn_ballot_w64(tmax > m_i + kLazyRescale<D>)) {
         const float m_new = fmaxf(m_i, tmax);
         const float alpha = (m_new == kNegInf) ? 1.f : __builtin_amdgcn_exp2f(m_i - m_new);
         l_i *= alpha;
@@ -321,7 +354,7 @@ __device__ __forceinline__ void fwd16_item(const fa_fwd_params& p, int num_m_blo
       for (int j = 0; j < C::NPV; ++j)
 #pragma unroll
         for (int db = 0; db < C::NDB; ++db) {
-          const s16x8 a = tr_op_rowmap<D>(Vs, 0, 32 * db, j, lane);
+          const s16x8 a = tr_op_rowmap<C::DO>(Vs, 0, 32 * db, j, lane);
           acc[db] = EL::mma(a, pb[j], acc[db]);
           if constexpr (PSPLIT) acc[db] = EL::mma(a, pl[j], acc[db]);
         }
@@ -363,16 +396,27 @@ __device__ __forceinline__ void fwd16_item(const fa_fwd_params& p, int num_m_blo
     m_i = mn;
   }
 
+  if constexpr (SPLIT) {
+    static_assert(NH == 1, "one key half per share");
+#pragma unroll
+    for (int db = 0; db < C::NDB; ++db) park_acc(part + (wave * C::NDB + db) * 1024, lane, acc[db]);
+    if (h == 0) {
+      part[C::PART_O + 32 * wave + l32] = m_i;
+      part[C::PART_O + C::BM + 32 * wave + l32] = l_i;
+    }
+    return;
+  }
+
   const float l_safe = (l_i == 0.f) ? 1.f : l_i;
   const float inv = 1.f / l_safe;
   // Whole-row output stores through this wave's LDS block: with NH = 2 the
   // block this wave's merge partner parked into (read above), with NH = 1 a
   // stage buffer (every tile read ended at the loop's last barrier).
   S* orow0 = reinterpret_cast<S*>(p.out) + b * p.out_stride[0] + hq * p.out_stride[1] +
-             (int64_t)(q_start + m0w) * p.out_stride[2];
-  store_rows_staged<Tag, D>(acc, inv, reinterpret_cast<uint16_t*>(smem_raw + wave * C::NDB * 4096), orow0,
+             (int64_t)(q_start + m0w) * p.out_stride[2] + dc * C::DO;
+  store_rows_staged<Tag, C::DO>(acc, inv, reinterpret_cast<uint16_t*>(smem_raw + wave * C::OUT_WAVE_BYTES), orow0,
                             p.out_stride[2], mrows, lane);
-  if (mvalid && h == 0) {
+  if (mvalid && h == 0 && dc == 0) {
     float* lb = p.lse + b * p.lse_stride[0] + hq * p.lse_stride[1] + (int64_t)(q_start + m) * p.lse_stride[2];
     *lb = (m_i == kNegInf || l_i == 0.f) ? kNegInf : (m_i + __log2f(l_safe)) * kLn2;
   }
@@ -384,7 +428,7 @@ __device__ __forceinline__ void fwd16_item(const fa_fwd_params& p, int num_m_blo
 // masking the two carry the same number of key tiles together, and both
 // read the same head's K / V, which the workgroup's XCD then holds in L2.
 template <typename Tag, int D, int MODE, int NH, bool PAIR>
-__global__ __launch_bounds__(256 * NH, 3 - NH) void fwd16_kernel(fa_fwd_params p, int num_m_blocks) {
+__global__ __launch_bounds__(256 * NH, D > 128 ? 1 : 3 - NH) void fwd16_kernel(fa_fwd_params p, int num_m_blocks) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   if constexpr (!PAIR) {
     fwd16_item<Tag, D, MODE, NH>(p, num_m_blocks, blockIdx.x, smem_raw, false);
@@ -396,6 +440,70 @@ __global__ __launch_bounds__(256 * NH, 3 - NH) void fwd16_kernel(fa_fwd_params p
     fwd16_item<Tag, D, MODE, NH>(p, num_m_blocks, j * bh_count + bh, smem_raw, j2 != j);
     if (j2 != j) fwd16_item<Tag, D, MODE, NH>(p, num_m_blocks, j2 * bh_count + bh, smem_raw, false);
   }
+}
+
+// Few wide row blocks: each block's key tiles shared out over nsplit
+// workgroups (blockIdx = item * nsplit + split).  The shares' states are fp32
+// and unnormalised, so the merge loses nothing against one workgroup.
+template <typename Tag, int D, int MODE>
+__global__ __launch_bounds__(256, D > 128 ? 1 : 2) void fwd16_split_kernel(fa_fwd_params p, int num_m_blocks,
+                                                                           int nsplit, float* ws) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  const int item = blockIdx.x / nsplit;
+  fwd16_item<Tag, D, MODE, 1, true>(p, num_m_blocks, item, smem_raw, false, blockIdx.x - item * nsplit, nsplit,
+                                    ws + (int64_t)blockIdx.x * Fwd16Cfg<D, 1>::PART);
+}
+
+// Merge of fwd16_split_kernel's shares, 64 output columns of one row block
+// per workgroup: O = sum_s 2^(m_s - M) O_s / sum_s 2^(m_s - M) l_s in the
+// accumulator layout the shares were parked in (1 KiB per load), then whole
+// 128-byte row pieces through LDS.
+template <typename Tag, int D>
+__global__ __launch_bounds__(256) void fwd16_merge_kernel(fa_fwd_params p, int num_m_blocks, int nsplit,
+                                                          const float* ws) {
+  using C = Fwd16Cfg<D, 1>;
+  using S = uint16_t;
+  constexpr int MD = 64;  // columns per workgroup
+  constexpr int PER = C::DO / MD;
+  __shared__ __align__(16) uint16_t stage[C::NQ * 32 * (MD + 8)];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int h = lane >> 5, l32 = lane & 31;
+  const int cc = blockIdx.x % PER;
+  const int item = blockIdx.x / PER;
+  const int dc = item % C::NDC;
+  const int bh_count = p.batch * p.heads_q;
+  const int mb_rev = item / C::NDC / bh_count;
+  const int bh = item / C::NDC - mb_rev * bh_count;
+  const int b = bh / p.heads_q, hq = bh - b * p.heads_q;
+  const int m0w = (num_m_blocks - 1 - mb_rev) * C::BM + 32 * wave;
+  const int mrows = min(32, p.seqlen_q - m0w);
+  const float* src = ws + (int64_t)item * nsplit * C::PART;
+  float M = kNegInf;
+  for (int s = 0; s < nsplit; ++s) M = fmaxf(M, src[(int64_t)s * C::PART + C::PART_O + 32 * wave + l32]);
+  const float Mu = (M == kNegInf) ? 0.f : M;
+  float L = 0.f;
+  f32x16 acc[MD / 32];
+#pragma unroll
+  for (int i = 0; i < MD / 32; ++i) acc[i] = zero16();
+  for (int s = 0; s < nsplit; ++s) {
+    const float* ps = src + (int64_t)s * C::PART;
+    const float w = __builtin_amdgcn_exp2f(ps[C::PART_O + 32 * wave + l32] - Mu);
+    L += ps[C::PART_O + C::BM + 32 * wave + l32] * w;
+#pragma unroll
+    for (int i = 0; i < MD / 32; ++i) {
+      const f32x16 o = unpark_acc(ps + (wave * C::NDB + cc * (MD / 32) + i) * 1024, lane);
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][e] += o[e] * w;
+    }
+  }
+  const float l_safe = (L == 0.f) ? 1.f : L;
+  S* orow0 = reinterpret_cast<S*>(p.out) + b * p.out_stride[0] + hq * p.out_stride[1] +
+             (int64_t)m0w * p.out_stride[2] + dc * C::DO + cc * MD;
+  store_rows_staged<Tag, MD>(acc, 1.f / l_safe, stage + wave * 32 * (MD + 8), orow0, p.out_stride[2], mrows, lane);
+  if (l32 < mrows && h == 0 && dc == 0 && cc == 0)
+    p.lse[b * p.lse_stride[0] + hq * p.lse_stride[1] + (int64_t)(m0w + l32) * p.lse_stride[2]] =
+        (M == kNegInf || L == 0.f) ? kNegInf : (M + __log2f(l_safe)) * kLn2;
 }
 
 }  // namespace fa

@@ -2,5 +2,5 @@
 #include "fa_fwd_impl.hpp"
 
 namespace fa {
-template hipError_t fwd_by_mods<bf16_t>(const fa_fwd_params& p, hipStream_t s);
+template hipError_t fwd_by_mods<bf16_t>(const fa_fwd_params& p, const FwdScratch& w, hipStream_t s);
 }  // namespace fa

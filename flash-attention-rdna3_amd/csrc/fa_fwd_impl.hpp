@@ -284,7 +284,40 @@ static hipError_t launch_fwd16(const fa_fwd_params& p, long grid, int nmb, hipSt
 }
 
 template <typename Tag, int D, int MODE>
-static hipError_t run_fwd(const fa_fwd_params& p, hipStream_t stream) {
+static hipError_t launch_fwd16_split(const fa_fwd_params& p, int nmb, int nsplit, float* ws, hipStream_t stream) {
+  using C = Fwd16Cfg<D, 1>;
+  auto kern = fwd16_split_kernel<Tag, D, MODE>;
+  hipError_t e = allow_lds((const void*)kern, C::LDS_BYTES);
+  if (e != hipSuccess) return e;
+  const unsigned items = (unsigned)(nmb * p.batch * p.heads_q * C::NDC);
+  hipLaunchKernelGGL(kern, dim3(items * nsplit), dim3(C::NT), C::LDS_BYTES, stream, p, nmb, nsplit, ws);
+  e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL((fwd16_merge_kernel<Tag, D>), dim3(items * (C::DO / 64)), dim3(256), 0, stream, p, nmb, nsplit,
+                     (const float*)ws);
+  return hipGetLastError();
+}
+
+template <typename Tag, int D, int MODE>
+static hipError_t run_fwd(const fa_fwd_params& p, const FwdScratch& scratch, hipStream_t stream) {
+  if constexpr (!std::is_same<Tag, f32_t>::value && D > 128) {
+    // Wide heads: one wave per SIMD with all 512 registers (O^T of 32 rows
+    // takes 128 of them, Q 64 to 128; at two waves per SIMD the D = 256 form
+    // spilled 38), one key half.  Measured against fwd_kernel (O^T split two
+    // to four ways over the grid, scores recomputed for each):
+    // D = 256 bf16 causal, 1 x 16 x 2048 (34 GFLOP): 207 -> 115 us;
+    // D = 512 fp16, 1 x 1 x 4096 (34 GFLOP), with key splits: 787 -> 92 us
+    // (shares 79, merge 13; 52 GFLOP with the scores of both column halves).
+    using C = Fwd16Cfg<D, 1>;
+    if (buf_rows_ok(p.k_stride[2], C::BN) && buf_rows_ok(p.v_stride[2], C::BN)) {
+      const int nmb = (p.seqlen_q + C::BM - 1) / C::BM;
+      const long grid = (long)nmb * p.batch * p.heads_q * C::NDC;
+      const int nsplit = fwd_split_count(p);
+      if (nsplit > 1 && scratch.ptr && scratch.bytes >= (int64_t)fwd_workspace_bytes(p))
+        return launch_fwd16_split<Tag, D, MODE>(p, nmb, nsplit, static_cast<float*>(scratch.ptr), stream);
+      return launch_fwd16<Tag, D, MODE, 1>(p, grid, nmb, stream);
+    }
+  }
   if constexpr (!std::is_same<Tag, f32_t>::value && D <= 128) {
     using C = Fwd16Cfg<D>;
     if (buf_rows_ok(p.k_stride[2], C::BN) && buf_rows_ok(p.v_stride[2], C::BN)) {
@@ -320,26 +353,26 @@ static hipError_t run_fwd(const fa_fwd_params& p, hipStream_t stream) {
 }
 
 template <typename Tag, int MODE>
-static hipError_t fwd_by_dim(const fa_fwd_params& p, hipStream_t s) {
+static hipError_t fwd_by_dim(const fa_fwd_params& p, const FwdScratch& w, hipStream_t s) {
   switch (p.head_dim) {
-    case 32: return run_fwd<Tag, 32, MODE>(p, s);
-    case 64: return run_fwd<Tag, 64, MODE>(p, s);
-    case 128: return run_fwd<Tag, 128, MODE>(p, s);
-    case 256: return run_fwd<Tag, 256, MODE>(p, s);
-    case 512: return run_fwd<Tag, 512, MODE>(p, s);
+    case 32: return run_fwd<Tag, 32, MODE>(p, w, s);
+    case 64: return run_fwd<Tag, 64, MODE>(p, w, s);
+    case 128: return run_fwd<Tag, 128, MODE>(p, w, s);
+    case 256: return run_fwd<Tag, 256, MODE>(p, w, s);
+    case 512: return run_fwd<Tag, 512, MODE>(p, w, s);
   }
   return hipErrorInvalidValue;
 }
 
 template <typename Tag>
-hipError_t fwd_by_mods(const fa_fwd_params& p, hipStream_t s) {
+hipError_t fwd_by_mods(const fa_fwd_params& p, const FwdScratch& w, hipStream_t s) {
   // 0: plain, 1: softcap / bias / ALiBi, 2: also dropout (Philox per score),
   // 3: softcap without bias or ALiBi (16-bit kernels; one score variant).
-  if (p.dropout_p > 0.f) return fwd_by_dim<Tag, 2>(p, s);
+  if (p.dropout_p > 0.f) return fwd_by_dim<Tag, 2>(p, w, s);
   if constexpr (!std::is_same<Tag, f32_t>::value)
-    if (p.softcap > 0.f && !p.bias && !p.alibi_slopes) return fwd_by_dim<Tag, 3>(p, s);
-  if (p.softcap > 0.f || p.bias || p.alibi_slopes) return fwd_by_dim<Tag, 1>(p, s);
-  return fwd_by_dim<Tag, 0>(p, s);
+    if (p.softcap > 0.f && !p.bias && !p.alibi_slopes) return fwd_by_dim<Tag, 3>(p, w, s);
+  if (p.softcap > 0.f || p.bias || p.alibi_slopes) return fwd_by_dim<Tag, 1>(p, w, s);
+  return fwd_by_dim<Tag, 0>(p, w, s);
 }
 
 }  // namespace fa

@@ -1,6 +1,8 @@
 // fa_internal.hpp - host-side launchers behind the C ABI (fa_api.cpp).
 #pragma once
 
+#include <algorithm>
+
 #include <hip/hip_runtime.h>
 
 #include "../../include/fa_mi355x.h"
@@ -13,11 +15,21 @@ inline bool buf_rows_ok(int64_t stride_elems, int rows) {
   return stride_elems >= 0 && stride_elems * 2 * (int64_t)rows < (int64_t(1) << 31);
 }
 
+// Optional caller memory of a forward (fa_fwd_ws); ptr NULL: none.
+struct FwdScratch {
+  void* ptr;
+  int64_t bytes;
+};
+// Workgroups that share a row block's keys (1: none), and the scratch their
+// states take.
+int fwd_split_count(const fa_fwd_params& p);
+size_t fwd_workspace_bytes(const fa_fwd_params& p);
+
 // Each launcher validates nothing beyond what it needs to pick a kernel
 // instantiation; fa_api.cpp has already checked the arguments.  They return
 // hipSuccess, hipErrorInvalidValue for an unsupported configuration, or the
 // launch error.
-hipError_t launch_fwd(const fa_fwd_params& p, hipStream_t stream);
+hipError_t launch_fwd(const fa_fwd_params& p, const FwdScratch& w, hipStream_t stream);
 // phases: bit 0 delta, bit 1 dK/dV, bit 2 dQ.
 hipError_t launch_bwd(const fa_bwd_params& p, int phases, hipStream_t stream);
 hipError_t launch_decode(const fa_decode_params& p, hipStream_t stream);

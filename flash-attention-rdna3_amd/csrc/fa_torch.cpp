@@ -192,7 +192,10 @@ std::tuple<Tensor, Tensor> forward_impl(const Tensor& query, const Tensor& key, 
   Tensor lse = at::empty({q.size(0), q.size(1), q.size(2)}, query.options().dtype(at::kFloat));
   fa_fwd_params p;
   const Extras ex = fill_fwd(p, q, k, v, out, lse, o);
-  check_status(fa_fwd(&p, stream_of(query)), "fa_fwd");
+  Tensor ws;
+  const size_t bytes = fa_fwd_workspace_bytes(&p);
+  if (bytes > 0) ws = at::empty({(int64_t)bytes}, query.options().dtype(at::kByte));
+  check_status(fa_fwd_ws(&p, bytes > 0 ? ws.data_ptr() : nullptr, bytes, stream_of(query)), "fa_fwd");
   if (kdim != head_dim) out = out.narrow(-1, 0, head_dim).contiguous();
   return {out, lse};
 }

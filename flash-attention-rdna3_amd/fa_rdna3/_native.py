@@ -125,7 +125,7 @@ _STRUCTS = (FwdParams, BwdParams, DecodeParams, PagedParams, TinyParams, AppendP
 EXPORTS = (
     "fa_abi_version", "fa_last_error_string", "fa_params_size", "fa_decode_workspace_bytes",
     "fa_decode_ticket_count",
-    "fa_fwd", "fa_bwd", "fa_bwd_phase", "fa_bwd_workspace_bytes", "fa_bwd_workspace_min_bytes", "fa_decode_splitk", "fa_decode_splitk_noalloc", "fa_decode_paged",
+    "fa_fwd", "fa_fwd_ws", "fa_fwd_workspace_bytes", "fa_bwd", "fa_bwd_phase", "fa_bwd_workspace_bytes", "fa_bwd_workspace_min_bytes", "fa_decode_splitk", "fa_decode_splitk_noalloc", "fa_decode_paged",
     "fa_tiny_fwd_f32",
     "fa_kvcache_append",
     "fa_hbm_read_probe_count", "fa_hbm_read_probe_name", "fa_hbm_read_probe",
@@ -159,6 +159,10 @@ def lib():
         handle.fa_params_size.argtypes = [ctypes.c_int]
         handle.fa_decode_workspace_bytes.restype = ctypes.c_size_t
         handle.fa_decode_workspace_bytes.argtypes = [ctypes.c_int] * 5
+        handle.fa_fwd_ws.restype = ctypes.c_int
+        handle.fa_fwd_ws.argtypes = [ctypes.POINTER(FwdParams), ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]
+        handle.fa_fwd_workspace_bytes.restype = ctypes.c_size_t
+        handle.fa_fwd_workspace_bytes.argtypes = [ctypes.c_void_p]
         handle.fa_bwd_workspace_bytes.restype = ctypes.c_size_t
         handle.fa_bwd_workspace_bytes.argtypes = [ctypes.c_void_p]
         handle.fa_bwd_workspace_min_bytes.restype = ctypes.c_size_t

@@ -313,6 +313,16 @@ size_t fa_decode_workspace_bytes(int batch, int heads_q, int seqlen_q,
                                  int head_dim, int num_splits);
 
 int fa_fwd(const fa_fwd_params* params, void* stream);
+/* fa_fwd with caller scratch (no counterpart in the reference): with at least
+ * fa_fwd_workspace_bytes(params) bytes, 16-byte aligned, a forward whose row
+ * blocks would leave most compute units idle shares each block's keys out
+ * over several workgroups and merges their fp32 states.  NULL or less: one
+ * workgroup per row block, as fa_fwd.  Results agree to the rounding of the
+ * accumulation order. */
+int fa_fwd_ws(const fa_fwd_params* params, void* workspace, size_t workspace_bytes, void* stream);
+/* Scratch fa_fwd_ws can use (0: none; it depends on the current device's
+ * compute unit count). */
+size_t fa_fwd_workspace_bytes(const fa_fwd_params* params);
 int fa_bwd(const fa_bwd_params* params, void* stream);
 /* One stage of fa_bwd: 0 = delta, 1 = dK/dV, 2 = dQ (1 and 2 read delta).
  * No counterpart in the reference (its three backward launches are separate
@@ -324,8 +334,8 @@ int fa_bwd(const fa_bwd_params* params, void* stream);
  * between cannot be detected). */
 int fa_bwd_phase(const fa_bwd_params* params, int phase, void* stream);
 /* Bytes of ds_workspace the backward of `params` can use (0: the dS path
- * does not apply: fp32, head_dim other than 64 or 128, or more than 512
- * varlen sequences).
+ * does not apply: fp32, head_dim other than 64, 128 or (dense) 256, or more
+ * than 512 varlen sequences).
  * Dense: batch * heads_q * ceil(Sk / 64) * ceil(Sq / 128) * 16 KiB plus
  * 1 KiB; varlen, an upper bound from max_seqlen_k, total_q and batch.  With dS scratch, phase 2 of
  * fa_bwd_phase reads the dS that phase 1 stored. */

@@ -1,0 +1,97 @@
+"""16-bit forward at head dims 256 and 512 (one wave per SIMD, key splits)
+against 64-bit attention, at tile edges, splits and modifiers."""
+
+import ctypes
+import math
+
+import pytest
+import torch
+
+from attn_refs import attention
+from fa_rdna3 import _native, flash_attention
+from fa_rdna3.interface import _fwd_params
+
+pytestmark = pytest.mark.gpu
+# Largest relative 2-norm error: four roundings to the 16-bit type lie on any
+# result's path (P or dS, out in delta, the operand products' inputs are
+# exact, the result), each at most one unit 2^-11 / 2^-8 of what it rounds.
+BOUND = {torch.float16: 4 * 2.0 ** -11, torch.bfloat16: 4 * 2.0 ** -8}
+
+
+def _rand(shape, dtype, gen):
+    return torch.randn(shape, generator=gen).to(dtype).cuda()
+
+
+def _close(got, want, dtype):
+    want = want.double()
+    assert torch.isfinite(got).all()
+    err = (got.double() - want).norm() / want.norm().clamp_min(1e-30)
+    assert err <= BOUND[dtype], float(err)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("head_dim", [256, 512])
+@pytest.mark.parametrize("sq,sk,opts", [
+    (1, 1, {}), (33, 31, {"causal": True}), (127, 129, {}), (128, 128, {"causal": True}),
+    (129, 1024, {}), (700, 700, {"causal": True, "window": (200, 0)}), (300, 2000, {"softcap": 20.0}),
+    (257, 1500, {"scale": 0.0}), (64, 640, {"causal": True, "softcap": 5.0}),
+])
+def test_forward(dtype, head_dim, sq, sk, opts):
+    gen = torch.Generator().manual_seed(sq * 7 + sk)
+    q = _rand((2, sq, 2, head_dim), dtype, gen).transpose(1, 2)  # heads within a row
+    k, v = (_rand((2, 1, sk, head_dim), dtype, gen) for _ in range(2))
+    opts = dict(opts)
+    window, scale = opts.pop("window", (-1, -1)), opts.pop("scale", None)
+    out = flash_attention(q, k, v, softmax_scale=scale, window_size=window, **opts)
+    ref = attention(q.double(), k.double(), v.double(), scale=scale, window=window, **opts)
+    _close(out, ref, dtype)
+
+
+@pytest.mark.parametrize("head_dim", [256, 512])
+@pytest.mark.parametrize("hidden", ["none", "row", "share"])
+def test_key_splits_agree_with_one_workgroup(head_dim, hidden):
+    """fa_fwd_ws with and without its scratch, output and LSE; a row that sees
+    no key at all, and one whose first share of the keys is hidden."""
+    gen = torch.Generator().manual_seed(5)
+    dtype, sq, sk = torch.float16, 150, 1100
+    q, k, v = (_rand((1, 1, n, head_dim), dtype, gen) for n in (sq, sk, sk))
+    bias = torch.zeros((1, 1, sq, sk), device="cuda")
+    if hidden == "row":
+        bias[:, :, 7] = float("-inf")
+    elif hidden == "share":
+        bias[:, :, 7, :600] = float("-inf")
+    lib, got = _native.lib(), []
+    for split in (True, False):
+        out = torch.full((1, 1, sq, head_dim), float("nan"), device="cuda", dtype=dtype)
+        lse = torch.full((1, 1, sq), float("nan"), device="cuda")
+        p = _fwd_params(q, k, v, out, lse, dense=True, causal=False, softmax_scale=1 / math.sqrt(head_dim),
+                        window=(-1, -1), softcap=0.0, bias=bias, alibi=None, dropout_p=0.0, dropout_seed=0)
+        need = lib.fa_fwd_workspace_bytes(ctypes.byref(p))
+        assert need > 0
+        ws = torch.empty(need if split else 0, dtype=torch.uint8, device="cuda")
+        rc = lib.fa_fwd_ws(ctypes.byref(p), ws.data_ptr() if split else None, need if split else 0,
+                           torch.cuda.current_stream().cuda_stream)
+        assert rc == 0, lib.fa_last_error_string()
+        got.append((out, lse))
+    ref = attention(q.double(), k.double(), v.double(), bias=bias.double())
+    for out, lse in got:
+        _close(out, ref, dtype)
+        if hidden == "row":
+            assert (out[:, :, 7] == 0).all() and lse[0, 0, 7] == float("-inf")
+    finite = torch.isfinite(got[0][1])
+    assert torch.equal(finite, torch.isfinite(got[1][1]))
+    # fp32 sums of at most 1100 terms taken in another order
+    assert (got[0][1] - got[1][1])[finite].abs().max() <= 1100 * 2.0 ** -24 * 8
+
+
+def test_no_splits_without_room_to_gain():
+    p = _native.FwdParams()
+    p.dtype, p.head_dim, p.batch, p.heads_q, p.heads_kv, p.seqlen_q, p.seqlen_k = 0, 256, 1, 16, 16, 2048, 2048
+    need = _native.lib().fa_fwd_workspace_bytes
+    assert need(ctypes.byref(p)) == 0  # 256 row blocks fill the CUs
+    p.heads_q = p.heads_kv = 1
+    assert need(ctypes.byref(p)) > 0
+    p.seqlen_k = 200  # fewer than two shares of four tiles
+    assert need(ctypes.byref(p)) == 0
+    p.seqlen_k, p.head_dim = 2048, 128
+    assert need(ctypes.byref(p)) == 0
