@@ -9,7 +9,8 @@ hipError_t bwd_by_mods(const fa_bwd_params& p, int ph, hipStream_t s);
 
 size_t bwd_ds_bytes(const fa_bwd_params& p) {
   const fa_fwd_params& f = p.fwd;
-  if (f.dtype == FA_DTYPE_F32 || f.head_dim > 128 || f.head_dim < 64) return 0;
+  if (f.dtype == FA_DTYPE_F32 || f.head_dim > 256 || f.head_dim < 64) return 0;
+  if (f.head_dim > 128 && f.cu_seqlens_q) return 0;
   if (f.batch <= 0 || f.heads_q <= 0 || f.seqlen_q <= 0 || f.seqlen_k <= 0) return 0;
   int64_t elems;
   if (f.cu_seqlens_q) {

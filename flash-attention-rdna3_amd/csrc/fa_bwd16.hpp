@@ -798,6 +798,8 @@ __global__ __launch_bounds__(512, 1) void dq16_kernel(fa_bwd_params p, int num_m
 //    steps through a 4-stage ring (64 KiB of LDS), two workgroups per CU, so
 //    one workgroup's prologue (its first loads) and epilogue (the half merge
 //    and dQ store) overlap the other's steady state.
+// D = 256 takes 16-key steps with one workgroup per CU (96 KiB of ring; a
+// wave's dQ alone is 128 registers).
 // Measured at config 2 (512 workgroups) 43 us with OCC = 1 against 50 us;
 // at config 5 (4608 workgroups) 310 us with OCC = 2 against 369 us.
 template <int D, int OCC>
@@ -807,9 +809,9 @@ struct Dqs16Cfg {
   static constexpr int NT = 64 * NW;
   static constexpr int NTH = 64 * NQ;
   static constexpr int BM = 32 * NQ;
-  // keys per step (part of a dS tile); 16-key stages need D >= 128 to fill
+  // keys per step (part of a dS tile); 16-key steps need D >= 128 to fill
   // whole 16-byte chunks per thread
-  static constexpr int BN = (OCC == 2 && D >= 128) ? 16 : 32;
+  static constexpr int BN = (D >= 256 || (OCC == 2 && D >= 128)) ? 16 : 32;
   static constexpr int NSTG = 4;                   // ring of stages per key half
   static constexpr int KT = BN * D;                // K rows (elements)
   static constexpr int ST = BN * BM;               // dS rows: BN keys x BM queries

@@ -27,6 +27,7 @@
 #include "fa_internal.hpp"
 #include "fa_tiles.hpp"
 #include "fa_bwd16.hpp"
+#include "fa_bwd_roles.hpp"
 
 namespace fa {
 
@@ -599,8 +600,11 @@ __global__ __launch_bounds__(256) void bwd_dq_kernel(fa_bwd_params p, int num_m_
 // ---------------------------------------------------------------------------
 template <typename Tag, int D, int MODE>
 static hipError_t run_bwd_dkdv16(const fa_bwd_params& p, hipStream_t stream) {
-  using C = Dkdv16Cfg<D>;
-  auto kern = dkdv16_kernel<Tag, D, MODE>;
+  constexpr bool ROLES = D > 128;
+  using C = typename std::conditional<ROLES, DkdvRolesCfg<D>, Dkdv16Cfg<D>>::type;
+  void (*kern)(fa_bwd_params, int);
+  if constexpr (ROLES) kern = dkdv_roles_kernel<Tag, D, MODE>;
+  else kern = dkdv16_kernel<Tag, D, MODE>;
   hipError_t e = allow_lds((const void*)kern, C::LDS_BYTES);
   if (e != hipSuccess) return e;
   const int nnb = (p.fwd.seqlen_k + C::BN - 1) / C::BN;
@@ -623,11 +627,13 @@ static hipError_t launch_dqs16(const fa_bwd_params& p, long grid, int nmb, float
 template <typename Tag, int D, int MODE>
 static hipError_t run_bwd(const fa_bwd_params& p, int phases, hipStream_t stream) {
   const fa_fwd_params& f = p.fwd;
-  constexpr bool FAST = !std::is_same<Tag, f32_t>::value && D <= 128;
+  constexpr bool FAST = !std::is_same<Tag, f32_t>::value && D <= 256;
+  // dQ recomputed from Q, K, V (no dS scratch): 16-bit kernel up to D = 128.
+  constexpr bool FAST_DQ = FAST && D <= 128;
   bool fast_ok = false;
   if constexpr (FAST)
-    fast_ok = buf_rows_ok(f.q_stride[2], Dkdv16Cfg<D>::BMQ) && buf_rows_ok(p.dout_stride[2], Dkdv16Cfg<D>::BMQ) &&
-              buf_rows_ok(f.k_stride[2], Dq16Cfg<D>::BN) && buf_rows_ok(f.v_stride[2], Dq16Cfg<D>::BN);
+    fast_ok = buf_rows_ok(f.q_stride[2], 32) && buf_rows_ok(p.dout_stride[2], 32) &&
+              buf_rows_ok(f.k_stride[2], D <= 64 ? 64 : 32) && buf_rows_ok(f.v_stride[2], D <= 64 ? 64 : 32);
   // With score-gradient scratch the dK/dV kernel stores dS and dQ = dS K
   // runs after it (dqs16_kernel); without it, the full 16-bit backward
   // computes delta inside the dQ kernel, which then runs first.  Otherwise
@@ -684,7 +690,7 @@ static hipError_t run_bwd(const fa_bwd_params& p, int phases, hipStream_t stream
       }
     }
   }
-  const bool fused_delta = fast_ok && !use_ds && (phases & 1) && (phases & 4);
+  const bool fused_delta = FAST_DQ && fast_ok && !use_ds && (phases & 1) && (phases & 4);
   if ((phases & 1) && !fused_delta) {
     constexpr int rows = 16 * delta_rows_per_thread<Tag, D>();
     const int nrb = (f.seqlen_q + rows - 1) / rows;
@@ -724,40 +730,49 @@ static hipError_t run_bwd(const fa_bwd_params& p, int phases, hipStream_t stream
         if constexpr (D >= 128) {
           const long cus = device_cu_count();
           const long pairs = (long)((nmb + 1) / 2) * f.batch * f.heads_q;
-          if (grid > 3L * cus) return launch_dqs16<Tag, D, 2, false, VL>(p, grid, nmb, dq_scale, ds_nt, stream);
+          if constexpr (D == 128)
+            if (grid > 3L * cus) return launch_dqs16<Tag, D, 2, false, VL>(p, grid, nmb, dq_scale, ds_nt, stream);
           if (pairs >= cus) return launch_dqs16<Tag, D, 1, true, VL>(p, pairs, nmb, dq_scale, ds_nt, stream);
         }
         return launch_dqs16<Tag, D, 1, false, VL>(p, grid, nmb, dq_scale, ds_nt, stream);
       };
-      hipError_t e = f.cu_seqlens_q ? launch_all(std::true_type{}) : launch_all(std::false_type{});
+      hipError_t e;
+      if constexpr (FAST_DQ) e = f.cu_seqlens_q ? launch_all(std::true_type{}) : launch_all(std::false_type{});
+      else e = launch_all(std::false_type{});  // (varlen has no dS scratch above D = 128)
       if (e != hipSuccess) return e;
       // Varlen: a sequence longer than max_seqlen / total promised has no
       // room in the scratch; dQ from dS left its heads alone and they get
       // the recomputed dQ here (one workgroup per sequence, which returns at
       // once when its last head's region fit, and so all of them).  Dense
       // scratch is sized exactly, so no such head exists.
-      if (f.cu_seqlens_q) {
-        using CQ = Dq16Cfg<D>;
-        auto kq = dq16_kernel<Tag, D, MODE>;
-        e = allow_lds((const void*)kq, CQ::LDS_BYTES);
+      if constexpr (FAST_DQ) {
+        if (f.cu_seqlens_q) {
+          using CQ = Dq16Cfg<D>;
+          auto kq = dq16_kernel<Tag, D, MODE>;
+          e = allow_lds((const void*)kq, CQ::LDS_BYTES);
+          if (e != hipSuccess) return e;
+          const int nq = (f.seqlen_q + CQ::BM - 1) / CQ::BM;
+          hipLaunchKernelGGL(kq, dim3((unsigned)f.batch), dim3(CQ::NT), CQ::LDS_BYTES, stream, p, nq, 2);
+          e = hipGetLastError();
+          if (e != hipSuccess) return e;
+        }
+      }
+      phases &= ~4;
+    }
+    }
+    if constexpr (FAST_DQ) {
+      if (phases & 4) {
+        using C = Dq16Cfg<D>;
+        auto kern = dq16_kernel<Tag, D, MODE>;
+        hipError_t e = allow_lds((const void*)kern, C::LDS_BYTES);
         if (e != hipSuccess) return e;
-        const int nq = (f.seqlen_q + CQ::BM - 1) / CQ::BM;
-        hipLaunchKernelGGL(kq, dim3((unsigned)f.batch), dim3(CQ::NT), CQ::LDS_BYTES, stream, p, nq, 2);
+        const int nmb = (f.seqlen_q + C::BM - 1) / C::BM;
+        const long grid = (long)nmb * f.batch * f.heads_q;
+        hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(C::NT), C::LDS_BYTES, stream, p, nmb, fused_delta ? 1 : 0);
         e = hipGetLastError();
         if (e != hipSuccess) return e;
+        phases &= ~4;
       }
-    }
-    }
-    if ((phases & 4) && !use_ds) {
-      using C = Dq16Cfg<D>;
-      auto kern = dq16_kernel<Tag, D, MODE>;
-      hipError_t e = allow_lds((const void*)kern, C::LDS_BYTES);
-      if (e != hipSuccess) return e;
-      const int nmb = (f.seqlen_q + C::BM - 1) / C::BM;
-      const long grid = (long)nmb * f.batch * f.heads_q;
-      hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(C::NT), C::LDS_BYTES, stream, p, nmb, fused_delta ? 1 : 0);
-      e = hipGetLastError();
-      if (e != hipSuccess) return e;
     }
     if (phases & 2) {
       // Without dS scratch the kernel must not store dS (ds_workspace is
@@ -766,8 +781,8 @@ static hipError_t run_bwd(const fa_bwd_params& p, int phases, hipStream_t stream
       if (!use_ds) q.ds_workspace = nullptr;
       hipError_t e = run_bwd_dkdv16<Tag, D, MODE>(q, stream);
       if (e != hipSuccess) return e;
+      phases &= ~2;
     }
-    return hipSuccess;
   }
   }
   constexpr int GMODE = MODE == 3 ? 1 : MODE;  // no softcap-only generic variant

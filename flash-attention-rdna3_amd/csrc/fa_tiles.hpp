@@ -401,6 +401,48 @@ __device__ inline uint32_t lds_addr(const void* p) {
   return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
 }
 
+// The reads of swz_op and tr_op_rowmap from one lane address.  In a tile
+// whose LDS address is a multiple of 256 bytes, the swizzle only changes
+// address bits 4 to 7, so every operand of a lane sits at its first
+// operand's address XOR a constant, plus a constant.  One register then
+// replaces the address per operand that the compiler otherwise keeps across
+// a loop (48 registers for a 32 x 256 tile read both ways).
+// tile_lane: an address recomputed per tile; opaque, so that the XORs are
+// not hoisted out of the loop again.
+__device__ inline uint32_t tile_lane(uint32_t tile, uint32_t lane_off) {
+  uint32_t a = tile + lane_off;
+  asm volatile("" : "+v"(a));
+  return a;
+}
+template <int COLS>
+__device__ inline uint32_t row_lane_off(int lane) {
+  const int l32 = lane & 31, h = lane >> 5;
+  return (uint32_t)(l32 * COLS * 2 + ((h ^ swz<COLS>(l32)) << 4));
+}
+// swz_op<COLS>(tile, 32 * blk + l32, 2 * s + h)
+template <int COLS>
+__device__ inline s16x8 row_op(uint32_t a, int s, int blk = 0) {
+  constexpr int SX = COLS >= 128 ? 7 : COLS / 16 - 1;  // k-steps within one 256-byte (or whole) row piece
+  typedef const __attribute__((address_space(3))) s16x8 lds_op;
+  return *(lds_op*)((a ^ (uint32_t)((s & SX) << 5)) + (uint32_t)((s & ~SX) << 5) + (uint32_t)(blk * 32 * COLS * 2));
+}
+template <int COLS>
+__device__ inline uint32_t tr_lane_off(int lane) {
+  return (uint32_t)(swz_off<COLS>(4 * (lane >> 5) + ((lane & 15) >> 2), 16 * ((lane >> 4) & 1) + 4 * (lane & 3)) * 2);
+}
+// tr_op_rowmap<COLS>(tile, 0, 32 * db, j, lane)
+template <int COLS>
+__device__ inline s16x8 tr_op(uint32_t a, int j, int db) {
+  constexpr int DX = COLS >= 128 ? 3 : COLS / 32 - 1;  // column blocks within one row piece
+  typedef short s4 __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) s4 lds_s4;
+  const uint32_t x = (uint32_t)((db & DX) << 6), o = (uint32_t)((db & ~DX) << 6) + (uint32_t)(16 * j * COLS * 2);
+  const s4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)((a ^ x) + o));
+  const s4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)((a ^ x ^ 32u) + o + (uint32_t)(8 * COLS * 2)));
+  s16x8 r = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+  return r;
+}
+
 // Scheduling hint for a block of N MFMAs that each consume RPM LDS reads:
 // issue the reads of the first AHEAD MFMAs first, then alternate one MFMA
 // with the reads of a later one, so LDS latency overlaps MFMA execution
@@ -419,6 +461,19 @@ __device__ inline void sched_read_ahead() {
   __builtin_amdgcn_sched_group_barrier(0x008, A, 0);
 }
 
+
+// The same for GROUPS groups of RPG reads that each feed MPG MFMAs.
+template <int GROUPS, int AHEAD, int RPG, int MPG>
+__device__ inline void sched_reads() {
+  constexpr int A = AHEAD < GROUPS ? AHEAD : GROUPS;
+  __builtin_amdgcn_sched_group_barrier(0x100, A * RPG, 0);
+#pragma unroll
+  for (int i = 0; i < GROUPS - A; ++i) {
+    __builtin_amdgcn_sched_group_barrier(0x008, MPG, 0);
+    __builtin_amdgcn_sched_group_barrier(0x100, RPG, 0);
+  }
+  __builtin_amdgcn_sched_group_barrier(0x008, A * MPG, 0);
+}
 
 // A 32x32 fp32 accumulator (16 values per lane) parked in LDS and read back
 // as four 16-byte chunks per lane, chunk-major (chunk c of lane L at float

@@ -1,5 +1,6 @@
-"""16-bit forward at head dims 256 and 512 (one wave per SIMD, key splits)
-against 64-bit attention, at tile edges, splits and modifiers."""
+"""16-bit forward and backward at head dims 256 and 512 (one wave per SIMD,
+key-split forward, dK/dV with its two products on two waves) against 64-bit
+attention, at tile edges, splits and modifiers."""
 
 import ctypes
 import math
@@ -7,8 +8,8 @@ import math
 import pytest
 import torch
 
-from attn_refs import attention
-from fa_rdna3 import _native, flash_attention
+from attn_refs import attention, grads, varlen_attention
+from fa_rdna3 import _native, alibi_slopes, flash_attention, flash_attention_varlen
 from fa_rdna3.interface import _fwd_params
 
 pytestmark = pytest.mark.gpu
@@ -95,3 +96,72 @@ def test_no_splits_without_room_to_gain():
     assert need(ctypes.byref(p)) == 0
     p.seqlen_k, p.head_dim = 2048, 128
     assert need(ctypes.byref(p)) == 0
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("heads,kv,sq,sk,opts", [
+    (2, 2, 1, 1, {}), (2, 1, 31, 33, {"causal": True}), (2, 2, 64, 64, {"causal": True}), (4, 2, 129, 65, {}),
+    (4, 2, 333, 700, {"causal": True}), (2, 1, 500, 500, {"softcap": 10.0}),
+    (2, 2, 500, 500, {"causal": True, "window": (90, 0), "softcap": 30.0}),
+    (2, 2, 400, 257, {"bias": True, "window": (100, 60)}), (2, 2, 257, 400, {"alibi": True, "causal": True}),
+])
+def test_backward_256(dtype, heads, kv, sq, sk, opts):
+    gen = torch.Generator().manual_seed(sq + 3 * sk)
+    opts = dict(opts)
+    q, do = (_rand((1, sq, heads, 256), dtype, gen).transpose(1, 2) for _ in range(2))
+    k, v = (_rand((1, kv, sk, 256), dtype, gen) for _ in range(2))
+    window = opts.pop("window", (-1, -1))
+    bias = _rand((1, heads, sq, sk), torch.float32, gen) if opts.pop("bias", False) else None
+    slopes = alibi_slopes(heads) if opts.pop("alibi", False) else None
+    got = grads(lambda a, b, c: flash_attention(a, b, c, window_size=window, bias=bias, alibi_slopes=slopes, **opts),
+                q, k, v, do)
+    want = grads(lambda a, b, c: attention(a, b, c, window=window, bias=None if bias is None else bias.double(),
+                                           alibi=None if slopes is None else slopes.double(), **opts),
+                 q.double(), k.double(), v.double(), do.double())
+    scale = max(float(w.norm()) for w in want)
+    for g, w in zip(got, want):
+        if float(w.norm()) <= 1e-6 * scale:  # one visible key: dQ and dK are rounding noise around zero
+            assert float(g.double().norm()) <= BOUND[dtype] * scale
+        else:
+            _close(g, w, dtype)
+
+
+def test_dropout_256_equals_zero_padded_128():
+    """The dropout mask depends on positions and seed only, so a head of 128
+    padded with zeros to 256 must give the 128-wide kernels' result."""
+    gen = torch.Generator().manual_seed(9)
+    q, k, v, do = (_rand((1, 2, 300, 128), torch.float16, gen) for _ in range(4))
+    pad = lambda t: torch.nn.functional.pad(t, (0, 128))
+    tail = (False, 0.1, -1, -1, 0.0, None, None, 0.3, 1234)
+    ops = _native.ops()
+    out, lse = ops.forward(q, k, v, *tail)
+    wide, wlse = ops.forward(pad(q), pad(k), pad(v), *tail)
+    _close(wide[..., :128], out, torch.float16)
+    assert (wlse - lse).abs().max() <= 1e-5
+    for g, w in zip(ops.backward(pad(do), pad(q), pad(k), pad(v), wide, wlse, *tail),
+                    ops.backward(do, q, k, v, out, lse, *tail)):
+        _close(g[..., :128], w, torch.float16)
+        assert (g[..., 128:] == 0).all()
+
+
+@pytest.mark.parametrize("limit", [0, None])
+def test_backward_256_varlen_and_without_scratch(limit):
+    gen = torch.Generator().manual_seed(11)
+    lens = [1, 70, 300, 129]
+    q, do = (_rand((sum(lens), 4, 256), torch.bfloat16, gen) for _ in range(2))
+    k, v = (_rand((sum(lens), 2, 256), torch.bfloat16, gen) for _ in range(2))
+    cu = torch.tensor([0, 1, 71, 371, 500], dtype=torch.int32, device="cuda")
+    before = _native.ds_scratch_limit()
+    try:
+        if limit is not None:
+            _native.set_ds_scratch_limit(limit)
+        got = grads(lambda a, b, c: flash_attention_varlen(a, b, c, cu, cu, 300, 300, causal=True), q, k, v, do)
+        dense = grads(lambda a, b, c: flash_attention(a, b, c, causal=True), *(
+            t[71:371].transpose(0, 1)[None] for t in (q, k, v, do)))
+    finally:
+        _native.set_ds_scratch_limit(before)
+    want = grads(lambda a, b, c: varlen_attention(a, b, c, lens, lens, causal=True),
+                 q.double(), k.double(), v.double(), do.double())
+    for g, d, w in zip(got, dense, want):
+        _close(g, w, torch.bfloat16)
+        _close(d[0].transpose(0, 1), w[71:371], torch.bfloat16)
