@@ -13,8 +13,12 @@
 // operand set in registers, so every MFMA reads at most one operand from LDS
 // where dkdv16_kernel's score products read two.  That makes D = 256 fit two
 // waves per SIMD (a wave holding dK and dV of 32 keys would need 256 registers
-// for them alone).  LDS reads and the two barriers per step bound it.
-// Measured at 1 x 16/8 x 2048 x 256 bf16 causal (69 GFLOP): 175 us with the
+// for them alone).  LDS reads and the two barriers per step bound it.  The
+// registers are full, so whatever lives across the step loop is kept small
+// (row_op / tr_op / DmaLeanTile addresses, LDS reads two MFMAs ahead, dS
+// stores by buffer window): a reload from scratch inside the loop waits for
+// the next stage's loads too, and cost 25 us of the figure below.
+// Measured at 1 x 16/8 x 2048 x 256 bf16 causal (69 GFLOP): 148 us with the
 // dS stores, against 920 us for bwd_dkdv_kernel; dQ from that dS 47 us against
 // 453 us for bwd_dq_kernel.
 #pragma once
@@ -117,7 +121,7 @@ __global__ __launch_bounds__(512, 1) void dkdv_roles_kernel(fa_bwd_params p, int
 #pragma unroll
     for (int i = 0; i < C::NDB; ++i) acc[kb][i] = zero16();
 
-  DmaSwzTile<C::BMQ, D, C::NTH> qd, gd;
+  DmaLeanTile<C::BMQ, D, C::NTH> qd, gd;
   qd.init(f.q_stride[2], htid);
   gd.init(p.dout_stride[2], htid);
   unsigned char* const hsmem = smem_raw + qhalf * C::HALF_BYTES;
@@ -176,23 +180,16 @@ __global__ __launch_bounds__(512, 1) void dkdv_roles_kernel(fa_bwd_params p, int
       }
     };
 
-    // dS of this lane's first key in the scratch (see dkdv16_kernel).
+    // dS of this wave's first key in the scratch (see dkdv16_kernel).
     bool ds_on = false;
-    S* dsn = nullptr;
-    S* ds_dump = nullptr;
+    const S* dsn = nullptr;
     if (p.ds_workspace != nullptr) {
       const int64_t region = ds_region_at(p, ds_base, hq, sq, sk);
       ds_on = region >= 0;
-      S* const ws = reinterpret_cast<S*>(p.ds_workspace);
-      const int n = n0w + l32;
-      dsn = ws + (ds_on ? region : 0) + (int64_t)(n / kDsTileKeys) * ds_qblocks(sq) * kDsTileElems +
-            (n % kDsTileKeys) * kDsSubQueries;
-      ds_dump = ws + (p.ds_workspace_bytes - 1024) / 2;
+      dsn = reinterpret_cast<const S*>(p.ds_workspace) + (ds_on ? region : 0) +
+            (int64_t)(n0w / kDsTileKeys) * ds_qblocks(sq) * kDsTileElems + (n0w % kDsTileKeys) * kDsSubQueries;
     }
     const VisBounds kvb = key_block_bounds(md, n0w, ncols);
-    int rlo[KB], rhi[KB];
-#pragma unroll
-    for (int kb = 0; kb < KB; ++kb) row_bounds(md, n0w + 32 * kb + l32, rlo[kb], rhi[kb]);
     if (my_count > 0) {
       const int m_first = mlo + my_first * C::BMQ;
       load_stage(m_first, 0);
@@ -229,12 +226,14 @@ __global__ __launch_bounds__(512, 1) void dkdv_roles_kernel(fa_bwd_params p, int
         }
         const uint32_t ra = tile_lane(qtile + (kwave ? C::QT * 2u : 0u), row_off);
 #pragma unroll
-        for (int s = 0; s < C::NSTEP; ++s) {
+        for (int i = 0; i < C::NSTEP; ++i) {
+          // k-steps 8 apart share an address (row_op): taken in turn.
+          const int s = C::NSTEP <= 8 ? i : (i >> 1) + 8 * (i & 1);
           const s16x8 a = row_op<D>(ra, s);
 #pragma unroll
           for (int kb = 0; kb < KB; ++kb) x[kb] = EL::mma(a, op[kb][s], x[kb]);
         }
-        sched_reads<C::NSTEP, 4, 1, KB>();
+        sched_reads<C::NSTEP, 2, 1, KB>();
         if (!kwave) {
           // P, and what the K wave needs of it: P times the softcap's
           // derivative (MODE 3: a quarter of it), negative where dropout
@@ -244,7 +243,12 @@ __global__ __launch_bounds__(512, 1) void dkdv_roles_kernel(fa_bwd_params p, int
             constexpr bool MASK = decltype(mask_t)::value;
 #pragma unroll
             for (int kb = 0; kb < KB; ++kb) {
-              const Span rs = make_span(rlo[kb], rhi[kb], m0 + 4 * h);
+              Span rs{0, 0};
+              if constexpr (MASK) {
+                int rlo, rhi;
+                row_bounds(md, n0w + 32 * kb + l32, rlo, rhi);
+                rs = make_span(rlo, rhi, m0 + 4 * h);
+              }
               f32x16 w;
 #pragma unroll
               for (int q4 = 0; q4 < 4; ++q4) {
@@ -333,7 +337,7 @@ __global__ __launch_bounds__(512, 1) void dkdv_roles_kernel(fa_bwd_params p, int
 #pragma unroll
             for (int kb = 0; kb < KB; ++kb) acc[kb][db] = EL::mma(a, xb[kb][j], acc[kb][db]);
           }
-        sched_reads<C::NPV * C::NDB, 4, 2, KB>();
+        sched_reads<C::NPV * C::NDB, 2, 2, KB>();
       }
       if (t + 1 < my_count) store_stage(st ^ 1, m0 + C::BMQ);
       const bool ds_store = ds_on && vis && kwave;
@@ -350,12 +354,16 @@ __global__ __launch_bounds__(512, 1) void dkdv_roles_kernel(fa_bwd_params p, int
             w0[i] = r[0];
             w1[i] = r[1];
           }
-          S* const at = n0w + 32 * kb + l32 >= sk
-                            ? ds_dump
-                            : dsn + kb * 32 * kDsSubQueries + (int64_t)(m0 / kDsTileQueries) * kDsTileElems +
-                                  (m0 % kDsTileQueries) / kDsSubQueries * kDsSubElems + 16 * h;
-          *reinterpret_cast<u32x4*>(at) = u32x4{w0[0], w0[1], w1[0], w1[1]};
-          *reinterpret_cast<u32x4*>(at + 8) = u32x4{w0[2], w0[3], w1[2], w1[3]};
+          // A buffer window over this wave's rows of the sub-tile: lanes past
+          // the last key fall outside it and store nothing, yet every wave
+          // issues the same stores (the wait below counts them).
+          const int rows = min(32, ncols - 32 * kb);
+          const S* at = dsn + kb * 32 * kDsSubQueries + (int64_t)(m0 / kDsTileQueries) * kDsTileElems +
+                        (m0 % kDsTileQueries) / kDsSubQueries * kDsSubElems;
+          const __amdgpu_buffer_rsrc_t rs = rows_rsrc<kDsSubQueries>(at, kDsSubQueries, rows);
+          const uint32_t o = (uint32_t)(l32 * kDsSubQueries * 2 + 32 * h);
+          __builtin_amdgcn_raw_buffer_store_b128(u32x4{w0[0], w0[1], w1[0], w1[1]}, rs, o, 0, 0);
+          __builtin_amdgcn_raw_buffer_store_b128(u32x4{w0[2], w0[3], w1[2], w1[3]}, rs, o + 16, 0, 0);
         }
       }
       // The next stage must have landed; this step's dS stores, issued after

@@ -390,6 +390,41 @@ struct DmaSwzTile {
   }
 };
 
+// DmaSwzTile with the fewest registers: rows 16 apart share a swizzle, so a
+// thread's chunks need one offset per swizzle phase and a scalar step (the
+// sum is formed per load; opaque, or the compiler keeps every sum in a
+// register across the loop).
+template <int R, int COLS, int NT>
+struct DmaLeanTile {
+  static constexpr int CPR = COLS / 8;
+  static constexpr int CH = R * CPR;
+  static_assert(CH % NT == 0 && NT % CPR == 0, "whole rows, whole chunks per thread");
+  static constexpr int PT = CH / NT;
+  static constexpr int RPJ = NT / CPR;  // rows per load of all threads
+  static constexpr int NV = RPJ >= 16 ? 1 : (16 / RPJ < PT ? 16 / RPJ : PT);
+  static_assert(RPJ >= 16 ? RPJ % 16 == 0 : 16 % RPJ == 0, "swizzle period");
+  uint32_t voff[NV];
+  uint32_t step;  // bytes between loads of one phase (uniform)
+
+  __device__ inline void init(int64_t stride, int tid) {
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      const int slot = NT * j + tid;
+      const int row = slot / CPR;
+      voff[j] = (uint32_t)(row * stride * 2 + ((slot % CPR) ^ swz<COLS>(row)) * 16);
+    }
+    step = (uint32_t)(NV * RPJ * stride * 2);
+  }
+  __device__ inline void load(i32x4 rs, uint32_t lds_tile, int wave) const {
+#pragma unroll
+    for (int j = 0; j < PT; ++j) {
+      uint32_t v = voff[j % NV];
+      asm volatile("" : "+v"(v));
+      buf_load_lds16(rs, v + (uint32_t)(j / NV) * step, lds_tile + (uint32_t)(NT * j + 64 * wave) * 16u);
+    }
+  }
+};
+
 // s_waitcnt vmcnt(n) with the other counters left alone (gfx9 encoding).
 template <int N>
 __device__ inline void wait_vm() {
