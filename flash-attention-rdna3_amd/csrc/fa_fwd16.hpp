@@ -78,11 +78,7 @@ struct Fwd16Cfg {
 };
 
 // Largest growth of the running max (log2 domain) absorbed without rescaling.
-// Wide heads follow the max exactly: the largest weights are then 1 or just
-// below it, where a 16-bit float rounds least (measured output error at
-// D = 512 fp16: 2.85e-4 of the norm against 2.93e-4 with a lazy max).
-template <int D>
-constexpr float kLazyRescale = D <= 128 ? 8.0f : 0.0f;
+constexpr float kLazyRescale = 8.0f;
 
 // One work item: the 128 query rows of row block (num_m_blocks - 1 - mb_rev)
 // of (batch, head) bh, output columns [dc * DO, (dc + 1) * DO),
@@ -158,8 +154,8 @@ __device__ __forceinline__ void fwd16_item(const fa_fwd_params& p, int num_m_blo
 #pragma unroll
   for (int i = 0; i < C::NDB; ++i) acc[i] = zero16();
 
-  DmaSwzTile<C::BN, D, C::NTH> kt;
-  DmaSwzTile<C::BN, C::DO, C::NTH> vt;
+  DmaLeanTile<C::BN, D, C::NTH> kt;
+  DmaLeanTile<C::BN, C::DO, C::NTH> vt;
   kt.init(ks, htid);
   vt.init(vs, htid);
   // Both halves run nh0 steps so their barriers line up.
@@ -171,6 +167,8 @@ __device__ __forceinline__ void fwd16_item(const fa_fwd_params& p, int num_m_blo
   constexpr int TSTEP = NH;
   const int my_count = NH == 1 ? ntiles : khalf == 0 ? nh0 : ntiles - nh0;
   const uint32_t lds0 = lds_addr(smem) + (uint32_t)(khalf * C::HALF) * 2u;
+  const uint32_t row_off = row_lane_off<D>(lane), tr_off = tr_lane_off<C::DO>(lane);
+  static_assert(C::KTILE % 128 == 0 && C::STAGE % 128 == 0, "row_op / tr_op addressing");
   // Tile sources advance by BN rows per load (scalar pointer arithmetic).
   int n_next = lo + my_first * C::BN;
   const S* k_next = kb + (int64_t)n_next * ks;
@@ -185,6 +183,14 @@ __device__ __forceinline__ void fwd16_item(const fa_fwd_params& p, int num_m_blo
     v_next += (int64_t)(TSTEP * C::BN) * vs;
   };
   const VisBounds vbnd = row_block_bounds(md, m0w, mrows);
+  // Wide heads and the dense fp16 form with one key half follow the max
+  // exactly: the largest weights are then 1 or just below it, where a 16-bit
+  // float rounds least.  (The split form keeps two maxima per row, which is
+  // as good as that; bf16 carries P in two parts.)  Output error against 64
+  // bits, lazy and exact: 2.92e-4 and 2.84e-4 of the norm at 2 x 10 x 4096 x 64,
+  // 2.93e-4 and 2.78e-4 at 1 x 1 x 4096 x 512.
+  const bool exact_max = D > 128 || (NH == 1 && std::is_same<Tag, f16_t>::value && p.cu_seqlens_q == nullptr);
+  const float lazy = exact_max ? 0.f : kLazyRescale;
 
   // The first tiles' DMA and the Q loads share one round trip to memory.
   if (my_count > 0) load_tiles(0);
@@ -206,8 +212,8 @@ __device__ __forceinline__ void fwd16_item(const fa_fwd_params& p, int num_m_blo
     const int vis = t < my_count ? bounds_vis(vbnd, n0, n0 + C::BN - 1) : 0;
     if (!vis && t + 1 < my_count) load_tiles(stage ^ 1);
     if (vis) {
-      const S* Ks = smem + khalf * C::HALF + stage * C::STAGE;
-      const S* Vs = Ks + C::KTILE;
+      const uint32_t ktile = lds0 + (uint32_t)(stage * C::STAGE) * 2u;
+      const uint32_t ka = tile_lane(ktile, row_off);
       f32x16 sacc[C::NKB];
 #pragma unroll
       for (int kb2 = 0; kb2 < C::NKB; ++kb2) sacc[kb2] = zero16();
@@ -215,7 +221,7 @@ __device__ __forceinline__ void fwd16_item(const fa_fwd_params& p, int num_m_blo
       for (int s = 0; s < C::NSTEP; ++s)
 #pragma unroll
         for (int kb2 = 0; kb2 < C::NKB; ++kb2)
-          sacc[kb2] = EL::mma(swz_op<D>(Ks, kb2 * 32 + l32, 2 * s + h), qop[s], sacc[kb2]);
+          sacc[kb2] = EL::mma(row_op<D>(ka, s, kb2), qop[s], sacc[kb2]);
       sched_read_ahead<C::NSTEP * C::NKB, 4>();
       // The next tile's loads go out while the score MFMAs drain (issuing
       // them before the MFMAs would hold the MFMAs back behind the queue).
@@ -239,17 +245,21 @@ __device__ __forceinline__ void fwd16_item(const fa_fwd_params& p, int num_m_blo
         // with modifiers skips the per-score interval test.
         auto masked_scores = [&](auto cap_t, auto bias_t, auto alibi_t, auto mask_t) {
 #pragma unroll
-          for (int kb2 = 0; kb2 < C::NKB; ++kb2)
+          for (int kb2 = 0; kb2 < C::NKB; ++kb2) {
+            constexpr int BIASK = decltype(bias_t)::value;
+            f32x16 bv = zero16();
+            if constexpr (BIASK != 0) bv = load_bias16<BIASK>(md, m, n0 + kb2 * 32 + 4 * h);
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
               const int n = n0 + kb2 * 32 + acc_row(i, h);
               float tc;
-              float x = score_m<decltype(cap_t)::value, decltype(bias_t)::value, decltype(alibi_t)::value>(
-                  md, sacc[kb2][i], m, n, tc);
+              float x = score_bv<decltype(cap_t)::value, BIASK != 0, decltype(alibi_t)::value>(
+                  md, sacc[kb2][i], m, n, tc, BIASK != 0 ? bv[i] : 0.f);
               if constexpr (decltype(mask_t)::value) x = in_span(ks, kb2 * 32 + acc_row(i, 0)) ? x : kNegInf;
               sacc[kb2][i] = x;
               tmax = fmaxf(tmax, x);
             }
+          }
         };
         using T_ = std::true_type;
         using F_ = std::false_type;
@@ -284,7 +294,7 @@ __device__ __forceinline__ void fwd16_item(const fa_fwd_params& p, int num_m_blo
       }
       tmax = half_max(tmax);
       // Lazy rescale, decided for the whole wave.
-      if (__builtin_amdgcn_ballot_w64(tmax > m_i + kLazyRescale<D>)) {
+      if (__builtin_amdgcn_ballot_w64(tmax > m_i + lazy)) {
         const float m_new = fmaxf(m_i, tmax);
         const float alpha = (m_new == kNegInf) ? 1.f : __builtin_amdgcn_exp2f(m_i - m_new);
         l_i *= alpha;
@@ -350,11 +360,12 @@ __device__ __forceinline__ void fwd16_item(const fa_fwd_params& p, int num_m_blo
 #pragma unroll
         for (int j = 0; j < C::NPV; ++j) pl[j] = pack_op<Tag>(sacc[j >> 1], j & 1);
       }
+      const uint32_t va = tile_lane(ktile + C::KTILE * 2u, tr_off);
 #pragma unroll
       for (int j = 0; j < C::NPV; ++j)
 #pragma unroll
         for (int db = 0; db < C::NDB; ++db) {
-          const s16x8 a = tr_op_rowmap<C::DO>(Vs, 0, 32 * db, j, lane);
+          const s16x8 a = tr_op<C::DO>(va, j, db);
           acc[db] = EL::mma(a, pb[j], acc[db]);
           if constexpr (PSPLIT) acc[db] = EL::mma(a, pl[j], acc[db]);
         }
@@ -429,7 +440,7 @@ __device__ __forceinline__ void fwd16_item(const fa_fwd_params& p, int num_m_blo
 // read the same head's K / V, which the workgroup's XCD then holds in L2.
 template <typename Tag, int D, int MODE, int NH, bool PAIR>
 __global__ __launch_bounds__(256 * NH, D > 128 ? 1 : 3 - NH) void fwd16_kernel(fa_fwd_params p, int num_m_blocks) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
+  extern __shared__ __align__(256) unsigned char smem_raw[];
   if constexpr (!PAIR) {
     fwd16_item<Tag, D, MODE, NH>(p, num_m_blocks, blockIdx.x, smem_raw, false);
   } else {
@@ -448,7 +459,7 @@ __global__ __launch_bounds__(256 * NH, D > 128 ? 1 : 3 - NH) void fwd16_kernel(f
 template <typename Tag, int D, int MODE>
 __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void fwd16_split_kernel(fa_fwd_params p, int num_m_blocks,
                                                                            int nsplit, float* ws) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
+  extern __shared__ __align__(256) unsigned char smem_raw[];
   const int item = blockIdx.x / nsplit;
   fwd16_item<Tag, D, MODE, 1, true>(p, num_m_blocks, item, smem_raw, false, blockIdx.x - item * nsplit, nsplit,
                                     ws + (int64_t)blockIdx.x * Fwd16Cfg<D, 1>::PART);

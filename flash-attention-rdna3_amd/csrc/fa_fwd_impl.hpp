@@ -324,18 +324,26 @@ static hipError_t run_fwd(const fa_fwd_params& p, const FwdScratch& scratch, hip
     const int nmb = (p.seqlen_q + C::BM - 1) / C::BM;
     const long grid = (long)nmb * p.batch * p.heads_q;
     if (grid <= 0) return hipSuccess;
-    // One key half, two workgroups per CU, for packed varlen batches and for
-    // dense grids of more than eight rounds of one 8-wave workgroup per CU.
+    // One key half, independent 4-wave workgroups, for packed varlen batches,
+    // for blocks of equal cost (no causal mask) once there are more of them
+    // than CUs, and for causal grids of more than four rounds of one 8-wave
+    // workgroup per CU.  Equal blocks gain nothing from the key split, and
+    // 640 of them in pairs took two rounds of 256 CUs: 2 x 10 x 4096 x 64
+    // fp16 190 -> 140 us, 2 x 10 x 4096 x 154 with a key mask 41 -> 20 us.
+    // Causal 1 x 32/8 x 8000 x 128 bf16: 847 -> 809 us; two rounds (config 2)
+    // keep the key split, 61.0 against 59.2 us.
     // (Varlen always: a sequence's output then does not depend on the batch
     // it is packed with.  The two forms sum the key tiles in different
     // orders, so they agree to rounding, not bit for bit.)
-    if (p.cu_seqlens_q || grid > 8L * device_cu_count())
+    const long cus = device_cu_count();
+    if (p.cu_seqlens_q || (p.causal ? grid > 4 * cus : grid > cus))
       return launch_fwd16<Tag, D, MODE, 1>(p, grid, nmb, stream);
-    // Heavy and light row blocks of a head paired in one workgroup, when
-    // the pairs still give every CU a workgroup (config 2: 256 pairs):
-    // forward 52.5 -> 51.4 us, same results bit for bit.
+    // Heavy and light row blocks of a head paired in one workgroup, when the
+    // pairs fill whole rounds of the CUs (config 2: 256 pairs): forward
+    // 52.5 -> 51.4 us, same results bit for bit.
     const long pairs = (long)((nmb + 1) / 2) * p.batch * p.heads_q;
-    if (pairs >= device_cu_count()) return launch_fwd16<Tag, D, MODE, 2, true>(p, pairs, nmb, stream);
+    if (pairs >= cus && (cus - pairs % cus) % cus * 8 <= pairs)
+      return launch_fwd16<Tag, D, MODE, 2, true>(p, pairs, nmb, stream);
     return launch_fwd16<Tag, D, MODE, 2>(p, grid, nmb, stream);
     }
   }
