@@ -118,10 +118,15 @@ template <typename Tag, int D>
 struct DkdvCfg {
   using EL = Elem<Tag>;
   using S = typename EL::S;
-  static constexpr int NW = 4;
+  // fp32 up to D = 64: 64 keys and their query steps split between two halves
+  // of two waves (see FwdCfg), partial sums added through LDS.
+  static constexpr int NH = (sizeof(S) == 4 && D <= 64) ? 2 : 1;
+  static constexpr int NWK = 4 / NH;   // key waves per half
+  static constexpr int NW = NWK * NH;
   static constexpr int NT = 64 * NW;
-  static constexpr int BN = 32 * NW;  // keys per workgroup
-  static constexpr int BMQ = 32;      // query rows per inner step
+  static constexpr int NTH = 64 * NWK;
+  static constexpr int BN = 32 * NWK;  // keys per workgroup
+  static constexpr int BMQ = 32;       // query rows per inner step
   static constexpr int DO = (D <= 128) ? D : ((sizeof(S) == 4 && D == 512) ? 64 : 128);
   static constexpr bool KVREG = (sizeof(S) == 2) ? (D <= 128) : (D <= 64);
   static constexpr int QLD = D + EL::CE;     // Q / dO row-major tiles
@@ -131,8 +136,11 @@ struct DkdvCfg {
   // stage: Q, dO, Q^T, dO^T (elements of S) then lse2, delta (floats)
   static constexpr int STAGE_ELEMS = 2 * QTILE + 2 * TTILE;
   static constexpr int STAGE_BYTES = STAGE_ELEMS * (int)sizeof(S) + 2 * BMQ * 4;
-  static constexpr int NSTAGE = (2 * STAGE_BYTES <= 160 * 1024) ? 2 : 1;
-  static constexpr int LDS_BYTES = NSTAGE * STAGE_BYTES;
+  static constexpr int NSTAGE = (2 * NH * STAGE_BYTES <= 160 * 1024) ? 2 : 1;
+  static constexpr int HALF_BYTES = NSTAGE * STAGE_BYTES;
+  static constexpr int MERGE_BYTES = NH == 1 ? 0 : NWK * 2 * (DO / 32) * 4096;
+  static constexpr int LDS_BYTES = NH * HALF_BYTES > MERGE_BYTES ? NH * HALF_BYTES : MERGE_BYTES;
+  static_assert(NH == 1 || NSTAGE == 2, "two stages per half");
   static constexpr int NSTEP = D / EL::KSTEP;
   static constexpr int NMB = BMQ / 32;
   static constexpr int NPV = BMQ / (2 * EL::E);
@@ -149,7 +157,9 @@ __global__ __launch_bounds__(256) void bwd_dkdv_kernel(fa_bwd_params p, int num_
   const fa_fwd_params& f = p.fwd;
 
   const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform (SGPR)
+  const int wave_all = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform (SGPR)
+  const int qhalf = wave_all / C::NWK, wave = wave_all % C::NWK;
+  const int htid = tid % C::NTH;
   const int h = lane >> 5, l32 = lane & 31;
   const int ndc = D / C::DO;
   const int bhk_count = f.batch * f.heads_kv;
@@ -178,14 +188,14 @@ __global__ __launch_bounds__(256) void bwd_dkdv_kernel(fa_bwd_params p, int num_
   const int ncols = min(32, sk - n0w);  // <= 0: the wave only helps load
   const int n = n0w + l32;
   const bool nvalid = n < sk;
-  const S* krow = kbase + (int64_t)(nvalid ? n : 0) * f.k_stride[2] + EL::E * h;
-  const S* vrow = vbase + (int64_t)(nvalid ? n : 0) * f.v_stride[2] + EL::E * h;
+  const S* krow = kbase + (int64_t)(nvalid ? n : 0) * f.k_stride[2];
+  const S* vrow = vbase + (int64_t)(nvalid ? n : 0) * f.v_stride[2];
   Op kop[C::KVREG ? C::NSTEP : 1], vop[C::KVREG ? C::NSTEP : 1];
   if constexpr (C::KVREG) {
 #pragma unroll
     for (int s = 0; s < C::NSTEP; ++s) {
-      kop[s] = nvalid ? load_op<Tag>(krow + EL::KSTEP * s) : zero_op<Tag>();
-      vop[s] = nvalid ? load_op<Tag>(vrow + EL::KSTEP * s) : zero_op<Tag>();
+      kop[s] = nvalid ? load_op<Tag>(krow + kslot<Tag>(s, h)) : zero_op<Tag>();
+      vop[s] = nvalid ? load_op<Tag>(vrow + kslot<Tag>(s, h)) : zero_op<Tag>();
     }
     wait_vm_all();
   }
@@ -194,8 +204,8 @@ __global__ __launch_bounds__(256) void bwd_dkdv_kernel(fa_bwd_params p, int num_
 #pragma unroll
   for (int i = 0; i < C::NDB; ++i) { dk[i] = zero16(); dv[i] = zero16(); }
 
-  RowTile<Tag, C::BMQ, D, C::NT> qt, gt;
-  TransTile<Tag, C::BMQ, C::DO, C::NT> qtt, gtt;
+  RowTile<Tag, C::BMQ, D, C::NTH> qt, gt;
+  TransTile<Tag, C::BMQ, C::DO, C::NTH> qtt, gtt;
 
   const int nlast = min(n0 + C::BN, sk) - 1;
   for (int g = 0; g < group; ++g) {
@@ -219,46 +229,50 @@ __global__ __launch_bounds__(256) void bwd_dkdv_kernel(fa_bwd_params p, int num_
     const int nsteps = mhi > mlo ? (mhi - mlo + C::BMQ - 1) / C::BMQ : 0;
 
     auto load_stage = [&](int m0) {
-      qt.load([&](int r) -> const S* { int m = m0 + r; return m < sq ? qbase + (int64_t)m * qs : nullptr; }, qbase, tid);
-      gt.load([&](int r) -> const S* { int m = m0 + r; return m < sq ? gbase + (int64_t)m * gs : nullptr; }, gbase, tid);
+      qt.load([&](int r) -> const S* { int m = m0 + r; return m < sq ? qbase + (int64_t)m * qs : nullptr; }, qbase, htid);
+      gt.load([&](int r) -> const S* { int m = m0 + r; return m < sq ? gbase + (int64_t)m * gs : nullptr; }, gbase, htid);
       qtt.load([&](int r) -> const S* {
-        int m = m0 + r; return m < sq ? qbase + (int64_t)m * qs + dc * C::DO : nullptr; }, qbase + dc * C::DO, tid);
+        int m = m0 + r; return m < sq ? qbase + (int64_t)m * qs + dc * C::DO : nullptr; }, qbase + dc * C::DO, htid);
       gtt.load([&](int r) -> const S* {
-        int m = m0 + r; return m < sq ? gbase + (int64_t)m * gs + dc * C::DO : nullptr; }, gbase + dc * C::DO, tid);
+        int m = m0 + r; return m < sq ? gbase + (int64_t)m * gs + dc * C::DO : nullptr; }, gbase + dc * C::DO, htid);
     };
     auto store_stage = [&](int st, int m0) {
-      unsigned char* base = smem_raw + st * C::STAGE_BYTES;
+      unsigned char* base = smem_raw + qhalf * C::HALF_BYTES + st * C::STAGE_BYTES;
       S* sp = reinterpret_cast<S*>(base);
-      qt.store(sp, C::QLD, tid);
-      gt.store(sp + C::QTILE, C::QLD, tid);
-      qtt.store(sp + 2 * C::QTILE, C::TLD, tid);
-      gtt.store(sp + 2 * C::QTILE + C::TTILE, C::TLD, tid);
+      qt.store(sp, C::QLD, htid);
+      gt.store(sp + C::QTILE, C::QLD, htid);
+      qtt.store(sp + 2 * C::QTILE, C::TLD, htid);
+      gtt.store(sp + 2 * C::QTILE + C::TTILE, C::TLD, htid);
       float* lf = reinterpret_cast<float*>(base + C::STAGE_ELEMS * sizeof(S));
-      if (tid < C::BMQ) {
-        const int m = m0 + tid;
+      if (htid < C::BMQ) {
+        const int m = m0 + htid;
         float l = kNegInf, dl = 0.f;
         if (m < sq) {
           l = lbase[(int64_t)m * f.lse_stride[2]];
           dl = dbase[(int64_t)m * p.delta_stride[2]];
         }
-        lf[tid] = (l == kNegInf) ? kNegInf : l * kLog2e;
-        lf[C::BMQ + tid] = dl;
+        lf[htid] = (l == kNegInf) ? kNegInf : l * kLog2e;
+        lf[C::BMQ + htid] = dl;
       }
     };
 
-    if (nsteps > 0) {
-      load_stage(mlo);
-      store_stage(0, mlo);
+    // Steps [0, nh0) go to half 0, the rest to half 1; both run nh0.
+    const int nh0 = (nsteps + C::NH - 1) / C::NH;
+    const int my_first = qhalf * nh0;
+    const int my_count = qhalf == 0 ? nh0 : nsteps - nh0;
+    if (my_count > 0) {
+      load_stage(mlo + my_first * C::BMQ);
+      store_stage(0, mlo + my_first * C::BMQ);
     }
     __syncthreads();
-    for (int t = 0; t < nsteps; ++t) {
-      const int m0 = mlo + t * C::BMQ;
+    for (int t = 0; t < nh0; ++t) {
+      const int m0 = mlo + (my_first + t) * C::BMQ;
       const int st = (C::NSTAGE == 2) ? (t & 1) : 0;
-      if (C::NSTAGE == 2 && t + 1 < nsteps) load_stage(m0 + C::BMQ);
+      if (C::NSTAGE == 2 && t + 1 < my_count) load_stage(m0 + C::BMQ);
 
-      const int vis = ncols > 0 ? rect_visibility(md, m0, min(C::BMQ, sq - m0), n0w, ncols) : 0;
+      const int vis = ncols > 0 && t < my_count ? rect_visibility(md, m0, min(C::BMQ, sq - m0), n0w, ncols) : 0;
       if (vis) {
-        const unsigned char* base = smem_raw + st * C::STAGE_BYTES;
+        const unsigned char* base = smem_raw + qhalf * C::HALF_BYTES + st * C::STAGE_BYTES;
         const S* Qs = reinterpret_cast<const S*>(base);
         const S* Gs = Qs + C::QTILE;
         const S* QTs = Qs + 2 * C::QTILE;
@@ -271,18 +285,18 @@ __global__ __launch_bounds__(256) void bwd_dkdv_kernel(fa_bwd_params p, int num_
         for (int mb = 0; mb < C::NMB; ++mb) {
           sacc[mb] = zero16();
           pacc[mb] = zero16();
-          const S* qr = Qs + (mb * 32 + l32) * C::QLD + EL::E * h;
-          const S* gr = Gs + (mb * 32 + l32) * C::QLD + EL::E * h;
+          const S* qr = Qs + (mb * 32 + l32) * C::QLD;
+          const S* gr = Gs + (mb * 32 + l32) * C::QLD;
 #pragma unroll
           for (int s = 0; s < C::NSTEP; ++s) {
             Op kb_, vb_;
             if constexpr (C::KVREG) { kb_ = kop[s]; vb_ = vop[s]; }
             else {
-              kb_ = nvalid ? load_op<Tag>(krow + EL::KSTEP * s) : zero_op<Tag>();
-              vb_ = nvalid ? load_op<Tag>(vrow + EL::KSTEP * s) : zero_op<Tag>();
+              kb_ = nvalid ? load_op<Tag>(krow + kslot<Tag>(s, h)) : zero_op<Tag>();
+              vb_ = nvalid ? load_op<Tag>(vrow + kslot<Tag>(s, h)) : zero_op<Tag>();
             }
-            sacc[mb] = EL::mma(load_op<Tag>(qr + EL::KSTEP * s), kb_, sacc[mb]);
-            pacc[mb] = EL::mma(load_op<Tag>(gr + EL::KSTEP * s), vb_, pacc[mb]);
+            sacc[mb] = EL::mma(load_op<Tag>(qr + kslot<Tag>(s, h)), kb_, sacc[mb]);
+            pacc[mb] = EL::mma(load_op<Tag>(gr + kslot<Tag>(s, h)), vb_, pacc[mb]);
           }
         }
         // P_d -> sacc, dS -> pacc.
@@ -333,16 +347,36 @@ __global__ __launch_bounds__(256) void bwd_dkdv_kernel(fa_bwd_params p, int num_
         }
       }
       if (C::NSTAGE == 2) {
-        if (t + 1 < nsteps) store_stage(st ^ 1, m0 + C::BMQ);
+        if (t + 1 < my_count) store_stage(st ^ 1, m0 + C::BMQ);
         __syncthreads();
       } else {
         __syncthreads();
-        if (t + 1 < nsteps) {
+        if (t + 1 < my_count) {
           load_stage(m0 + C::BMQ);
           store_stage(0, m0 + C::BMQ);
         }
         __syncthreads();
       }
+    }
+  }
+
+  // First query half + second query half, in that order.
+  if constexpr (C::NH == 2) {
+    float* ow = reinterpret_cast<float*>(smem_raw) + wave * 2 * C::NDB * 1024;
+    __syncthreads();
+    if (qhalf == 1) {
+#pragma unroll
+      for (int db = 0; db < C::NDB; ++db) {
+        park_acc(ow + db * 1024, lane, dk[db]);
+        park_acc(ow + (C::NDB + db) * 1024, lane, dv[db]);
+      }
+    }
+    __syncthreads();
+    if (qhalf == 1) return;
+#pragma unroll
+    for (int db = 0; db < C::NDB; ++db) {
+      dk[db] += unpark_acc(ow + db * 1024, lane);
+      dv[db] += unpark_acc(ow + (C::NDB + db) * 1024, lane);
     }
   }
 
@@ -387,10 +421,15 @@ template <typename Tag, int D>
 struct DqCfg {
   using EL = Elem<Tag>;
   using S = typename EL::S;
-  static constexpr int NW = 4;
+  // fp32 up to D = 64: 64 rows, key tiles split by parity between two halves
+  // of two waves (see FwdCfg).
+  static constexpr int NH = (sizeof(S) == 4 && D <= 64) ? 2 : 1;
+  static constexpr int NWR = 4 / NH;
+  static constexpr int NW = NWR * NH;
   static constexpr int NT = 64 * NW;
-  static constexpr int BM = 32 * NW;
-  static constexpr int BN = (D <= 64) ? 64 : 32;
+  static constexpr int NTH = 64 * NWR;
+  static constexpr int BM = 32 * NWR;
+  static constexpr int BN = (D <= 64 && NH == 1) ? 64 : 32;
   static constexpr int DO = (D <= 128) ? D : ((sizeof(S) == 4 && D == 512) ? 64 : 128);
   static constexpr bool QREG = (sizeof(S) == 2) ? (D <= 128) : (D <= 64);
   static constexpr int KLD = D + EL::CE;
@@ -399,8 +438,10 @@ struct DqCfg {
   static constexpr int TTILE = DO * TLD;
   static constexpr int STAGE = 2 * KTILE + TTILE;  // K, V, K^T
   static constexpr int STAGE_BYTES = STAGE * (int)sizeof(S);
-  static constexpr int NSTAGE = (2 * STAGE_BYTES <= 160 * 1024) ? 2 : 1;
-  static constexpr int LDS_BYTES = NSTAGE * STAGE_BYTES;
+  static constexpr int NSTAGE = (2 * NH * STAGE_BYTES <= 160 * 1024) ? 2 : 1;
+  static constexpr int MERGE_BYTES = NH == 1 ? 0 : NWR * (DO / 32) * 4096;
+  static constexpr int LDS_BYTES = NH * NSTAGE * STAGE_BYTES > MERGE_BYTES ? NH * NSTAGE * STAGE_BYTES : MERGE_BYTES;
+  static_assert(NH == 1 || NSTAGE == 2, "two stages per half");
   static constexpr int NSTEP = D / EL::KSTEP;
   static constexpr int NKB = BN / 32;
   static constexpr int NPV = BN / (2 * EL::E);
@@ -418,7 +459,9 @@ __global__ __launch_bounds__(256) void bwd_dq_kernel(fa_bwd_params p, int num_m_
   const fa_fwd_params& f = p.fwd;
 
   const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform (SGPR)
+  const int wave_all = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform (SGPR)
+  const int khalf = wave_all / C::NWR, wave = wave_all % C::NWR;
+  const int htid = tid % C::NTH;
   const int h = lane >> 5, l32 = lane & 31;
   const int ndc = D / C::DO;
   const int bh_count = f.batch * f.heads_q;
@@ -458,15 +501,15 @@ __global__ __launch_bounds__(256) void bwd_dq_kernel(fa_bwd_params p, int num_m_
   const int m = m0w + l32;
   const bool mvalid = m < sq;
   const S* qrow = reinterpret_cast<const S*>(f.q) + b * f.q_stride[0] + hq * f.q_stride[1] +
-                  (int64_t)(q_start + (mvalid ? m : 0)) * f.q_stride[2] + EL::E * h;
+                  (int64_t)(q_start + (mvalid ? m : 0)) * f.q_stride[2];
   const S* grow = reinterpret_cast<const S*>(p.dout) + b * p.dout_stride[0] + hq * p.dout_stride[1] +
-                  (int64_t)(q_start + (mvalid ? m : 0)) * p.dout_stride[2] + EL::E * h;
+                  (int64_t)(q_start + (mvalid ? m : 0)) * p.dout_stride[2];
   Op qop[C::QREG ? C::NSTEP : 1], gop[C::QREG ? C::NSTEP : 1];
   if constexpr (C::QREG) {
 #pragma unroll
     for (int s = 0; s < C::NSTEP; ++s) {
-      qop[s] = mvalid ? load_op<Tag>(qrow + EL::KSTEP * s) : zero_op<Tag>();
-      gop[s] = mvalid ? load_op<Tag>(grow + EL::KSTEP * s) : zero_op<Tag>();
+      qop[s] = mvalid ? load_op<Tag>(qrow + kslot<Tag>(s, h)) : zero_op<Tag>();
+      gop[s] = mvalid ? load_op<Tag>(grow + kslot<Tag>(s, h)) : zero_op<Tag>();
     }
   }
   float lse2 = kNegInf, dlt = 0.f;
@@ -481,33 +524,35 @@ __global__ __launch_bounds__(256) void bwd_dq_kernel(fa_bwd_params p, int num_m_
 #pragma unroll
   for (int i = 0; i < C::NDB; ++i) dq[i] = zero16();
 
-  RowTile<Tag, C::BN, D, C::NT> kt, vt;
-  TransTile<Tag, C::BN, C::DO, C::NT> ktt;
+  RowTile<Tag, C::BN, D, C::NTH> kt, vt;
+  TransTile<Tag, C::BN, C::DO, C::NTH> ktt;
   auto load_stage = [&](int n0) {
-    kt.load([&](int r) -> const S* { int nn = n0 + r; return nn < sk ? kbase + (int64_t)nn * ks : nullptr; }, kbase, tid);
-    vt.load([&](int r) -> const S* { int nn = n0 + r; return nn < sk ? vbase + (int64_t)nn * vs : nullptr; }, vbase, tid);
+    kt.load([&](int r) -> const S* { int nn = n0 + r; return nn < sk ? kbase + (int64_t)nn * ks : nullptr; }, kbase, htid);
+    vt.load([&](int r) -> const S* { int nn = n0 + r; return nn < sk ? vbase + (int64_t)nn * vs : nullptr; }, vbase, htid);
     ktt.load([&](int r) -> const S* {
-      int nn = n0 + r; return nn < sk ? kbase + (int64_t)nn * ks + dc * C::DO : nullptr; }, kbase + dc * C::DO, tid);
+      int nn = n0 + r; return nn < sk ? kbase + (int64_t)nn * ks + dc * C::DO : nullptr; }, kbase + dc * C::DO, htid);
   };
   auto store_stage = [&](int st) {
-    S* base = smem + st * C::STAGE;
-    kt.store(base, C::KLD, tid);
-    vt.store(base + C::KTILE, C::KLD, tid);
-    ktt.store(base + 2 * C::KTILE, C::TLD, tid);
+    S* base = smem + (khalf * C::NSTAGE + st) * C::STAGE;
+    kt.store(base, C::KLD, htid);
+    vt.store(base + C::KTILE, C::KLD, htid);
+    ktt.store(base + 2 * C::KTILE, C::TLD, htid);
   };
 
-  if (ntiles > 0) {
-    load_stage(lo);
+  const int nh0 = (ntiles + C::NH - 1) / C::NH;
+  const int my_count = (ntiles - khalf + C::NH - 1) / C::NH;
+  if (my_count > 0) {
+    load_stage(lo + khalf * C::BN);
     store_stage(0);
   }
   __syncthreads();
-  for (int t = 0; t < ntiles; ++t) {
-    const int n0 = lo + t * C::BN;
+  for (int t = 0; t < nh0; ++t) {
+    const int n0 = lo + (khalf + C::NH * t) * C::BN;
     const int st = (C::NSTAGE == 2) ? (t & 1) : 0;
-    if (C::NSTAGE == 2 && t + 1 < ntiles) load_stage(n0 + C::BN);
-    const int vis = mrows > 0 ? rect_visibility(md, m0w, mrows, n0, C::BN) : 0;
+    if (C::NSTAGE == 2 && t + 1 < my_count) load_stage(n0 + C::NH * C::BN);
+    const int vis = mrows > 0 && t < my_count ? rect_visibility(md, m0w, mrows, n0, C::BN) : 0;
     if (vis) {
-      const S* Ks = smem + st * C::STAGE;
+      const S* Ks = smem + (khalf * C::NSTAGE + st) * C::STAGE;
       const S* Vs = Ks + C::KTILE;
       const S* KTs = Ks + 2 * C::KTILE;
       f32x16 sacc[C::NKB], pacc[C::NKB];
@@ -515,18 +560,18 @@ __global__ __launch_bounds__(256) void bwd_dq_kernel(fa_bwd_params p, int num_m_
       for (int kb2 = 0; kb2 < C::NKB; ++kb2) {
         sacc[kb2] = zero16();
         pacc[kb2] = zero16();
-        const S* kr = Ks + (kb2 * 32 + l32) * C::KLD + EL::E * h;
-        const S* vr = Vs + (kb2 * 32 + l32) * C::KLD + EL::E * h;
+        const S* kr = Ks + (kb2 * 32 + l32) * C::KLD;
+        const S* vr = Vs + (kb2 * 32 + l32) * C::KLD;
 #pragma unroll
         for (int s = 0; s < C::NSTEP; ++s) {
           Op qb_, gb_;
           if constexpr (C::QREG) { qb_ = qop[s]; gb_ = gop[s]; }
           else {
-            qb_ = mvalid ? load_op<Tag>(qrow + EL::KSTEP * s) : zero_op<Tag>();
-            gb_ = mvalid ? load_op<Tag>(grow + EL::KSTEP * s) : zero_op<Tag>();
+            qb_ = mvalid ? load_op<Tag>(qrow + kslot<Tag>(s, h)) : zero_op<Tag>();
+            gb_ = mvalid ? load_op<Tag>(grow + kslot<Tag>(s, h)) : zero_op<Tag>();
           }
-          sacc[kb2] = EL::mma(load_op<Tag>(kr + EL::KSTEP * s), qb_, sacc[kb2]);
-          pacc[kb2] = EL::mma(load_op<Tag>(vr + EL::KSTEP * s), gb_, pacc[kb2]);
+          sacc[kb2] = EL::mma(load_op<Tag>(kr + kslot<Tag>(s, h)), qb_, sacc[kb2]);
+          pacc[kb2] = EL::mma(load_op<Tag>(vr + kslot<Tag>(s, h)), gb_, pacc[kb2]);
         }
       }
 #pragma unroll
@@ -561,16 +606,29 @@ __global__ __launch_bounds__(256) void bwd_dq_kernel(fa_bwd_params p, int num_m_
       }
     }
     if (C::NSTAGE == 2) {
-      if (t + 1 < ntiles) store_stage(st ^ 1);
+      if (t + 1 < my_count) store_stage(st ^ 1);
       __syncthreads();
     } else {
       __syncthreads();
-      if (t + 1 < ntiles) {
-        load_stage(n0 + C::BN);
+      if (t + 1 < my_count) {
+        load_stage(n0 + C::NH * C::BN);
         store_stage(0);
       }
       __syncthreads();
     }
+  }
+
+  // First key half + second key half, in that order.
+  if constexpr (C::NH == 2) {
+    float* ow = reinterpret_cast<float*>(smem_raw) + wave * C::NDB * 1024;
+    if (khalf == 1) {
+#pragma unroll
+      for (int db = 0; db < C::NDB; ++db) park_acc(ow + db * 1024, lane, dq[db]);
+    }
+    __syncthreads();
+    if (khalf == 1) return;
+#pragma unroll
+    for (int db = 0; db < C::NDB; ++db) dq[db] += unpark_acc(ow + db * 1024, lane);
   }
 
   if (!mvalid) return;

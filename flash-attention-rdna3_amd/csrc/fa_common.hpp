@@ -108,6 +108,14 @@ __device__ inline typename Elem<Tag>::Op load_op(const typename Elem<Tag>::S* p)
   }
 }
 
+// First element of half h's k-slots of MFMA s over the contracted index.  fp32
+// slots are permuted so that four MFMAs take four consecutive elements of a
+// half: their operands then come as one 16-byte read.
+template <typename Tag>
+__device__ constexpr inline int kslot(int s, int h) {
+  return Elem<Tag>::E == 8 ? 16 * s + 8 * h : 8 * (s >> 2) + 4 * h + (s & 3);
+}
+
 template <typename Tag>
 __device__ inline typename Elem<Tag>::Op zero_op() {
   if constexpr (Elem<Tag>::E == 8) {

@@ -34,10 +34,20 @@ template <typename Tag, int D>
 struct FwdCfg {
   using EL = Elem<Tag>;
   using S = typename EL::S;
-  static constexpr int NW = 4;
+  // fp32 up to D = 128: 64 query rows (two waves) and their key tiles split
+  // by parity between two halves of two waves, merged through LDS.  A wave is
+  // MFMA-bound (64 cycles for 32x32x2), so what counts is that there are
+  // enough of them: 1 x 16 x 1000 rows in blocks of 128 left half the CUs
+  // idle.  At D = 64 the forward takes 61 us there against 100 us, dK/dV 119
+  // against 203, dQ 86 against 135 (the operands of four MFMAs in one LDS
+  // read, kslot, included); 4.1 / 8.2 / 6.1 GFLOP, card 153 TFLOP/s in fp32.
+  static constexpr int NH = (sizeof(S) == 4 && D <= 128) ? 2 : 1;
+  static constexpr int NWR = 4 / NH;          // row waves per half
+  static constexpr int NW = NWR * NH;
   static constexpr int NT = 64 * NW;
-  static constexpr int BM = 32 * NW;
-  static constexpr int BN = (D <= 128) ? 64 : 32;
+  static constexpr int NTH = 64 * NWR;        // threads per half
+  static constexpr int BM = 32 * NWR;
+  static constexpr int BN = (D <= 128 && !(NH == 2 && D == 128)) ? 64 : 32;
   // Output columns per workgroup: D > 128 splits O^T over the grid (each
   // split recomputes the scores) to bound the accumulator registers.
   static constexpr int DO = (D <= 128) ? D : ((sizeof(S) == 4 && D == 512) ? 64 : 128);
@@ -47,7 +57,9 @@ struct FwdCfg {
   static constexpr int KTILE = BN * KLD;
   static constexpr int VTILE = DO * VLD;
   static constexpr int STAGE = KTILE + VTILE;
-  static constexpr int LDS_BYTES = 2 * STAGE * (int)sizeof(S);
+  static constexpr int LOOP_BYTES = 2 * STAGE * (int)sizeof(S) * NH;
+  static constexpr int MERGE_BYTES = NH == 1 ? 0 : NWR * (DO / 32) * 4096 + 2 * NWR * 64 * 4;
+  static constexpr int LDS_BYTES = LOOP_BYTES > MERGE_BYTES ? LOOP_BYTES : MERGE_BYTES;
   static constexpr int NSTEP = D / EL::KSTEP;   // MFMA k-steps over D
   static constexpr int NKB = BN / 32;           // 32-key accumulator blocks
   static constexpr int NPV = BN / (2 * EL::E);  // P.V MFMAs per d-block
@@ -64,7 +76,9 @@ __global__ __launch_bounds__(256) void fwd_kernel(fa_fwd_params p, int num_m_blo
   S* smem = reinterpret_cast<S*>(smem_raw);
 
   const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform (SGPR)
+  const int wave_all = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform (SGPR)
+  const int khalf = wave_all / C::NWR, wave = wave_all % C::NWR;
+  const int htid = tid % C::NTH;
   const int h = lane >> 5, l32 = lane & 31;
 
   const int ndc = D / C::DO;
@@ -115,11 +129,11 @@ __global__ __launch_bounds__(256) void fwd_kernel(fa_fwd_params p, int num_m_blo
   const bool mvalid = m < sq;
 
   Op qop[C::QREG ? C::NSTEP : 1];
-  const S* qrow = qb + (int64_t)(mvalid ? m : 0) * qs + EL::E * h;
+  const S* qrow = qb + (int64_t)(mvalid ? m : 0) * qs;
   if constexpr (C::QREG) {
 #pragma unroll
     for (int s = 0; s < C::NSTEP; ++s)
-      qop[s] = mvalid ? load_op<Tag>(qrow + EL::KSTEP * s) : zero_op<Tag>();
+      qop[s] = mvalid ? load_op<Tag>(qrow + kslot<Tag>(s, h)) : zero_op<Tag>();
     wait_vm_all();
   }
 
@@ -128,45 +142,48 @@ __global__ __launch_bounds__(256) void fwd_kernel(fa_fwd_params p, int num_m_blo
 #pragma unroll
   for (int i = 0; i < C::NDB; ++i) acc[i] = zero16();
 
-  RowTile<Tag, C::BN, D, C::NT> kt;
-  TransTile<Tag, C::BN, C::DO, C::NT> vt;
+  RowTile<Tag, C::BN, D, C::NTH> kt;
+  TransTile<Tag, C::BN, C::DO, C::NTH> vt;
 
   auto load_tiles = [&](int n0) {
-    kt.load([&](int r) -> const S* { int n = n0 + r; return n < sk ? kb + (int64_t)n * ks : nullptr; }, kb, tid);
-    vt.load([&](int r) -> const S* { int n = n0 + r; return n < sk ? vb + (int64_t)n * vs : nullptr; }, vb, tid);
+    kt.load([&](int r) -> const S* { int n = n0 + r; return n < sk ? kb + (int64_t)n * ks : nullptr; }, kb, htid);
+    vt.load([&](int r) -> const S* { int n = n0 + r; return n < sk ? vb + (int64_t)n * vs : nullptr; }, vb, htid);
   };
   auto store_tiles = [&](int stage) {
-    S* base = smem + stage * C::STAGE;
-    kt.store(base, C::KLD, tid);
-    vt.store(base + C::KTILE, C::VLD, tid);
+    S* base = smem + (2 * khalf + stage) * C::STAGE;
+    kt.store(base, C::KLD, htid);
+    vt.store(base + C::KTILE, C::VLD, htid);
   };
 
-  if (ntiles > 0) {
-    load_tiles(lo);
+  // Half 0 takes the even key tiles, half 1 the odd ones; both run nh0 steps.
+  const int nh0 = (ntiles + C::NH - 1) / C::NH;
+  const int my_count = (ntiles - khalf + C::NH - 1) / C::NH;
+  if (my_count > 0) {
+    load_tiles(lo + khalf * C::BN);
     store_tiles(0);
   }
   __syncthreads();
 
-  for (int t = 0; t < ntiles; ++t) {
-    const int n0 = lo + t * C::BN;
+  for (int t = 0; t < nh0; ++t) {
+    const int n0 = lo + (khalf + C::NH * t) * C::BN;
     const int stage = t & 1;
-    if (t + 1 < ntiles) load_tiles(n0 + C::BN);
+    if (t + 1 < my_count) load_tiles(n0 + C::NH * C::BN);
 
-    const int vis = mrows > 0 ? rect_visibility(md, m0w, mrows, n0, C::BN) : 0;
+    const int vis = mrows > 0 && t < my_count ? rect_visibility(md, m0w, mrows, n0, C::BN) : 0;
     if (vis) {
-      const S* Ks = smem + stage * C::STAGE;
+      const S* Ks = smem + (2 * khalf + stage) * C::STAGE;
       const S* Vs = Ks + C::KTILE;
       f32x16 sacc[C::NKB];
 #pragma unroll
       for (int kb2 = 0; kb2 < C::NKB; ++kb2) {
         sacc[kb2] = zero16();
-        const S* krow = Ks + (kb2 * 32 + l32) * C::KLD + EL::E * h;
+        const S* krow = Ks + (kb2 * 32 + l32) * C::KLD;
 #pragma unroll
         for (int s = 0; s < C::NSTEP; ++s) {
-          Op a = load_op<Tag>(krow + EL::KSTEP * s);
+          Op a = load_op<Tag>(krow + kslot<Tag>(s, h));
           Op bq;
           if constexpr (C::QREG) bq = qop[s];
-          else bq = mvalid ? load_op<Tag>(qrow + EL::KSTEP * s) : zero_op<Tag>();
+          else bq = mvalid ? load_op<Tag>(qrow + kslot<Tag>(s, h)) : zero_op<Tag>();
           sacc[kb2] = EL::mma(a, bq, sacc[kb2]);
         }
       }
@@ -243,8 +260,35 @@ __global__ __launch_bounds__(256) void fwd_kernel(fa_fwd_params p, int num_m_blo
       }
     }
 
-    if (t + 1 < ntiles) store_tiles(stage ^ 1);
+    if (t + 1 < my_count) store_tiles(stage ^ 1);
     __syncthreads();
+  }
+
+  // Half 1 parks (O^T, m, l) in LDS, half 0 folds them in (as fwd16_item).
+  if constexpr (C::NH == 2) {
+    float* ow = reinterpret_cast<float*>(smem_raw);
+    float* mw = ow + C::NWR * C::NDB * 1024;
+    float* lw = mw + C::NWR * 64;
+    if (khalf == 1) {
+#pragma unroll
+      for (int db = 0; db < C::NDB; ++db) park_acc(ow + (wave * C::NDB + db) * 1024, lane, acc[db]);
+      mw[wave * 64 + lane] = m_i;
+      lw[wave * 64 + lane] = l_i;
+    }
+    __syncthreads();
+    if (khalf == 1) return;
+    const float m2 = mw[wave * 64 + lane], l2 = lw[wave * 64 + lane];
+    const float mn = fmaxf(m_i, m2);
+    const float mu = (mn == kNegInf) ? 0.f : mn;
+    const float sa = exp2f(m_i - mu), sb = exp2f(m2 - mu);
+#pragma unroll
+    for (int db = 0; db < C::NDB; ++db) {
+      const f32x16 o2 = unpark_acc(ow + (wave * C::NDB + db) * 1024, lane);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[db][i] = acc[db][i] * sa + o2[i] * sb;
+    }
+    l_i = l_i * sa + l2 * sb;
+    m_i = mn;
   }
 
   if (!mvalid) return;
