@@ -1,5 +1,5 @@
-// fa_torch.cpp - native host path of the dense forward / backward for
-// PyTorch callers.
+// fa_torch.cpp - native host path of the dense forward / backward and of
+// decode for PyTorch callers.
 //
 // The C ABI (include/fa_mi355x.h) takes plain pointers; this library is the
 // PyTorch-side caller of it for dense (B, H, S, D) attention.  It fills
@@ -17,6 +17,9 @@
 //             bias?, alibi?, dropout_p, dropout_seed) -> out   (differentiable)
 //   forward(...same...) -> (out, lse)
 //   backward(dout, q, k, v, out, lse, ...same options...) -> (dq, dk, dv)
+//   decode(q, k, v, new_k?, new_v?, lens?, ...) -> out    split-K decode, after
+//             writing new_k / new_v into the cache when given
+//   decode_paged(q, k_cache, v_cache, block_table, context_lens, ...) -> out
 //   set_ds_scratch_limit(bytes) / ds_scratch_limit() -> bytes
 // Argument contracts are checked by the Python layer with the reference's
 // messages before any of these is called; the C ABI re-checks what could
@@ -350,6 +353,156 @@ Tensor attention_op(const Tensor& q, const Tensor& k, const Tensor& v, bool caus
   return AttentionFn::apply(q, k, v, causal, scale, wl, wr, softcap, bias, alibi, dropout_p, seed);
 }
 
+// ---------------------------------------------------------------------------
+// Decode (reference interface.py:427-479, :643-728): tensors to the C ABI's
+// structs, output and split workspace from torch's allocator.  The Python
+// layer has checked the arguments, chosen the split count and passes the
+// stream's arrival counters (none: two-launch merge).  Filling the structs
+// through ctypes took most of a call's host time: the append + decode call
+// 42 us of host time, its two kernels 23 us.
+// ---------------------------------------------------------------------------
+Tensor decode_output(const Tensor& q, int64_t kdim) {
+  return at::empty({q.size(0), q.size(1), q.size(2), kdim}, q.options());
+}
+
+Tensor decode_workspace(const Tensor& q, int64_t kdim, int64_t num_splits) {
+  const size_t bytes = fa_decode_workspace_bytes((int)q.size(0), (int)q.size(1), (int)q.size(2), (int)kdim,
+                                                 (int)num_splits);
+  return at::empty({(int64_t)bytes}, q.options().dtype(at::kByte));
+}
+
+void check_with_query(const Tensor& q, std::initializer_list<const Tensor*> others) {
+  TORCH_CHECK(q.is_cuda() && q.dim() == 4, "fa_mi355x: query must be a 4-D GPU tensor");
+  for (const Tensor* t : others)
+    TORCH_CHECK(t->device() == q.device(), "fa_mi355x: all tensors must be on the query's device");
+}
+
+void append_rows(const Tensor& query, const Tensor& k_cache, const Tensor& v_cache, const Tensor& key,
+                 const Tensor& value, const Tensor& lens) {
+  const Tensor kn = kernel_ready(key), vn = kernel_ready(value);
+  fa_append_params p;
+  std::memset(&p, 0, sizeof(p));
+  p.abi_version = FA_ABI_VERSION;
+  p.dtype = dtype_code(query.scalar_type());
+  p.k_new = kn.data_ptr();
+  p.v_new = vn.data_ptr();
+  p.k_cache = k_cache.data_ptr();
+  p.v_cache = v_cache.data_ptr();
+  p.cache_seqlens = lens.data_ptr<int32_t>();
+  p.cache_seqlens_stride = lens.stride(0);
+  abi_strides4(p.k_new_stride, kn);
+  abi_strides4(p.v_new_stride, vn);
+  abi_strides4(p.k_cache_stride, k_cache);
+  abi_strides4(p.v_cache_stride, v_cache);
+  p.batch = (int32_t)k_cache.size(0);
+  p.heads_kv = (int32_t)k_cache.size(1);
+  p.seqlen_new = (int32_t)key.size(2);
+  p.seqlen_cache = (int32_t)k_cache.size(2);
+  p.head_dim = (int32_t)k_cache.size(3);
+  check_status(fa_kvcache_append(&p, stream_of(query)), "fa_kvcache_append");
+}
+
+Tensor decode_op(const Tensor& query, const Tensor& key, const Tensor& value, const OptTensor& new_key,
+                 const OptTensor& new_value, const OptTensor& lens, bool causal, double scale, int64_t num_splits,
+                 bool kv_fp8, double k_scale, double v_scale, const OptTensor& tickets) {
+  check_with_query(query, {&key, &value});
+  c10::DeviceGuard guard(query.device());
+  const int64_t head_dim = query.size(3), kdim = std::max(kMinKernelHeadDim, head_dim);
+  int64_t added = 0;
+  if (new_key.has_value()) {
+    added = new_key->size(2);
+    if (added > 0) append_rows(query, key, value, *new_key, *new_value, *lens);
+  }
+  // (fp8 caches have one of the kernels' head dims: no padding)
+  const Tensor q = kernel_ready(pad_head_dim(query, kdim));
+  const Tensor k = kernel_ready(kv_fp8 ? key : pad_head_dim(key, kdim));
+  const Tensor v = kernel_ready(kv_fp8 ? value : pad_head_dim(value, kdim));
+  const Tensor out = decode_output(query, kdim), ws = decode_workspace(query, kdim, num_splits);
+  fa_decode_params p;
+  std::memset(&p, 0, sizeof(p));
+  p.abi_version = FA_ABI_VERSION;
+  p.dtype = dtype_code(query.scalar_type());
+  p.q = q.data_ptr();
+  p.k = k.data_ptr();
+  p.v = v.data_ptr();
+  p.out = out.data_ptr();
+  abi_strides4(p.q_stride, q);
+  abi_strides4(p.k_stride, k);
+  abi_strides4(p.v_stride, v);
+  abi_strides4(p.out_stride, out);
+  p.batch = (int32_t)query.size(0);
+  p.heads_q = (int32_t)query.size(1);
+  p.heads_kv = (int32_t)key.size(1);
+  p.seqlen_q = (int32_t)query.size(2);
+  p.seqlen_k = (int32_t)key.size(2);
+  p.head_dim = (int32_t)kdim;
+  if (lens.has_value()) {
+    p.cache_seqlens = lens->data_ptr<int32_t>();
+    p.cache_seqlens_stride = lens->stride(0);
+  }
+  p.cache_seqlens_add = (int32_t)added;
+  p.softmax_scale = (float)scale;
+  p.num_splits = (int32_t)num_splits;
+  p.workspace = ws.data_ptr();
+  p.causal = causal ? 1 : 0;
+  if (kv_fp8) {
+    p.kv_fp8 = 1;
+    p.k_scale = (float)k_scale;
+    p.v_scale = (float)v_scale;
+  }
+  if (tickets.has_value()) p.tickets = reinterpret_cast<uint32_t*>(tickets->data_ptr<int32_t>());
+  check_status(fa_decode_splitk(&p, stream_of(query)), "fa_decode_splitk");
+  return kdim != head_dim ? out.narrow(-1, 0, head_dim) : out;
+}
+
+Tensor decode_paged_op(const Tensor& query, const Tensor& k_cache, const Tensor& v_cache, const Tensor& block_table,
+                       const Tensor& context_lens, bool causal, double scale, int64_t num_splits, bool kv_fp8,
+                       double k_scale, double v_scale, const OptTensor& tickets) {
+  check_with_query(query, {&k_cache, &v_cache, &block_table, &context_lens});
+  c10::DeviceGuard guard(query.device());
+  const int64_t head_dim = query.size(3), kdim = std::max(kMinKernelHeadDim, head_dim);
+  const Tensor q = kernel_ready(pad_head_dim(query, kdim));
+  const Tensor k = kernel_ready(kv_fp8 ? k_cache : pad_head_dim(k_cache, kdim));
+  const Tensor v = kernel_ready(kv_fp8 ? v_cache : pad_head_dim(v_cache, kdim));
+  const Tensor out = decode_output(query, kdim), ws = decode_workspace(query, kdim, num_splits);
+  fa_paged_params p;
+  std::memset(&p, 0, sizeof(p));
+  p.abi_version = FA_ABI_VERSION;
+  p.dtype = dtype_code(query.scalar_type());
+  p.q = q.data_ptr();
+  p.k_cache = k.data_ptr();
+  p.v_cache = v.data_ptr();
+  p.out = out.data_ptr();
+  p.block_table = block_table.data_ptr<int32_t>();
+  p.context_lens = context_lens.data_ptr<int32_t>();
+  abi_strides4(p.q_stride, q);
+  abi_strides4(p.k_stride, k);
+  abi_strides4(p.v_stride, v);
+  abi_strides4(p.out_stride, out);
+  for (int i = 0; i < 2; ++i) p.block_table_stride[i] = block_table.stride(i);
+  p.context_lens_stride = context_lens.stride(0);
+  p.batch = (int32_t)query.size(0);
+  p.heads_q = (int32_t)query.size(1);
+  p.heads_kv = (int32_t)k_cache.size(2);
+  p.head_dim = (int32_t)kdim;
+  p.num_blocks = (int32_t)k_cache.size(0);
+  p.block_size = (int32_t)k_cache.size(1);
+  p.max_blocks = (int32_t)block_table.size(1);
+  p.num_splits = (int32_t)num_splits;
+  p.softmax_scale = (float)scale;
+  p.seqlen_q = (int32_t)query.size(2);
+  p.workspace = ws.data_ptr();
+  p.causal = causal ? 1 : 0;
+  if (kv_fp8) {
+    p.kv_fp8 = 1;
+    p.k_scale = (float)k_scale;
+    p.v_scale = (float)v_scale;
+  }
+  if (tickets.has_value()) p.tickets = reinterpret_cast<uint32_t*>(tickets->data_ptr<int32_t>());
+  check_status(fa_decode_paged(&p, stream_of(query)), "fa_decode_paged");
+  return kdim != head_dim ? out.narrow(-1, 0, head_dim) : out;
+}
+
 int64_t set_ds_scratch_limit(int64_t bytes) {
   return g_ds_limit.exchange(bytes < 0 ? 0 : bytes);
 }
@@ -366,6 +519,10 @@ TORCH_LIBRARY(fa_mi355x, m) {
   m.def("backward(Tensor dout, Tensor q, Tensor k, Tensor v, Tensor out, Tensor lse, bool causal, float scale, "
         "int window_left, int window_right, float softcap, Tensor? bias, Tensor? alibi, float dropout_p, "
         "int dropout_seed) -> (Tensor, Tensor, Tensor)");
+  m.def("decode(Tensor q, Tensor(a!) k, Tensor(b!) v, Tensor? new_k, Tensor? new_v, Tensor? lens, bool causal, "
+        "float scale, int num_splits, bool kv_fp8, float k_scale, float v_scale, Tensor(c!)? tickets) -> Tensor");
+  m.def("decode_paged(Tensor q, Tensor k_cache, Tensor v_cache, Tensor block_table, Tensor context_lens, bool causal, "
+        "float scale, int num_splits, bool kv_fp8, float k_scale, float v_scale, Tensor(a!)? tickets) -> Tensor");
   m.def("set_ds_scratch_limit(int bytes) -> int", &set_ds_scratch_limit);
   m.def("ds_scratch_limit() -> int", &ds_scratch_limit);
 }
@@ -375,6 +532,8 @@ TORCH_LIBRARY_IMPL(fa_mi355x, CompositeImplicitAutograd, m) { m.impl("attention"
 TORCH_LIBRARY_IMPL(fa_mi355x, CUDA, m) {
   m.impl("forward", &forward_op);
   m.impl("backward", &backward_op);
+  m.impl("decode", &decode_op);
+  m.impl("decode_paged", &decode_paged_op);
 }
 
 TORCH_LIBRARY_IMPL(fa_mi355x, Meta, m) {

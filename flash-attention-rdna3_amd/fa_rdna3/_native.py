@@ -286,8 +286,8 @@ _tickets = {}
 
 
 def decode_tickets(device_tensor, batch, heads_q, seqlen_q):
-    """Address of zeroed uint32 arrival counters for one decode call on the
-    current stream of the tensor's device, or None for the two-launch merge.
+    """Zeroed int32 arrival counters for one decode call on the current
+    stream of the tensor's device, or None for the two-launch merge.
 
     The decode kernels leave every counter at zero, so one buffer per
     (device, stream) serves all calls issued in stream order; it grows when
@@ -314,7 +314,7 @@ def decode_tickets(device_tensor, batch, heads_q, seqlen_q):
             _retired_tickets.append(buf)
         buf = torch.zeros(size, dtype=torch.int32, device=device_tensor.device)
         _tickets[key] = buf
-    return buf.data_ptr()
+    return buf
 
 
 _retired_tickets = []

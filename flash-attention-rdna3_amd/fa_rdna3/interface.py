@@ -506,51 +506,23 @@ def _validate_fp8_kv(query, key, value, k_scale, v_scale):
         raise ValueError(f"fp8 KV caches need head_dim 32, 64, 128, 256 or 512, got {query.shape[3]}")
 
 
-def _decode_launch(query, key, value, softmax_scale, lens, causal, lens_add=0, fp8_scales=None):
+def _decode_launch(query, key, value, softmax_scale, lens, causal, new_rows=(None, None), fp8_scales=None):
     """Split-K decode launch shared by flash_attention_decode and
-    flash_attention_with_kvcache (arguments already validated)."""
+    flash_attention_with_kvcache (arguments already validated), after the
+    append of ``new_rows`` when given."""
     batch, heads, seqlen_q, head_dim = query.shape
     seqlen_k = key.shape[2]
     kdim = _kernel_head_dim(head_dim)
-    if fp8_scales is not None:
-        # fp8 rows: unit last stride and 16-byte aligned rows (contiguous copy
-        # otherwise); head_dim is one of the kernel's dims, so no padding.
-        q = _prep(query)[0]
-        k, v = _native.kernel_ready(key), _native.kernel_ready(value)
-    else:
-        q, k, v = _prep(_pad_head_dim(query, kdim), _pad_head_dim(key, kdim), _pad_head_dim(value, kdim))
     if kdim <= 128:
         group = heads // key.shape[1]
         num_splits = _streaming_decode_splits(batch, key.shape[1], group * seqlen_q, seqlen_k,
                                               _cu_count(query.device))
     else:
         num_splits = _decode_num_splits(batch, heads, seqlen_q, seqlen_k, 4 * _cu_count(query.device))
-    out = torch.empty((batch, heads, seqlen_q, kdim), dtype=query.dtype, device=query.device)
-    workspace = torch.empty(
-        _native.decode_workspace_bytes(batch, heads, seqlen_q, kdim, num_splits),
-        dtype=torch.uint8, device=query.device)
-    p = _native.DecodeParams()
-    p.abi_version = ABI_VERSION
-    p.dtype = DTYPE_CODE[query.dtype]
-    p.q, p.k, p.v, p.out = q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr()
-    for name, t in (("q_stride", q), ("k_stride", k), ("v_stride", v), ("out_stride", out)):
-        _set(getattr(p, name), _native.strides(t))
-    p.batch, p.heads_q, p.seqlen_q, p.head_dim = batch, heads, seqlen_q, kdim
-    p.heads_kv, p.seqlen_k = key.shape[1], seqlen_k
-    if lens is not None:
-        p.cache_seqlens = lens.data_ptr()
-        p.cache_seqlens_stride = lens.stride(0)
-    p.softmax_scale = softmax_scale
-    p.num_splits = num_splits
-    p.workspace = workspace.data_ptr()
-    p.tickets = _native.decode_tickets(query, batch, heads, seqlen_q)
-    p.causal = 1 if causal else 0
-    p.cache_seqlens_add = int(lens_add)
-    if fp8_scales is not None:
-        p.kv_fp8 = 1
-        p.k_scale, p.v_scale = fp8_scales
-    _native.call("fa_decode_splitk", p, query)
-    return out[..., :head_dim] if kdim != head_dim else out
+    k_scale, v_scale = fp8_scales if fp8_scales is not None else (1.0, 1.0)
+    return _native.ops().decode(query, key, value, new_rows[0], new_rows[1], lens, causal, softmax_scale, num_splits,
+                                fp8_scales is not None, k_scale, v_scale,
+                                _native.decode_tickets(query, batch, heads, seqlen_q))
 
 
 def _rows_vector_ready(t):
@@ -606,24 +578,8 @@ def flash_attention_with_kvcache(query, k_cache, v_cache, key=None, value=None, 
             if not _rows_vector_ready(t):
                 raise ValueError(f"{name} must have a unit last stride and 16-byte aligned rows "
                                  "to be updated in place")
-        seqlen_new = key.shape[2]
-        if seqlen_new > 0:
-            kn, vn = _native.kernel_ready(key), _native.kernel_ready(value)
-            p = _native.AppendParams()
-            p.abi_version = ABI_VERSION
-            p.dtype = DTYPE_CODE[query.dtype]
-            p.k_new, p.v_new = kn.data_ptr(), vn.data_ptr()
-            p.k_cache, p.v_cache = k_cache.data_ptr(), v_cache.data_ptr()
-            p.cache_seqlens, p.cache_seqlens_stride = cache_seqlens.data_ptr(), cache_seqlens.stride(0)
-            for name, t in (("k_new_stride", kn), ("v_new_stride", vn), ("k_cache_stride", k_cache),
-                            ("v_cache_stride", v_cache)):
-                _set(getattr(p, name), _native.strides(t))
-            p.batch, p.heads_kv, p.seqlen_new = batch, heads_kv, seqlen_new
-            p.seqlen_cache, p.head_dim = seqlen_cache, head_dim
-            _native.call("fa_kvcache_append", p, query)
     softmax_scale = 1.0 / math.sqrt(head_dim) if softmax_scale is None else float(softmax_scale)
-    return _decode_launch(query, k_cache, v_cache, softmax_scale, lens, causal=bool(causal),
-                          lens_add=0 if key is None else key.shape[2])
+    return _decode_launch(query, k_cache, v_cache, softmax_scale, lens, causal=bool(causal), new_rows=(key, value))
 
 
 # ---------------------------------------------------------------------------
@@ -806,7 +762,7 @@ def _paged_launch(query, k_cache, v_cache, block_table, context_lens, softmax_sc
     max_context_len = None if max_context_len is None else int(max_context_len)
     num_splits = None if num_splits is None else int(num_splits)
     batch, q_heads, seqlen_q, head_dim = query.shape
-    num_blocks, block_size, kv_heads = k_cache.shape[0], k_cache.shape[1], k_cache.shape[2]
+    block_size, kv_heads = k_cache.shape[1], k_cache.shape[2]
     softmax_scale = 1.0 / math.sqrt(head_dim) if softmax_scale is None else float(softmax_scale)
 
     kdim = _kernel_head_dim(head_dim)
@@ -820,38 +776,10 @@ def _paged_launch(query, k_cache, v_cache, block_table, context_lens, softmax_sc
         splits = int(_paged_num_splits(batch, q_heads, block_size, block_table.shape[1],
                                        2 * _cu_count(query.device), max_context_len=max_context_len,
                                        requested_splits=num_splits))
-    if fp8_scales is not None:
-        q, kc, vc = _prep(query, k_cache, v_cache)  # head_dim is a kernel dim: no padding
-    else:
-        q, kc, vc = _prep(_pad_head_dim(query, kdim), _pad_head_dim(k_cache, kdim),
-                          _pad_head_dim(v_cache, kdim))
-    out = torch.empty((batch, q_heads, seqlen_q, kdim), dtype=query.dtype, device=query.device)
-    workspace = torch.empty(_native.decode_workspace_bytes(batch, q_heads, seqlen_q, kdim, splits),
-                            dtype=torch.uint8, device=query.device)
-    p = _native.PagedParams()
-    p.abi_version = ABI_VERSION
-    p.dtype = DTYPE_CODE[query.dtype]
-    p.q, p.k_cache, p.v_cache, p.out = q.data_ptr(), kc.data_ptr(), vc.data_ptr(), out.data_ptr()
-    p.block_table, p.context_lens = block_table.data_ptr(), context_lens.data_ptr()
-    _set(p.q_stride, _native.strides(q))
-    _set(p.k_stride, _native.strides(kc))
-    _set(p.v_stride, _native.strides(vc))
-    _set(p.out_stride, _native.strides(out))
-    _set(p.block_table_stride, block_table.stride())
-    p.context_lens_stride = context_lens.stride(0)
-    p.batch, p.heads_q, p.heads_kv, p.head_dim = batch, q_heads, kv_heads, kdim
-    p.num_blocks, p.block_size, p.max_blocks = num_blocks, block_size, block_table.shape[1]
-    p.num_splits = splits
-    p.softmax_scale = softmax_scale
-    p.seqlen_q = seqlen_q
-    p.causal = 1 if causal else 0
-    if fp8_scales is not None:
-        p.kv_fp8 = 1
-        p.k_scale, p.v_scale = fp8_scales
-    p.workspace = workspace.data_ptr()
-    p.tickets = _native.decode_tickets(query, batch, q_heads, seqlen_q)
-    _native.call("fa_decode_paged", p, query)
-    return out[..., :head_dim] if kdim != head_dim else out
+    k_scale, v_scale = fp8_scales if fp8_scales is not None else (1.0, 1.0)
+    return _native.ops().decode_paged(query, k_cache, v_cache, block_table, context_lens, causal, softmax_scale,
+                                      splits, fp8_scales is not None, k_scale, v_scale,
+                                      _native.decode_tickets(query, batch, q_heads, seqlen_q))
 
 
 def flash_attention_decode_paged_multi(query, k_cache, v_cache, block_table, context_lens, softmax_scale=None,
