@@ -183,13 +183,14 @@ __device__ __forceinline__ void fwd16_item(const fa_fwd_params& p, int num_m_blo
     v_next += (int64_t)(TSTEP * C::BN) * vs;
   };
   const VisBounds vbnd = row_block_bounds(md, m0w, mrows);
-  // Wide heads and the dense fp16 form with one key half follow the max
+  // fp16 wide heads and the dense fp16 form with one key half follow the max
   // exactly: the largest weights are then 1 or just below it, where a 16-bit
   // float rounds least.  (The split form keeps two maxima per row, which is
   // as good as that; bf16 carries P in two parts.)  Output error against 64
   // bits, lazy and exact: 2.92e-4 and 2.84e-4 of the norm at 2 x 10 x 4096 x 64,
   // 2.93e-4 and 2.78e-4 at 1 x 1 x 4096 x 512.
-  const bool exact_max = D > 128 || (NH == 1 && std::is_same<Tag, f16_t>::value && p.cu_seqlens_q == nullptr);
+  const bool exact_max =
+      std::is_same<Tag, f16_t>::value && (D > 128 || (NH == 1 && p.cu_seqlens_q == nullptr));
   const float lazy = exact_max ? 0.f : kLazyRescale;
 
   // The first tiles' DMA and the Q loads share one round trip to memory.
@@ -463,58 +464,6 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void fwd16_split_kernel(fa_fw
   const int item = blockIdx.x / nsplit;
   fwd16_item<Tag, D, MODE, 1, true>(p, num_m_blocks, item, smem_raw, false, blockIdx.x - item * nsplit, nsplit,
                                     ws + (int64_t)blockIdx.x * Fwd16Cfg<D, 1>::PART);
-}
-
-// Merge of fwd16_split_kernel's shares, 64 output columns of one row block
-// per workgroup: O = sum_s 2^(m_s - M) O_s / sum_s 2^(m_s - M) l_s in the
-// accumulator layout the shares were parked in (1 KiB per load), then whole
-// 128-byte row pieces through LDS.
-template <typename Tag, int D>
-__global__ __launch_bounds__(256) void fwd16_merge_kernel(fa_fwd_params p, int num_m_blocks, int nsplit,
-                                                          const float* ws) {
-  using C = Fwd16Cfg<D, 1>;
-  using S = uint16_t;
-  constexpr int MD = 64;  // columns per workgroup
-  constexpr int PER = C::DO / MD;
-  __shared__ __align__(16) uint16_t stage[C::NQ * 32 * (MD + 8)];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int h = lane >> 5, l32 = lane & 31;
-  const int cc = blockIdx.x % PER;
-  const int item = blockIdx.x / PER;
-  const int dc = item % C::NDC;
-  const int bh_count = p.batch * p.heads_q;
-  const int mb_rev = item / C::NDC / bh_count;
-  const int bh = item / C::NDC - mb_rev * bh_count;
-  const int b = bh / p.heads_q, hq = bh - b * p.heads_q;
-  const int m0w = (num_m_blocks - 1 - mb_rev) * C::BM + 32 * wave;
-  const int mrows = min(32, p.seqlen_q - m0w);
-  const float* src = ws + (int64_t)item * nsplit * C::PART;
-  float M = kNegInf;
-  for (int s = 0; s < nsplit; ++s) M = fmaxf(M, src[(int64_t)s * C::PART + C::PART_O + 32 * wave + l32]);
-  const float Mu = (M == kNegInf) ? 0.f : M;
-  float L = 0.f;
-  f32x16 acc[MD / 32];
-#pragma unroll
-  for (int i = 0; i < MD / 32; ++i) acc[i] = zero16();
-  for (int s = 0; s < nsplit; ++s) {
-    const float* ps = src + (int64_t)s * C::PART;
-    const float w = __builtin_amdgcn_exp2f(ps[C::PART_O + 32 * wave + l32] - Mu);
-    L += ps[C::PART_O + C::BM + 32 * wave + l32] * w;
-#pragma unroll
-    for (int i = 0; i < MD / 32; ++i) {
-      const f32x16 o = unpark_acc(ps + (wave * C::NDB + cc * (MD / 32) + i) * 1024, lane);
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][e] += o[e] * w;
-    }
-  }
-  const float l_safe = (L == 0.f) ? 1.f : L;
-  S* orow0 = reinterpret_cast<S*>(p.out) + b * p.out_stride[0] + hq * p.out_stride[1] +
-             (int64_t)m0w * p.out_stride[2] + dc * C::DO + cc * MD;
-  store_rows_staged<Tag, MD>(acc, 1.f / l_safe, stage + wave * 32 * (MD + 8), orow0, p.out_stride[2], mrows, lane);
-  if (l32 < mrows && h == 0 && dc == 0 && cc == 0)
-    p.lse[b * p.lse_stride[0] + hq * p.lse_stride[1] + (int64_t)(m0w + l32) * p.lse_stride[2]] =
-        (M == kNegInf || L == 0.f) ? kNegInf : (M + __log2f(l_safe)) * kLn2;
 }
 
 }  // namespace fa

@@ -337,9 +337,7 @@ static hipError_t launch_fwd16_split(const fa_fwd_params& p, int nmb, int nsplit
   hipLaunchKernelGGL(kern, dim3(items * nsplit), dim3(C::NT), C::LDS_BYTES, stream, p, nmb, nsplit, ws);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((fwd16_merge_kernel<Tag, D>), dim3(items * (C::DO / 64)), dim3(256), 0, stream, p, nmb, nsplit,
-                     (const float*)ws);
-  return hipGetLastError();
+  return launch_fwd_merge(p, nmb, nsplit, ws, stream);
 }
 
 template <typename Tag, int D, int MODE>

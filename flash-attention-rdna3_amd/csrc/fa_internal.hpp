@@ -24,6 +24,8 @@ struct FwdScratch {
 // states take.
 int fwd_split_count(const fa_fwd_params& p);
 size_t fwd_workspace_bytes(const fa_fwd_params& p);
+// Output of a split forward from its shares' states (fwd16_split_kernel).
+hipError_t launch_fwd_merge(const fa_fwd_params& p, int nmb, int nsplit, const float* ws, hipStream_t stream);
 
 // Each launcher validates nothing beyond what it needs to pick a kernel
 // instantiation; fa_api.cpp has already checked the arguments.  They return
