@@ -1,11 +1,51 @@
 // Dtype dispatch of the bwd kernels (instantiated in fa_bwd_{f16,bf16,f32}.hip).
 #include "fa_internal.hpp"
-#include "fa_common.hpp"
+#include "fa_bwd_roles.hpp"
 
 namespace fa {
 
 template <typename Tag>
 hipError_t bwd_by_mods(const fa_bwd_params& p, int ph, hipStream_t s);
+
+// Shares of the D = 256 dK/dV pass: a grid that would leave half the CUs
+// idle is split until it fills them (at least eight query steps of 32 rows
+// each), and a causal grid of one round at most in two, since it lasts as long
+// as its heaviest block, twice the mean (1 x 16/8 x 2048 x 256 bf16: dK/dV
+// 150 -> 108 us and 14 for the merge).  At 1 x 4 x 500 x 256, two shares of
+// eight steps, it is 26.7 -> 21.2 + 4.3 us.
+int bwd_share_count(const fa_bwd_params& p) {
+  const fa_fwd_params& f = p.fwd;
+  if (f.dtype == FA_DTYPE_F32 || f.head_dim != 256 || f.cu_seqlens_q) return 1;
+  if (f.batch <= 0 || f.heads_q <= 0 || f.heads_kv <= 0 || f.seqlen_q <= 0 || f.seqlen_k <= 0) return 1;
+  // (problems that may run in chunks of KV heads have none, whole or chunked)
+  if (bwd_share_offset(p) >= kDsMinChunkBytes) return 1;
+  const int64_t groups = ((int64_t)f.seqlen_k + 63) / 64 * f.batch * f.heads_kv;
+  const int64_t steps = ((int64_t)f.seqlen_q + 31) / 32;
+  const int64_t cus = device_cu_count();
+  if (groups > cus) return 1;
+  if (groups * 2 > cus) return f.causal && steps >= 32 ? 2 : 1;
+  return (int)std::max<int64_t>(1, std::min({cus / groups, steps / 8, (int64_t)8}));
+}
+
+int64_t bwd_share_offset(const fa_bwd_params& p) {
+  const fa_fwd_params& f = p.fwd;
+  return (int64_t)f.batch * f.heads_q * ds_region_elems(f.seqlen_q, f.seqlen_k) * 2 + 1024;
+}
+
+template <typename Tag>
+static hipError_t run_dkdv_merge(const fa_bwd_params& p, int nshare, bool softcap4, hipStream_t s) {
+  const fa_fwd_params& f = p.fwd;
+  const unsigned items = (unsigned)((f.seqlen_k + 63) / 64 * f.batch * f.heads_kv);
+  const float* part = reinterpret_cast<const float*>(static_cast<const char*>(p.ds_workspace) + bwd_share_offset(p));
+  if (softcap4) hipLaunchKernelGGL((dkdv_merge_kernel<Tag, 256, true>), dim3(items * 4), dim3(256), 0, s, p, nshare, part);
+  else hipLaunchKernelGGL((dkdv_merge_kernel<Tag, 256, false>), dim3(items * 4), dim3(256), 0, s, p, nshare, part);
+  return hipGetLastError();
+}
+
+hipError_t launch_dkdv_merge(const fa_bwd_params& p, int nshare, bool softcap4, hipStream_t s) {
+  return p.fwd.dtype == FA_DTYPE_F16 ? run_dkdv_merge<f16_t>(p, nshare, softcap4, s)
+                                     : run_dkdv_merge<bf16_t>(p, nshare, softcap4, s);
+}
 
 size_t bwd_ds_bytes(const fa_bwd_params& p) {
   const fa_fwd_params& f = p.fwd;
@@ -22,7 +62,10 @@ size_t bwd_ds_bytes(const fa_bwd_params& p) {
   } else {
     elems = (int64_t)f.batch * f.heads_q * ds_region_elems(f.seqlen_q, f.seqlen_k);
   }
-  return (size_t)elems * 2 + 1024;
+  size_t bytes = (size_t)elems * 2 + 1024;
+  if (const int n = bwd_share_count(p); n > 1)  // 64 keys of dK and dV in fp32 per share
+    bytes += ((size_t)f.seqlen_k + 63) / 64 * f.batch * f.heads_kv * n * (2 * 64 * 256 * 4);
+  return bytes;
 }
 
 size_t bwd_ds_chunk_bytes(const fa_bwd_params& p, int kv_heads) {

@@ -660,15 +660,28 @@ template <typename Tag, int D, int MODE>
 static hipError_t run_bwd_dkdv16(const fa_bwd_params& p, hipStream_t stream) {
   constexpr bool ROLES = D > 128;
   using C = typename std::conditional<ROLES, DkdvRolesCfg<D>, Dkdv16Cfg<D>>::type;
-  void (*kern)(fa_bwd_params, int);
-  if constexpr (ROLES) kern = dkdv_roles_kernel<Tag, D, MODE>;
-  else kern = dkdv16_kernel<Tag, D, MODE>;
-  hipError_t e = allow_lds((const void*)kern, C::LDS_BYTES);
-  if (e != hipSuccess) return e;
   const int nnb = (p.fwd.seqlen_k + C::BN - 1) / C::BN;
   const long grid = (long)nnb * p.fwd.batch * p.fwd.heads_kv;
+  if constexpr (ROLES) {
+    auto kern = dkdv_roles_kernel<Tag, D, MODE>;
+    hipError_t e = allow_lds((const void*)kern, C::LDS_BYTES);
+    if (e != hipSuccess) return e;
+    // (ds_workspace is set only when it holds bwd_ds_bytes)
+    const int nshare = p.ds_workspace ? bwd_share_count(p) : 1;
+    float* part = nshare > 1
+                      ? reinterpret_cast<float*>(static_cast<char*>(p.ds_workspace) + bwd_share_offset(p))
+                      : nullptr;
+    hipLaunchKernelGGL(kern, dim3((unsigned)(grid * nshare)), dim3(C::NT), C::LDS_BYTES, stream, p, nnb, nshare, part);
+    e = hipGetLastError();
+    if (e != hipSuccess || nshare == 1) return e;
+    return launch_dkdv_merge(p, nshare, MODE == 3, stream);
+  } else {
+  auto kern = dkdv16_kernel<Tag, D, MODE>;
+  hipError_t e = allow_lds((const void*)kern, C::LDS_BYTES);
+  if (e != hipSuccess) return e;
   hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(C::NT), C::LDS_BYTES, stream, p, nnb);
   return hipGetLastError();
+  }
 }
 
 template <typename Tag, int D, int OCC, bool PAIR = false, bool VARLEN = false>

@@ -56,8 +56,12 @@ struct DkdvRolesCfg {
   static_assert(32 * (D + 8) * 2 <= PARK_WAVE_BYTES, "rows leave through the wave's merge block");
 };
 
+// nshare > 1: the query steps of a key block (of each of its query heads) are
+// shared out over nshare workgroups, blockIdx = (block, KV head) * nshare +
+// share, which leave their sums in `part` for dkdv_merge_kernel.
 template <typename Tag, int D, int MODE>
-__global__ __launch_bounds__(512, 1) void dkdv_roles_kernel(fa_bwd_params p, int num_n_blocks) {
+__global__ __launch_bounds__(512, 1) void dkdv_roles_kernel(fa_bwd_params p, int num_n_blocks, int nshare,
+                                                            float* part) {
   using C = DkdvRolesCfg<D>;
   using EL = Elem<Tag>;
   using S = uint16_t;
@@ -76,8 +80,10 @@ __global__ __launch_bounds__(512, 1) void dkdv_roles_kernel(fa_bwd_params p, int
   const int h = lane >> 5, l32 = lane & 31;
   const int bhk_count = f.batch * f.heads_kv;
   // Low key blocks first: under causal masking they see the most query rows.
-  const int nblk = blockIdx.x / bhk_count;
-  const int bhk = blockIdx.x - nblk * bhk_count;
+  const int item = blockIdx.x / nshare;
+  const int share = blockIdx.x - item * nshare;
+  const int nblk = item / bhk_count;
+  const int bhk = item - nblk * bhk_count;
   const int b = bhk / f.heads_kv, hk = bhk - b * f.heads_kv;
   const int group = f.heads_q / f.heads_kv;
 
@@ -150,7 +156,10 @@ __global__ __launch_bounds__(512, 1) void dkdv_roles_kernel(fa_bwd_params p, int
     if (f.window_right >= 0) mlo = max(mlo, n0 - md.off - f.window_right);
     if (f.window_left >= 0) mhi = min(mhi, nlast - md.off + f.window_left + 1);
     mlo = max(mlo, 0) / C::BMQ * C::BMQ;
-    const int nsteps = mhi > mlo ? (mhi - mlo + C::BMQ - 1) / C::BMQ : 0;
+    int nsteps = mhi > mlo ? (mhi - mlo + C::BMQ - 1) / C::BMQ : 0;
+    const int step0 = nsteps * share / nshare;
+    nsteps = nsteps * (share + 1) / nshare - step0;
+    mlo += step0 * C::BMQ;
     // Steps [0, nh0) go to half 0, [nh0, nsteps) to half 1; both run nh0
     // iterations so their barriers line up.
     const int nh0 = (nsteps + 1) / 2;
@@ -391,6 +400,14 @@ __global__ __launch_bounds__(512, 1) void dkdv_roles_kernel(fa_bwd_params p, int
 #pragma unroll
       for (int db = 0; db < C::NDB; ++db) acc[kb][db] += unpark_acc(ow + (kb * C::NDB + db) * 1024, lane);
   }
+  if (nshare > 1) {
+    float* pw = part + ((int64_t)blockIdx.x * 2 * C::NK + slot) * (KB * C::NDB * 1024);
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+      for (int db = 0; db < C::NDB; ++db) park_acc(pw + (kb * C::NDB + db) * 1024, lane, acc[kb][db]);
+    return;
+  }
   // Whole-row stores through this wave's merge block (read back already).
   const int64_t ost = kwave ? p.dk_stride[2] : p.dv_stride[2];
   S* orow0 = kwave ? reinterpret_cast<S*>(p.dk) + b * p.dk_stride[0] + hk * p.dk_stride[1]
@@ -401,6 +418,40 @@ __global__ __launch_bounds__(512, 1) void dkdv_roles_kernel(fa_bwd_params p, int
   for (int kb = 0; kb < KB; ++kb)
     store_rows_staged<Tag, D>(acc[kb], sc, stage, orow0 + (int64_t)(k_start + n0w + 32 * kb) * ost, ost,
                               ncols - 32 * kb, lane);
+}
+
+// dK / dV of the shares above, added in share order: 64 columns of one item
+// per workgroup, one wave per (pair, role).
+template <typename Tag, int D, bool CAP4>
+__global__ __launch_bounds__(256) void dkdv_merge_kernel(fa_bwd_params p, int nshare, const float* part) {
+  using C = DkdvRolesCfg<D>;
+  using S = uint16_t;
+  constexpr int MD = 64, PER = D / MD;
+  static_assert(C::KB == 1 && 2 * C::NK == 4, "one wave per merge block");
+  __shared__ __align__(16) uint16_t stage[4 * 32 * (MD + 8)];
+  const fa_fwd_params& f = p.fwd;
+  const int lane = threadIdx.x & 63;
+  const int slot = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const bool kwave = (slot & 1) != 0;
+  const int cc = blockIdx.x % PER, item = blockIdx.x / PER;
+  const int bhk_count = f.batch * f.heads_kv;
+  const int nblk = item / bhk_count, bhk = item - nblk * bhk_count;
+  const int b = bhk / f.heads_kv, hk = bhk - b * f.heads_kv;
+  const int n0w = nblk * C::BN + 32 * (slot >> 1);
+  f32x16 acc[MD / 32];
+#pragma unroll
+  for (int i = 0; i < MD / 32; ++i) acc[i] = zero16();
+  for (int s = 0; s < nshare; ++s) {
+    const float* pw = part + (((int64_t)item * nshare + s) * 4 + slot) * (C::NDB * 1024) + cc * (MD / 32) * 1024;
+#pragma unroll
+    for (int i = 0; i < MD / 32; ++i) acc[i] += unpark_acc(pw + i * 1024, lane);
+  }
+  const int64_t ost = kwave ? p.dk_stride[2] : p.dv_stride[2];
+  S* orow0 = kwave ? reinterpret_cast<S*>(p.dk) + b * p.dk_stride[0] + hk * p.dk_stride[1]
+                   : reinterpret_cast<S*>(p.dv) + b * p.dv_stride[0] + hk * p.dv_stride[1];
+  const float sc = kwave ? f.softmax_scale * (CAP4 ? 4.f : 1.f) : 1.f;
+  store_rows_staged<Tag, MD>(acc, sc, stage + slot * 32 * (MD + 8), orow0 + (int64_t)n0w * ost + cc * MD, ost,
+                             min(32, f.seqlen_k - n0w), lane);
 }
 
 }  // namespace fa

@@ -104,6 +104,8 @@ def test_no_splits_without_room_to_gain():
     (4, 2, 333, 700, {"causal": True}), (2, 1, 500, 500, {"softcap": 10.0}),
     (2, 2, 500, 500, {"causal": True, "window": (90, 0), "softcap": 30.0}),
     (2, 2, 400, 257, {"bias": True, "window": (100, 60)}), (2, 2, 257, 400, {"alibi": True, "causal": True}),
+    (2, 1, 1100, 900, {"causal": True, "softcap": 20.0}),  # dK/dV in four shares of the query steps
+    (4, 2, 2000, 300, {}), (16, 8, 2000, 2048, {"causal": True}),  # seven shares; a full grid in two
 ])
 def test_backward_256(dtype, heads, kv, sq, sk, opts):
     gen = torch.Generator().manual_seed(sq + 3 * sk)
