@@ -11,7 +11,7 @@ hipError_t fwd_by_mods(const fa_fwd_params& p, const FwdScratch& w, hipStream_t 
 // too few blocks (an autoencoder's single head of 4096 rows is 64 workgroups),
 // or a causal grid of one round at most, which lasts as long as its heaviest
 // block, twice the mean (1 x 16 x 2048 x 256 bf16: 115 us, in two shares 77
-// and 10 for their merge).  Each share keeps at least four 32-key tiles, so
+// and 15 for their merge).  Each share keeps at least four 32-key tiles, so
 // its state (512 KiB at most per 128 rows) costs less to store and merge than
 // the keys it takes over.
 int fwd_split_count(const fa_fwd_params& p) {

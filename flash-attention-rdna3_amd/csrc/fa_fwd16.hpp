@@ -41,9 +41,10 @@ namespace fa {
 // the 128 rows and no merge is needed.  Its 64 KiB of LDS and 4 waves let two
 // workgroups share a CU, so one workgroup's prologue (Q and first tiles) and
 // epilogue (output store) overlap the other's steady state.  It is launched
-// when the grid spans many rounds of workgroups (a packed varlen batch),
-// where that per-workgroup cost adds up; a short causal batch keeps NH = 2,
-// whose key split lets a heavy block use the whole CU.
+// for packed varlen batches, for causal grids of many rounds of workgroups,
+// where that per-workgroup cost adds up, and for blocks of equal cost that
+// outnumber the CUs; a short causal batch keeps NH = 2, whose key split lets
+// a heavy block use the whole CU.
 template <int D, int NH = 2>
 struct Fwd16Cfg {
   static constexpr int NQ = 4;                 // row quarters (waves per half)
@@ -154,8 +155,13 @@ __device__ __forceinline__ void fwd16_item(const fa_fwd_params& p, int num_m_blo
 #pragma unroll
   for (int i = 0; i < C::NDB; ++i) acc[i] = zero16();
 
-  DmaLeanTile<C::BN, D, C::NTH> kt;
-  DmaLeanTile<C::BN, C::DO, C::NTH> vt;
+  // Tile addresses in few registers (row_op, tr_op, DmaLeanTile) for wide heads,
+  // which need them, and fp16 (up to 3 % faster); bf16 up to D = 128 runs 1 %
+  // faster with an address per operand (1 x 32/8 x 8000 x 128 causal 785-788
+  // against 787-796 us, 1 x 16/4 x 4000 x 64 82 against 83).
+  constexpr bool LEAN = D > 128 || std::is_same<Tag, f16_t>::value;
+  typename std::conditional<LEAN, DmaLeanTile<C::BN, D, C::NTH>, DmaSwzTile<C::BN, D, C::NTH>>::type kt;
+  typename std::conditional<LEAN, DmaLeanTile<C::BN, C::DO, C::NTH>, DmaSwzTile<C::BN, C::DO, C::NTH>>::type vt;
   kt.init(ks, htid);
   vt.init(vs, htid);
   // Both halves run nh0 steps so their barriers line up.
@@ -214,7 +220,8 @@ __device__ __forceinline__ void fwd16_item(const fa_fwd_params& p, int num_m_blo
     if (!vis && t + 1 < my_count) load_tiles(stage ^ 1);
     if (vis) {
       const uint32_t ktile = lds0 + (uint32_t)(stage * C::STAGE) * 2u;
-      const uint32_t ka = tile_lane(ktile, row_off);
+      const S* const Ks = smem + khalf * C::HALF + stage * C::STAGE;
+      const uint32_t ka = LEAN ? tile_lane(ktile, row_off) : 0u;
       f32x16 sacc[C::NKB];
 #pragma unroll
       for (int kb2 = 0; kb2 < C::NKB; ++kb2) sacc[kb2] = zero16();
@@ -222,7 +229,7 @@ __device__ __forceinline__ void fwd16_item(const fa_fwd_params& p, int num_m_blo
       for (int s = 0; s < C::NSTEP; ++s)
 #pragma unroll
         for (int kb2 = 0; kb2 < C::NKB; ++kb2)
-          sacc[kb2] = EL::mma(row_op<D>(ka, s, kb2), qop[s], sacc[kb2]);
+          sacc[kb2] = EL::mma(LEAN ? row_op<D>(ka, s, kb2) : swz_op<D>(Ks, kb2 * 32 + l32, 2 * s + h), qop[s], sacc[kb2]);
       sched_read_ahead<C::NSTEP * C::NKB, 4>();
       // The next tile's loads go out while the score MFMAs drain (issuing
       // them before the MFMAs would hold the MFMAs back behind the queue).
@@ -361,12 +368,12 @@ __device__ __forceinline__ void fwd16_item(const fa_fwd_params& p, int num_m_blo
 #pragma unroll
         for (int j = 0; j < C::NPV; ++j) pl[j] = pack_op<Tag>(sacc[j >> 1], j & 1);
       }
-      const uint32_t va = tile_lane(ktile + C::KTILE * 2u, tr_off);
+      const uint32_t va = LEAN ? tile_lane(ktile + C::KTILE * 2u, tr_off) : 0u;
 #pragma unroll
       for (int j = 0; j < C::NPV; ++j)
 #pragma unroll
         for (int db = 0; db < C::NDB; ++db) {
-          const s16x8 a = tr_op<C::DO>(va, j, db);
+          const s16x8 a = LEAN ? tr_op<C::DO>(va, j, db) : tr_op_rowmap<C::DO>(Ks + C::KTILE, 0, 32 * db, j, lane);
           acc[db] = EL::mma(a, pb[j], acc[db]);
           if constexpr (PSPLIT) acc[db] = EL::mma(a, pl[j], acc[db]);
         }
