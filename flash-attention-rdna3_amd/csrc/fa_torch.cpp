@@ -536,6 +536,22 @@ TORCH_LIBRARY_IMPL(fa_mi355x, CUDA, m) {
   m.impl("decode_paged", &decode_paged_op);
 }
 
+// Decode is inference-only: like a launch on raw pointers, its output and the
+// caches it appends to stay outside autograd, whatever requires grad among
+// the inputs (new rows straight from a projection that is being trained).
+// torch's default for operators without a derivative would mark the output
+// as requiring grad, and its version counters would refuse caches made in
+// inference mode.
+TORCH_LIBRARY_IMPL(fa_mi355x, Autograd, m) {
+  m.impl("decode", torch::CppFunction::makeFallthrough());
+  m.impl("decode_paged", torch::CppFunction::makeFallthrough());
+}
+
+TORCH_LIBRARY_IMPL(fa_mi355x, ADInplaceOrView, m) {
+  m.impl("decode", torch::CppFunction::makeFallthrough());
+  m.impl("decode_paged", torch::CppFunction::makeFallthrough());
+}
+
 TORCH_LIBRARY_IMPL(fa_mi355x, Meta, m) {
   m.impl("forward", &forward_meta);
   m.impl("backward", &backward_meta);

@@ -113,3 +113,21 @@ def test_strided_cache_view_is_updated_in_place():
     np.testing.assert_array_equal(big_k[1].float().cpu().numpy(), rk)
     assert torch.all(big_k[0] == 0) and torch.all(big_k[2] == 0)
     np.testing.assert_allclose(out.float().cpu().numpy(), ref, atol=2e-3, rtol=0)
+
+
+@pytest.mark.parametrize("D", [16, 64])
+def test_append_stays_outside_autograd(D):
+    """New rows that require grad and caches made in inference mode: the
+    output and the caches carry no autograd state, and the result is that of
+    plain tensors.  (D = 16 has padded copies of the caches.)"""
+    q, kc, vc, kn, vn = (t.to(DEVICE) for t in _case(6, 2, 4, 2, 3, 96, 3, D, torch.float16))
+    lens = torch.tensor([5, 90], dtype=torch.int32, device=DEVICE)
+    pk, pv = kc.clone(), vc.clone()
+    want = flash_attention_with_kvcache(q, pk, pv, kn, vn, cache_seqlens=lens, causal=True)
+    with torch.inference_mode():
+        ik, iv = kc.clone(), vc.clone()
+    out = flash_attention_with_kvcache(q, ik, iv, kn.requires_grad_(), vn.requires_grad_(), cache_seqlens=lens,
+                                       causal=True)
+    assert not out.requires_grad and out.grad_fn is None
+    assert not ik.requires_grad and not iv.requires_grad
+    assert torch.equal(out, want) and torch.equal(ik, pk) and torch.equal(iv, pv)
