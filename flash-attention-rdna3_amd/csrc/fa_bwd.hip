@@ -33,18 +33,16 @@ int64_t bwd_share_offset(const fa_bwd_params& p) {
 }
 
 template <typename Tag>
-static hipError_t run_dkdv_merge(const fa_bwd_params& p, int nshare, bool softcap4, hipStream_t s) {
+static hipError_t run_dkdv_merge(const fa_bwd_params& p, int nshare, hipStream_t s) {
   const fa_fwd_params& f = p.fwd;
   const unsigned items = (unsigned)((f.seqlen_k + 63) / 64 * f.batch * f.heads_kv);
   const float* part = reinterpret_cast<const float*>(static_cast<const char*>(p.ds_workspace) + bwd_share_offset(p));
-  if (softcap4) hipLaunchKernelGGL((dkdv_merge_kernel<Tag, 256, true>), dim3(items * 4), dim3(256), 0, s, p, nshare, part);
-  else hipLaunchKernelGGL((dkdv_merge_kernel<Tag, 256, false>), dim3(items * 4), dim3(256), 0, s, p, nshare, part);
+  hipLaunchKernelGGL((dkdv_merge_kernel<Tag, 256>), dim3(items * 4), dim3(256), 0, s, p, nshare, part);
   return hipGetLastError();
 }
 
-hipError_t launch_dkdv_merge(const fa_bwd_params& p, int nshare, bool softcap4, hipStream_t s) {
-  return p.fwd.dtype == FA_DTYPE_F16 ? run_dkdv_merge<f16_t>(p, nshare, softcap4, s)
-                                     : run_dkdv_merge<bf16_t>(p, nshare, softcap4, s);
+hipError_t launch_dkdv_merge(const fa_bwd_params& p, int nshare, hipStream_t s) {
+  return p.fwd.dtype == FA_DTYPE_F16 ? run_dkdv_merge<f16_t>(p, nshare, s) : run_dkdv_merge<bf16_t>(p, nshare, s);
 }
 
 size_t bwd_ds_bytes(const fa_bwd_params& p) {

@@ -674,7 +674,7 @@ static hipError_t run_bwd_dkdv16(const fa_bwd_params& p, hipStream_t stream) {
     hipLaunchKernelGGL(kern, dim3((unsigned)(grid * nshare)), dim3(C::NT), C::LDS_BYTES, stream, p, nnb, nshare, part);
     e = hipGetLastError();
     if (e != hipSuccess || nshare == 1) return e;
-    return launch_dkdv_merge(p, nshare, MODE == 3, stream);
+    return launch_dkdv_merge(p, nshare, stream);
   } else {
   auto kern = dkdv16_kernel<Tag, D, MODE>;
   hipError_t e = allow_lds((const void*)kern, C::LDS_BYTES);
@@ -784,8 +784,9 @@ static hipError_t run_bwd(const fa_bwd_params& p, int phases, hipStream_t stream
       }
       const int nmb = (f.seqlen_q + Dqs16Cfg<D, 1>::BM - 1) / Dqs16Cfg<D, 1>::BM;
       const long grid = (long)nmb * f.batch * f.heads_q;
-      // MODE 3 stores dS / 4 (its softcap factor is (1 - tanh^2) / 4).
-      const float dq_scale = f.softmax_scale * (MODE == 3 ? 4.f : 1.f);
+      // Up to D = 128, MODE 3 stores dS / 4 (its softcap factor is
+      // (1 - tanh^2) / 4).
+      const float dq_scale = f.softmax_scale * (MODE == 3 && D <= 128 ? 4.f : 1.f);
       // A scratch bound above twice the 256 MiB memory-side cache: the dS
       // comes from HBM either way, and nontemporal loads keep it out of L2
       // (config 5, 3.0 GB bound: dQ 303.5 -> 295.2 us).  Below it the plain

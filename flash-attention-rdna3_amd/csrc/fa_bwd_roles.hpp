@@ -245,8 +245,11 @@ __global__ __launch_bounds__(512, 1) void dkdv_roles_kernel(fa_bwd_params p, int
         sched_reads<C::NSTEP, 2, 1, KB>();
         if (!kwave) {
           // P, and what the K wave needs of it: P times the softcap's
-          // derivative (MODE 3: a quarter of it), negative where dropout
-          // dropped the pair.
+          // derivative, negative where dropout dropped the pair.  (All of the
+          // derivative: a dS stored as a quarter, as the narrower kernels do,
+          // falls below fp16's smallest normal number four times sooner.  At
+          // 512 x 512, softcap 50, upstream gradients of 1e-3, dK is off by
+          // 4.4e-4 of its norm that way's 1.4e-3.)
           auto scores = [&](auto cap_t, auto bias_t, auto alibi_t, auto mask_t) {
             constexpr bool CAP = decltype(cap_t)::value;
             constexpr bool MASK = decltype(mask_t)::value;
@@ -279,7 +282,7 @@ __global__ __launch_bounds__(512, 1) void dkdv_roles_kernel(fa_bwd_params p, int
                   }
                   if constexpr (MASK) pv = in_span(rs, acc_row(i, 0)) ? pv : 0.f;
                   wv = pv;
-                  if constexpr (MODE == 3) wv *= tc;
+                  if constexpr (MODE == 3) wv *= 4.f * tc;
                   else if constexpr (CAP) wv *= (1.f - tc * tc);
                   if constexpr (MODE == 2) {
                     if (md.drop_p > 0.f) {
@@ -412,7 +415,7 @@ __global__ __launch_bounds__(512, 1) void dkdv_roles_kernel(fa_bwd_params p, int
   const int64_t ost = kwave ? p.dk_stride[2] : p.dv_stride[2];
   S* orow0 = kwave ? reinterpret_cast<S*>(p.dk) + b * p.dk_stride[0] + hk * p.dk_stride[1]
                    : reinterpret_cast<S*>(p.dv) + b * p.dv_stride[0] + hk * p.dv_stride[1];
-  const float sc = kwave ? f.softmax_scale * (MODE == 3 ? 4.f : 1.f) : 1.f;
+  const float sc = kwave ? f.softmax_scale : 1.f;
   uint16_t* const stage = reinterpret_cast<uint16_t*>(smem_raw + slot * C::PARK_WAVE_BYTES);
 #pragma unroll
   for (int kb = 0; kb < KB; ++kb)
@@ -422,7 +425,7 @@ __global__ __launch_bounds__(512, 1) void dkdv_roles_kernel(fa_bwd_params p, int
 
 // dK / dV of the shares above, added in share order: 64 columns of one item
 // per workgroup, one wave per (pair, role).
-template <typename Tag, int D, bool CAP4>
+template <typename Tag, int D>
 __global__ __launch_bounds__(256) void dkdv_merge_kernel(fa_bwd_params p, int nshare, const float* part) {
   using C = DkdvRolesCfg<D>;
   using S = uint16_t;
@@ -449,7 +452,7 @@ __global__ __launch_bounds__(256) void dkdv_merge_kernel(fa_bwd_params p, int ns
   const int64_t ost = kwave ? p.dk_stride[2] : p.dv_stride[2];
   S* orow0 = kwave ? reinterpret_cast<S*>(p.dk) + b * p.dk_stride[0] + hk * p.dk_stride[1]
                    : reinterpret_cast<S*>(p.dv) + b * p.dv_stride[0] + hk * p.dv_stride[1];
-  const float sc = kwave ? f.softmax_scale * (CAP4 ? 4.f : 1.f) : 1.f;
+  const float sc = kwave ? f.softmax_scale : 1.f;
   store_rows_staged<Tag, MD>(acc, sc, stage + slot * 32 * (MD + 8), orow0 + (int64_t)n0w * ost + cc * MD, ost,
                              min(32, f.seqlen_k - n0w), lane);
 }

@@ -65,8 +65,8 @@ size_t bwd_ds_bytes(const fa_bwd_params& p);
 // (1: none); their fp32 sums follow the dS in the scratch.
 int bwd_share_count(const fa_bwd_params& p);
 int64_t bwd_share_offset(const fa_bwd_params& p);  // bytes from the scratch's start
-// dK and dV from the shares' sums; softcap4: dS was stored as a quarter.
-hipError_t launch_dkdv_merge(const fa_bwd_params& p, int nshare, bool softcap4, hipStream_t stream);
+// dK and dV from the shares' sums.
+hipError_t launch_dkdv_merge(const fa_bwd_params& p, int nshare, hipStream_t stream);
 // dS scratch for `kv_heads` KV heads (with their query heads) of p, or 0
 // when the backward cannot run in KV-head chunks: the per-head modifiers
 // (bias, ALiBi, dropout) are indexed by the head, so only problems without

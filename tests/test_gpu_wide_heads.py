@@ -128,6 +128,41 @@ def test_backward_256(dtype, heads, kv, sq, sk, opts):
             _close(g, w, dtype)
 
 
+@pytest.mark.parametrize("opts", [{}, {"causal": True}, {"window": (150, 40)}])
+@pytest.mark.parametrize("upstream", [1.0, 1e-2, 1e-3, 1e-4])
+def test_softcap_256_keeps_small_gradients(upstream, opts):
+    """fp16 holds dS in full: the products of dQ and dK read dS rounded to
+    fp16 once, and below its smallest normal number (a mean loss without loss
+    scaling is there) the error follows from that rounding.  Modelled in 64
+    bits, with the results' own rounding; 1.15 covers the fp32 sums, delta and
+    the row sums' rounding (a dS stored as a quarter is at 1.06 to 3.6)."""
+    gen = torch.Generator().manual_seed(3)
+    dtype, n, cap = torch.float16, 512, 50.0
+    q, k, v = (_rand((1, 2, n, 256), dtype, gen) for _ in range(3))
+    do = (torch.randn((1, 2, n, 256), generator=gen) * upstream).to(dtype).cuda()
+    opts = dict(opts)
+    window = opts.pop("window", (-1, -1))
+    got = grads(lambda a, b, c: flash_attention(a, b, c, softcap=cap, window_size=window, **opts), q, k, v, do)
+    qd, kd, vd, dod = (t.double() for t in (q, k, v, do))
+    exact = grads(lambda a, b, c: attention(a, b, c, softcap=cap, window=window, **opts), qd, kd, vd, dod)
+    raw = torch.matmul(qd, kd.transpose(-1, -2).contiguous()) / 16
+    t = torch.tanh(raw / cap)
+    keep = torch.ones((n, n), dtype=torch.bool, device="cuda")
+    i, j = torch.arange(n, device="cuda")[:, None], torch.arange(n, device="cuda")[None, :]
+    if opts.get("causal"):
+        keep &= j <= i
+    if window[0] >= 0:
+        keep &= (j >= i - window[0]) & (j <= i + window[1])
+    p = torch.softmax((cap * t).masked_fill(~keep, float("-inf")), -1)
+    dp = torch.matmul(dod, vd.transpose(-1, -2).contiguous())
+    ds = p * (dp - (p * dp).sum(-1, keepdim=True)) * (1 - t * t)
+    r16 = lambda x: x.to(torch.float16).double()
+    model = (r16(torch.matmul(r16(ds), kd) / 16), r16(torch.matmul(r16(ds).transpose(-1, -2).contiguous(), qd) / 16))
+    for g, m, w in zip(got, model, exact):
+        err, floor = float((g.double() - w).norm()), float((m - w).norm())
+        assert err <= 1.15 * floor, (err / float(w.norm()), floor / float(w.norm()))
+
+
 def test_dropout_256_equals_zero_padded_128():
     """The dropout mask depends on positions and seed only, so a head of 128
     padded with zeros to 256 must give the 128-wide kernels' result."""
