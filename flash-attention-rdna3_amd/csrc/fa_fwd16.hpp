@@ -88,9 +88,10 @@ constexpr float kLazyRescale = 8.0f;
 // barrier once this item's LDS use (merge, staged stores) is over.
 // SPLIT: the item covers share `split` of `nsplit` of the block's key tiles
 // and leaves its unnormalised state in `part` for fwd16_merge_kernel.
+// `exact`: fp16 follows the row max exactly (below).
 template <typename Tag, int D, int MODE, int NH, bool SPLIT = false>
 __device__ __forceinline__ void fwd16_item(const fa_fwd_params& p, int num_m_blocks, int item,
-                                           unsigned char* smem_raw, bool end_barrier, int split = 0,
+                                           unsigned char* smem_raw, bool end_barrier, bool exact, int split = 0,
                                            int nsplit = 1, float* part = nullptr) {
   using C = Fwd16Cfg<D, NH>;
   using EL = Elem<Tag>;
@@ -189,14 +190,14 @@ __device__ __forceinline__ void fwd16_item(const fa_fwd_params& p, int num_m_blo
     v_next += (int64_t)(TSTEP * C::BN) * vs;
   };
   const VisBounds vbnd = row_block_bounds(md, m0w, mrows);
-  // fp16 wide heads and the dense fp16 form with one key half follow the max
-  // exactly: the largest weights are then 1 or just below it, where a 16-bit
+  // fp16 wide heads and, where `exact` asks for it, the fp16 form with one key
+  // half follow the max exactly: the largest weights are then 1 or just below it, where a 16-bit
   // float rounds least.  (The split form keeps two maxima per row, which is
   // as good as that; bf16 carries P in two parts.)  Output error against 64
   // bits, lazy and exact: 2.92e-4 and 2.84e-4 of the norm at 2 x 10 x 4096 x 64,
   // 2.93e-4 and 2.78e-4 at 1 x 1 x 4096 x 512.
   const bool exact_max =
-      std::is_same<Tag, f16_t>::value && (D > 128 || (NH == 1 && p.cu_seqlens_q == nullptr));
+      std::is_same<Tag, f16_t>::value && (D > 128 || (NH == 1 && exact));
   const float lazy = exact_max ? 0.f : kLazyRescale;
 
   // The first tiles' DMA and the Q loads share one round trip to memory.
@@ -447,17 +448,18 @@ __device__ __forceinline__ void fwd16_item(const fa_fwd_params& p, int num_m_blo
 // masking the two carry the same number of key tiles together, and both
 // read the same head's K / V, which the workgroup's XCD then holds in L2.
 template <typename Tag, int D, int MODE, int NH, bool PAIR>
-__global__ __launch_bounds__(256 * NH, D > 128 ? 1 : 3 - NH) void fwd16_kernel(fa_fwd_params p, int num_m_blocks) {
+__global__ __launch_bounds__(256 * NH, D > 128 ? 1 : 3 - NH) void fwd16_kernel(fa_fwd_params p, int num_m_blocks,
+                                                                              int exact) {
   extern __shared__ __align__(256) unsigned char smem_raw[];
   if constexpr (!PAIR) {
-    fwd16_item<Tag, D, MODE, NH>(p, num_m_blocks, blockIdx.x, smem_raw, false);
+    fwd16_item<Tag, D, MODE, NH>(p, num_m_blocks, blockIdx.x, smem_raw, false, exact);
   } else {
     const int bh_count = p.batch * p.heads_q;
     const int j = blockIdx.x / bh_count;
     const int bh = blockIdx.x - j * bh_count;
     const int j2 = num_m_blocks - 1 - j;
-    fwd16_item<Tag, D, MODE, NH>(p, num_m_blocks, j * bh_count + bh, smem_raw, j2 != j);
-    if (j2 != j) fwd16_item<Tag, D, MODE, NH>(p, num_m_blocks, j2 * bh_count + bh, smem_raw, false);
+    fwd16_item<Tag, D, MODE, NH>(p, num_m_blocks, j * bh_count + bh, smem_raw, j2 != j, false);
+    if (j2 != j) fwd16_item<Tag, D, MODE, NH>(p, num_m_blocks, j2 * bh_count + bh, smem_raw, false, false);
   }
 }
 
@@ -469,7 +471,7 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void fwd16_split_kernel(fa_fw
                                                                            int nsplit, float* ws) {
   extern __shared__ __align__(256) unsigned char smem_raw[];
   const int item = blockIdx.x / nsplit;
-  fwd16_item<Tag, D, MODE, 1, true>(p, num_m_blocks, item, smem_raw, false, blockIdx.x - item * nsplit, nsplit,
+  fwd16_item<Tag, D, MODE, 1, true>(p, num_m_blocks, item, smem_raw, false, true, blockIdx.x - item * nsplit, nsplit,
                                     ws + (int64_t)blockIdx.x * Fwd16Cfg<D, 1>::PART);
 }
 

@@ -318,12 +318,12 @@ __global__ __launch_bounds__(256) void fwd_kernel(fa_fwd_params p, int num_m_blo
 }
 
 template <typename Tag, int D, int MODE, int NH, bool PAIR = false>
-static hipError_t launch_fwd16(const fa_fwd_params& p, long grid, int nmb, hipStream_t stream) {
+static hipError_t launch_fwd16(const fa_fwd_params& p, long grid, int nmb, hipStream_t stream, bool exact) {
   using C = Fwd16Cfg<D, NH>;
   auto kern = fwd16_kernel<Tag, D, MODE, NH, PAIR>;
   hipError_t e = allow_lds((const void*)kern, C::LDS_BYTES);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(C::NT), C::LDS_BYTES, stream, p, nmb);
+  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(C::NT), C::LDS_BYTES, stream, p, nmb, exact ? 1 : 0);
   return hipGetLastError();
 }
 
@@ -357,7 +357,7 @@ static hipError_t run_fwd(const fa_fwd_params& p, const FwdScratch& scratch, hip
       const int nsplit = fwd_split_count(p);
       if (nsplit > 1 && scratch.ptr && scratch.bytes >= (int64_t)fwd_workspace_bytes(p))
         return launch_fwd16_split<Tag, D, MODE>(p, nmb, nsplit, static_cast<float*>(scratch.ptr), stream);
-      return launch_fwd16<Tag, D, MODE, 1>(p, grid, nmb, stream);
+      return launch_fwd16<Tag, D, MODE, 1>(p, grid, nmb, stream, true);
     }
   }
   if constexpr (!std::is_same<Tag, f32_t>::value && D <= 128) {
@@ -378,15 +378,20 @@ static hipError_t run_fwd(const fa_fwd_params& p, const FwdScratch& scratch, hip
     // it is packed with.  The two forms sum the key tiles in different
     // orders, so they agree to rounding, not bit for bit.)
     const long cus = device_cu_count();
-    if (p.cu_seqlens_q || (p.causal ? grid > 4 * cus : grid > cus))
-      return launch_fwd16<Tag, D, MODE, 1>(p, grid, nmb, stream);
+    if (p.cu_seqlens_q || (p.causal ? grid > 4 * cus : grid > cus)) {
+      // fp16 dense: as close as the key split's output up to the eight rounds
+      // where the key split is the alternative (fwd16_item).  Exact max
+      // against lazy: 5 % (96 x 4096 x 4096 x 64 522 against 497 us).
+      const bool exact = !p.cu_seqlens_q && grid <= 8 * cus;
+      return launch_fwd16<Tag, D, MODE, 1>(p, grid, nmb, stream, exact);
+    }
     // Heavy and light row blocks of a head paired in one workgroup, when the
     // pairs fill whole rounds of the CUs (config 2: 256 pairs): forward
     // 52.5 -> 51.4 us, same results bit for bit.
     const long pairs = (long)((nmb + 1) / 2) * p.batch * p.heads_q;
     if (pairs >= cus && (cus - pairs % cus) % cus * 8 <= pairs)
-      return launch_fwd16<Tag, D, MODE, 2, true>(p, pairs, nmb, stream);
-    return launch_fwd16<Tag, D, MODE, 2>(p, grid, nmb, stream);
+      return launch_fwd16<Tag, D, MODE, 2, true>(p, pairs, nmb, stream, false);
+    return launch_fwd16<Tag, D, MODE, 2>(p, grid, nmb, stream, false);
     }
   }
   // The generic kernel has no softcap-only variant (MODE 3 is MODE 1 there).

@@ -59,3 +59,20 @@ def test_bias_layouts(dtype, bias_dtype, layout, sq, sk, head_dim):
         bias[..., -5] = float("-inf")  # one hidden key
     out = flash_attention(q, k, v, bias=bias)
     _check(out, q, k, v, dtype, bias=bias.expand(2, 3, sq, sk)[:1].double())
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("head_dim", [32, 64])
+@pytest.mark.parametrize("heads,seqlen,window", [
+    (1020, 130, (-1, -1)), (1024, 130, (50, 50)),
+    (1030, 130, (-1, -1)), (1030, 130, (20, -1)),  # more than eight rounds
+])
+def test_equal_and_uneven_blocks(dtype, head_dim, heads, seqlen, window):
+    gen = torch.Generator(device="cuda").manual_seed(heads)
+    q, k, v = (torch.randn((1, heads, seqlen, head_dim), generator=gen, device="cuda").to(dtype) for _ in range(3))
+    out = flash_attention(q, k, v, window_size=window)
+    for h in (0, heads // 2, heads - 1):
+        ref = attention(*(t[:, h:h + 1].double() for t in (q, k, v)), window=window)
+        err = (out[:, h:h + 1].double() - ref).norm() / ref.norm()
+        assert err <= BOUND[dtype], (h, float(err))
+    assert torch.isfinite(out).all()
