@@ -88,8 +88,8 @@ constexpr float kLazyRescale = 8.0f;
 // barrier once this item's LDS use (merge, staged stores) is over.
 // SPLIT: the item covers share `split` of `nsplit` of the block's key tiles
 // and leaves its unnormalised state in `part` for fwd16_merge_kernel.
-// `exact`: fp16 follows the row max exactly (below).
-template <typename Tag, int D, int MODE, int NH, bool SPLIT = false>
+// FOLLOW, `exact`: how closely the row max is followed (below).
+template <typename Tag, int D, int MODE, int NH, bool FOLLOW = false, bool SPLIT = false>
 __device__ __forceinline__ void fwd16_item(const fa_fwd_params& p, int num_m_blocks, int item,
                                            unsigned char* smem_raw, bool end_barrier, bool exact, int split = 0,
                                            int nsplit = 1, float* part = nullptr) {
@@ -190,15 +190,24 @@ __device__ __forceinline__ void fwd16_item(const fa_fwd_params& p, int num_m_blo
     v_next += (int64_t)(TSTEP * C::BN) * vs;
   };
   const VisBounds vbnd = row_block_bounds(md, m0w, mrows);
-  // fp16 wide heads and, where `exact` asks for it, the fp16 form with one key
-  // half follow the max exactly: the largest weights are then 1 or just below it, where a 16-bit
-  // float rounds least.  (The split form keeps two maxima per row, which is
-  // as good as that; bf16 carries P in two parts.)  Output error against 64
-  // bits, lazy and exact: 2.92e-4 and 2.84e-4 of the norm at 2 x 10 x 4096 x 64,
-  // 2.93e-4 and 2.78e-4 at 1 x 1 x 4096 x 512.
-  const bool exact_max =
-      std::is_same<Tag, f16_t>::value && (D > 128 || (NH == 1 && exact));
-  const float lazy = exact_max ? 0.f : kLazyRescale;
+  // How far a row's max may grow before its state is rescaled.  bf16 carries
+  // P in two parts, so how its 16 bits round does not matter there.  fp16
+  // wide heads and, where `exact` asks for it, the narrower dense fp16 forms
+  // follow the max exactly: the largest weights are then 1 or just below it,
+  // where a 16-bit float rounds least.  FOLLOW also takes the max
+  // of each of the first tiles a wave sees for itself, downwards too (a
+  // negative `lazy`: every tile with a visible score rescales): the split
+  // form keeps a max per key half, and few visible keys lose by having one.
+  // Output error against 64 bits at 20 x 2048 rows x 64 of N(0, 1) inputs in
+  // 1e-4, split form / exact max / FOLLOW: 128 keys 2.631 / 2.669 / 2.631,
+  // 256 keys 2.768 / 2.686 / 2.609, 4096 keys 2.920 / 2.837 / 2.825;
+  // 1 x 1 x 4096 x 512, lazy and exact: 2.93 and 2.78.
+  constexpr bool F16 = std::is_same<Tag, f16_t>::value;
+  constexpr int kFollowTiles = 4;
+  constexpr float kFollowDrop = 16.f;  // growth of the state per tile, log2
+  static_assert(!FOLLOW || (F16 && NH == 1), "fp16, one max per row");
+  float lazy = FOLLOW ? kNegInf : F16 && (D > 128 || exact) ? 0.f : kLazyRescale;
+  int followed = 0;
 
   // The first tiles' DMA and the Q loads share one round trip to memory.
   if (my_count > 0) load_tiles(0);
@@ -304,7 +313,13 @@ __device__ __forceinline__ void fwd16_item(const fa_fwd_params& p, int num_m_blo
       tmax = half_max(tmax);
       // Lazy rescale, decided for the whole wave.
       if (__builtin_amdgcn_ballot_w64(tmax > m_i + lazy)) {
-        const float m_new = fmaxf(m_i, tmax);
+        float m_new = fmaxf(m_i, tmax);
+        if constexpr (FOLLOW) {
+          if (lazy < 0.f) {
+            if (m_i - tmax < kFollowDrop) m_new = tmax;  // (no visible score: infinitely lower)
+            if (++followed == kFollowTiles) lazy = 0.f;
+          }
+        }
         const float alpha = (m_new == kNegInf) ? 1.f : __builtin_amdgcn_exp2f(m_i - m_new);
         l_i *= alpha;
 #pragma unroll
@@ -447,12 +462,12 @@ __device__ __forceinline__ void fwd16_item(const fa_fwd_params& p, int num_m_blo
 // block j from the light end, of the same (batch, head): under causal
 // masking the two carry the same number of key tiles together, and both
 // read the same head's K / V, which the workgroup's XCD then holds in L2.
-template <typename Tag, int D, int MODE, int NH, bool PAIR>
+template <typename Tag, int D, int MODE, int NH, bool PAIR, bool FOLLOW>
 __global__ __launch_bounds__(256 * NH, D > 128 ? 1 : 3 - NH) void fwd16_kernel(fa_fwd_params p, int num_m_blocks,
                                                                               int exact) {
   extern __shared__ __align__(256) unsigned char smem_raw[];
   if constexpr (!PAIR) {
-    fwd16_item<Tag, D, MODE, NH>(p, num_m_blocks, blockIdx.x, smem_raw, false, exact);
+    fwd16_item<Tag, D, MODE, NH, FOLLOW>(p, num_m_blocks, blockIdx.x, smem_raw, false, exact);
   } else {
     const int bh_count = p.batch * p.heads_q;
     const int j = blockIdx.x / bh_count;
@@ -471,7 +486,7 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void fwd16_split_kernel(fa_fw
                                                                            int nsplit, float* ws) {
   extern __shared__ __align__(256) unsigned char smem_raw[];
   const int item = blockIdx.x / nsplit;
-  fwd16_item<Tag, D, MODE, 1, true>(p, num_m_blocks, item, smem_raw, false, true, blockIdx.x - item * nsplit, nsplit,
+  fwd16_item<Tag, D, MODE, 1, false, true>(p, num_m_blocks, item, smem_raw, false, true, blockIdx.x - item * nsplit, nsplit,
                                     ws + (int64_t)blockIdx.x * Fwd16Cfg<D, 1>::PART);
 }
 

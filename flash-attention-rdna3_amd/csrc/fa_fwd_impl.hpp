@@ -317,10 +317,10 @@ __global__ __launch_bounds__(256) void fwd_kernel(fa_fwd_params p, int num_m_blo
     lb[(int64_t)m * p.lse_stride[2]] = (m_i == kNegInf) ? kNegInf : (m_i + __log2f(l_safe)) * kLn2;
 }
 
-template <typename Tag, int D, int MODE, int NH, bool PAIR = false>
+template <typename Tag, int D, int MODE, int NH, bool PAIR = false, bool FOLLOW = false>
 static hipError_t launch_fwd16(const fa_fwd_params& p, long grid, int nmb, hipStream_t stream, bool exact) {
   using C = Fwd16Cfg<D, NH>;
-  auto kern = fwd16_kernel<Tag, D, MODE, NH, PAIR>;
+  auto kern = fwd16_kernel<Tag, D, MODE, NH, PAIR, FOLLOW>;
   hipError_t e = allow_lds((const void*)kern, C::LDS_BYTES);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(C::NT), C::LDS_BYTES, stream, p, nmb, exact ? 1 : 0);
@@ -380,9 +380,14 @@ static hipError_t run_fwd(const fa_fwd_params& p, const FwdScratch& scratch, hip
     const long cus = device_cu_count();
     if (p.cu_seqlens_q || (p.causal ? grid > 4 * cus : grid > cus)) {
       // fp16 dense: as close as the key split's output up to the eight rounds
-      // where the key split is the alternative (fwd16_item).  Exact max
-      // against lazy: 5 % (96 x 4096 x 4096 x 64 522 against 497 us).
+      // where the key split is the alternative (fwd16_item); FOLLOW for few
+      // visible keys, or where a bias may hide all but a few (otherwise it
+      // costs up to 3 %).  Exact max against lazy: 5 % (96 x 4096 x 4096 x 64
+      // 522 against 497 us).
       const bool exact = !p.cu_seqlens_q && grid <= 8 * cus;
+      if constexpr (std::is_same<Tag, f16_t>::value)
+        if (exact && (p.bias || visible_keys(p, C::BM) <= 512))
+          return launch_fwd16<Tag, D, MODE, 1, false, true>(p, grid, nmb, stream, exact);
       return launch_fwd16<Tag, D, MODE, 1>(p, grid, nmb, stream, exact);
     }
     // Heavy and light row blocks of a head paired in one workgroup, when the

@@ -85,4 +85,15 @@ hipError_t allow_lds(const void* kernel, int bytes);
 // Compute units of the current device (cached per device).
 int device_cu_count();
 
+// Most keys that `rows` consecutive query rows of a dense problem see.
+inline int64_t visible_keys(const fa_fwd_params& p, int rows) {
+  const int64_t right = p.causal ? 0 : p.window_right;
+  int64_t n = p.seqlen_k;
+  if (p.window_left >= 0) {
+    n = std::min<int64_t>(n, (int64_t)p.seqlen_q + p.window_left);
+    if (right >= 0) n = std::min<int64_t>(n, p.window_left + right + rows);
+  }
+  return n;
+}
+
 }  // namespace fa

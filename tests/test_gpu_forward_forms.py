@@ -61,6 +61,56 @@ def test_bias_layouts(dtype, bias_dtype, layout, sq, sk, head_dim):
     _check(out, q, k, v, dtype, bias=bias.expand(2, 3, sq, sk)[:1].double())
 
 
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("sk,hidden", [(77, 0), (100, 0), (128, 0), (154, 38), (300, 200), (1024, 900)])
+def test_few_visible_keys_round_against_their_own_tiles(head_dim, sk, hidden):
+    """fp16 weights are rounded relative to the max of their own 64 keys, so
+    the largest of each tile are exact.  Modelled in 64 bits with the result's
+    rounding; 1.004 leaves room for ties that fp32 takes the other way (one
+    max for both tiles of 128 keys is at 1.014)."""
+    gen = torch.Generator(device="cuda").manual_seed(sk)
+    q, k, v = (torch.randn((1, 20, n, head_dim), generator=gen, device="cuda").half() for n in (2048, sk, sk))
+    bias = None
+    if hidden:
+        bias = torch.zeros((1, 1, 1, sk), device="cuda", dtype=torch.float16)
+        bias[..., sk - hidden:] = float("-inf")
+    out = flash_attention(q, k, v, bias=bias)
+    n = sk - hidden
+    kd, vd = k[:, :, :n].double(), v[:, :, :n].double()
+    x = torch.matmul(q.double(), kd.transpose(-1, -2).contiguous()) / head_dim ** 0.5
+    weights = torch.exp(x - x.amax(-1, keepdim=True))
+    total = weights.sum(-1, keepdim=True)
+    exact = torch.matmul(weights, vd) / total
+    rounded = []
+    for t in weights.split(64, -1):
+        top = t.amax(-1, keepdim=True)
+        rounded.append((t / top).half().double() * top)
+    model = (torch.matmul(torch.cat(rounded, -1), vd) / total).half().double()
+    err, floor = float((out.double() - exact).norm()), float((model - exact).norm())
+    assert err <= 1.004 * floor, (err / float(exact.norm()), floor / float(exact.norm()))
+
+
+@pytest.mark.parametrize("head_dim", [32, 64, 128])
+@pytest.mark.parametrize("sk", [1, 65, 200, 400])
+@pytest.mark.parametrize("drop", [0.0, 40.0, 4000.0])
+def test_tile_maxima_far_apart(head_dim, sk, drop):
+    """Scores that fall or rise by `drop` from one 64-key tile to the next
+    (the row state is rescaled down and up), rows that see nothing, and rows
+    whose first tiles are hidden."""
+    gen = torch.Generator(device="cuda").manual_seed(sk)
+    heads, sq = 300, 270
+    q, k, v = (torch.randn((1, heads, n, head_dim), generator=gen, device="cuda").half() for n in (sq, sk, sk))
+    step = (torch.arange(sk, device="cuda") // 64).float() * drop
+    bias = torch.stack([-step, step, step.flip(0), -step.flip(0)]).repeat_interleave(68, 0)[:sq].contiguous()
+    bias[5] = float("-inf")
+    bias[100, :sk * 2 // 3] = float("-inf")
+    out = flash_attention(q, k, v, bias=bias[None, None])
+    ref = attention(q[:, :4].double(), k[:, :4].double(), v[:, :4].double(), bias=bias[None, None].double())
+    err = (out[:, :4].double() - ref).norm() / ref.norm()
+    assert torch.isfinite(out).all() and err <= BOUND[torch.float16], float(err)
+    assert (out[:, :, 5] == 0).all()
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("head_dim", [32, 64])
 @pytest.mark.parametrize("heads,seqlen,window", [
