@@ -367,18 +367,25 @@ static hipError_t run_fwd(const fa_fwd_params& p, const FwdScratch& scratch, hip
     const long grid = (long)nmb * p.batch * p.heads_q;
     if (grid <= 0) return hipSuccess;
     // One key half, independent 4-wave workgroups, for packed varlen batches,
-    // for blocks of equal cost (no causal mask) once there are more of them
-    // than CUs, and for causal grids of more than four rounds of one 8-wave
-    // workgroup per CU.  Equal blocks gain nothing from the key split, and
-    // 640 of them in pairs took two rounds of 256 CUs: 2 x 10 x 4096 x 64
-    // fp16 190 -> 140 us, 2 x 10 x 4096 x 154 with a key mask 41 -> 20 us.
-    // Causal 1 x 32/8 x 8000 x 128 bf16: 847 -> 809 us; two rounds (config 2)
-    // keep the key split, 61.0 against 59.2 us.
+    // for blocks of equal cost once there are more of them than CUs, and for
+    // other grids (causal, a window on one side) of more than four rounds of
+    // one 8-wave workgroup per CU (a window at D = 64: two).  Equal blocks gain nothing from the key
+    // split, and 640 of them in pairs took two rounds of 256 CUs:
+    // 2 x 10 x 4096 x 64 fp16 190 -> 140 us, 2 x 10 x 4096 x 154 with a key
+    // mask 41 -> 20 us.  At D = 32 two 8-wave workgroups fit a CU, so equal
+    // blocks keep the key split up to two per CU (300 blocks, 4096 keys:
+    // 59 against 71 us).  Causal 1 x 32/8 x 8000 x 128 bf16: 729 -> 711 us the
+    // call; two rounds (config 2) keep the key split, 61.0 against 59.2 us.
+    // A left window of 300 on 4096 x 4096, key split and one half: 10 heads of
+    // 64 bf16 80 and 94 us, 20 heads 123 and 122, 20 heads of 128 172 and 181.
     // (Varlen always: a sequence's output then does not depend on the batch
     // it is packed with.  The two forms sum the key tiles in different
     // orders, so they agree to rounding, not bit for bit.)
     const long cus = device_cu_count();
-    if (p.cu_seqlens_q || (p.causal ? grid > 4 * cus : grid > cus)) {
+    const bool one_sided = (p.window_left >= 0) != (p.window_right >= 0);
+    const bool uneven = p.causal || (one_sided && !equal_blocks(p));
+    const long split_rounds = p.causal ? 4 : uneven ? (D == 64 ? 2 : 4) : D == 32 ? 2 : 1;
+    if (p.cu_seqlens_q || grid > split_rounds * cus) {
       // fp16 dense: as close as the key split's output up to the eight rounds
       // where the key split is the alternative (fwd16_item); FOLLOW for few
       // visible keys, or where a bias may hide all but a few (otherwise it
@@ -394,9 +401,9 @@ static hipError_t run_fwd(const fa_fwd_params& p, const FwdScratch& scratch, hip
     // pairs fill whole rounds of the CUs (config 2: 256 pairs): forward
     // 52.5 -> 51.4 us, same results bit for bit.
     const long pairs = (long)((nmb + 1) / 2) * p.batch * p.heads_q;
-    if (pairs >= cus && (cus - pairs % cus) % cus * 8 <= pairs)
+    if (p.causal && pairs >= cus && (cus - pairs % cus) % cus * 8 <= pairs)
       return launch_fwd16<Tag, D, MODE, 2, true>(p, pairs, nmb, stream, false);
-    return launch_fwd16<Tag, D, MODE, 2>(p, grid, nmb, stream, false);
+    return launch_fwd16<Tag, D, MODE, 2>(p, grid, nmb, stream, !p.causal && grid > cus);
     }
   }
   // The generic kernel has no softcap-only variant (MODE 3 is MODE 1 there).

@@ -96,4 +96,23 @@ inline int64_t visible_keys(const fa_fwd_params& p, int rows) {
   return n;
 }
 
+// Whether a dense problem's row blocks cost about the same: the keys that
+// five rows, from the first to the last, see average at least two thirds of
+// the most any of them sees (a causal mask: half).
+inline bool equal_blocks(const fa_fwd_params& p) {
+  const int64_t off = (int64_t)p.seqlen_k - p.seqlen_q;
+  int64_t sum = 0, most = 0;
+  for (int i = 0; i < 5; ++i) {
+    const int64_t at = ((int64_t)p.seqlen_q - 1) * i / 4 + off;
+    int64_t lo = 0, hi = p.seqlen_k;
+    if (p.window_left >= 0) lo = std::max<int64_t>(lo, at - p.window_left);
+    if (p.window_right >= 0) hi = std::min<int64_t>(hi, at + p.window_right + 1);
+    if (p.causal) hi = std::min<int64_t>(hi, at + 1);
+    const int64_t seen = std::max<int64_t>(0, hi - lo);
+    sum += seen;
+    most = std::max(most, seen);
+  }
+  return 3 * sum >= 2 * 5 * most;
+}
+
 }  // namespace fa

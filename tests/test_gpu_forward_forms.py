@@ -114,7 +114,8 @@ def test_tile_maxima_far_apart(head_dim, sk, drop):
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("head_dim", [32, 64])
 @pytest.mark.parametrize("heads,seqlen,window", [
-    (1020, 130, (-1, -1)), (1024, 130, (50, 50)),
+    (200, 130, (-1, -1)), (256, 130, (-1, -1)), (257, 130, (-1, -1)),  # 400, 512 and 514 equal blocks
+    (200, 300, (40, -1)), (200, 300, (-1, 40)), (200, 300, (200, -1)), (400, 400, (50, -1)), (400, 400, (50, 50)),
     (1030, 130, (-1, -1)), (1030, 130, (20, -1)),  # more than eight rounds
 ])
 def test_equal_and_uneven_blocks(dtype, head_dim, heads, seqlen, window):
