@@ -188,14 +188,14 @@ __global__ __launch_bounds__(256) void bwd_dkdv_kernel(fa_bwd_params p, int num_
   const int ncols = min(32, sk - n0w);  // <= 0: the wave only helps load
   const int n = n0w + l32;
   const bool nvalid = n < sk;
-  const S* krow = kbase + (int64_t)(nvalid ? n : 0) * f.k_stride[2];
-  const S* vrow = vbase + (int64_t)(nvalid ? n : 0) * f.v_stride[2];
+  const S* krow = kbase + (int64_t)(nvalid ? n : 0) * f.k_stride[2] + khalf_slot<Tag>(h);
+  const S* vrow = vbase + (int64_t)(nvalid ? n : 0) * f.v_stride[2] + khalf_slot<Tag>(h);
   Op kop[C::KVREG ? C::NSTEP : 1], vop[C::KVREG ? C::NSTEP : 1];
   if constexpr (C::KVREG) {
 #pragma unroll
     for (int s = 0; s < C::NSTEP; ++s) {
-      kop[s] = nvalid ? load_op<Tag>(krow + kslot<Tag>(s, h)) : zero_op<Tag>();
-      vop[s] = nvalid ? load_op<Tag>(vrow + kslot<Tag>(s, h)) : zero_op<Tag>();
+      kop[s] = nvalid ? load_op<Tag>(krow + kslot<Tag>(s)) : zero_op<Tag>();
+      vop[s] = nvalid ? load_op<Tag>(vrow + kslot<Tag>(s)) : zero_op<Tag>();
     }
     wait_vm_all();
   }
@@ -285,18 +285,18 @@ __global__ __launch_bounds__(256) void bwd_dkdv_kernel(fa_bwd_params p, int num_
         for (int mb = 0; mb < C::NMB; ++mb) {
           sacc[mb] = zero16();
           pacc[mb] = zero16();
-          const S* qr = Qs + (mb * 32 + l32) * C::QLD;
-          const S* gr = Gs + (mb * 32 + l32) * C::QLD;
+          const S* qr = Qs + (mb * 32 + l32) * C::QLD + khalf_slot<Tag>(h);
+          const S* gr = Gs + (mb * 32 + l32) * C::QLD + khalf_slot<Tag>(h);
 #pragma unroll
           for (int s = 0; s < C::NSTEP; ++s) {
             Op kb_, vb_;
             if constexpr (C::KVREG) { kb_ = kop[s]; vb_ = vop[s]; }
             else {
-              kb_ = nvalid ? load_op<Tag>(krow + kslot<Tag>(s, h)) : zero_op<Tag>();
-              vb_ = nvalid ? load_op<Tag>(vrow + kslot<Tag>(s, h)) : zero_op<Tag>();
+              kb_ = nvalid ? load_op<Tag>(krow + kslot<Tag>(s)) : zero_op<Tag>();
+              vb_ = nvalid ? load_op<Tag>(vrow + kslot<Tag>(s)) : zero_op<Tag>();
             }
-            sacc[mb] = EL::mma(load_op<Tag>(qr + kslot<Tag>(s, h)), kb_, sacc[mb]);
-            pacc[mb] = EL::mma(load_op<Tag>(gr + kslot<Tag>(s, h)), vb_, pacc[mb]);
+            sacc[mb] = EL::mma(load_op<Tag>(qr + kslot<Tag>(s)), kb_, sacc[mb]);
+            pacc[mb] = EL::mma(load_op<Tag>(gr + kslot<Tag>(s)), vb_, pacc[mb]);
           }
         }
         // P_d -> sacc, dS -> pacc.
@@ -501,15 +501,15 @@ __global__ __launch_bounds__(256) void bwd_dq_kernel(fa_bwd_params p, int num_m_
   const int m = m0w + l32;
   const bool mvalid = m < sq;
   const S* qrow = reinterpret_cast<const S*>(f.q) + b * f.q_stride[0] + hq * f.q_stride[1] +
-                  (int64_t)(q_start + (mvalid ? m : 0)) * f.q_stride[2];
+                  (int64_t)(q_start + (mvalid ? m : 0)) * f.q_stride[2] + khalf_slot<Tag>(h);
   const S* grow = reinterpret_cast<const S*>(p.dout) + b * p.dout_stride[0] + hq * p.dout_stride[1] +
-                  (int64_t)(q_start + (mvalid ? m : 0)) * p.dout_stride[2];
+                  (int64_t)(q_start + (mvalid ? m : 0)) * p.dout_stride[2] + khalf_slot<Tag>(h);
   Op qop[C::QREG ? C::NSTEP : 1], gop[C::QREG ? C::NSTEP : 1];
   if constexpr (C::QREG) {
 #pragma unroll
     for (int s = 0; s < C::NSTEP; ++s) {
-      qop[s] = mvalid ? load_op<Tag>(qrow + kslot<Tag>(s, h)) : zero_op<Tag>();
-      gop[s] = mvalid ? load_op<Tag>(grow + kslot<Tag>(s, h)) : zero_op<Tag>();
+      qop[s] = mvalid ? load_op<Tag>(qrow + kslot<Tag>(s)) : zero_op<Tag>();
+      gop[s] = mvalid ? load_op<Tag>(grow + kslot<Tag>(s)) : zero_op<Tag>();
     }
   }
   float lse2 = kNegInf, dlt = 0.f;
@@ -560,18 +560,18 @@ __global__ __launch_bounds__(256) void bwd_dq_kernel(fa_bwd_params p, int num_m_
       for (int kb2 = 0; kb2 < C::NKB; ++kb2) {
         sacc[kb2] = zero16();
         pacc[kb2] = zero16();
-        const S* kr = Ks + (kb2 * 32 + l32) * C::KLD;
-        const S* vr = Vs + (kb2 * 32 + l32) * C::KLD;
+        const S* kr = Ks + (kb2 * 32 + l32) * C::KLD + khalf_slot<Tag>(h);
+        const S* vr = Vs + (kb2 * 32 + l32) * C::KLD + khalf_slot<Tag>(h);
 #pragma unroll
         for (int s = 0; s < C::NSTEP; ++s) {
           Op qb_, gb_;
           if constexpr (C::QREG) { qb_ = qop[s]; gb_ = gop[s]; }
           else {
-            qb_ = mvalid ? load_op<Tag>(qrow + kslot<Tag>(s, h)) : zero_op<Tag>();
-            gb_ = mvalid ? load_op<Tag>(grow + kslot<Tag>(s, h)) : zero_op<Tag>();
+            qb_ = mvalid ? load_op<Tag>(qrow + kslot<Tag>(s)) : zero_op<Tag>();
+            gb_ = mvalid ? load_op<Tag>(grow + kslot<Tag>(s)) : zero_op<Tag>();
           }
-          sacc[kb2] = EL::mma(load_op<Tag>(kr + kslot<Tag>(s, h)), qb_, sacc[kb2]);
-          pacc[kb2] = EL::mma(load_op<Tag>(vr + kslot<Tag>(s, h)), gb_, pacc[kb2]);
+          sacc[kb2] = EL::mma(load_op<Tag>(kr + kslot<Tag>(s)), qb_, sacc[kb2]);
+          pacc[kb2] = EL::mma(load_op<Tag>(vr + kslot<Tag>(s)), gb_, pacc[kb2]);
         }
       }
 #pragma unroll

@@ -129,11 +129,11 @@ __global__ __launch_bounds__(256) void fwd_kernel(fa_fwd_params p, int num_m_blo
   const bool mvalid = m < sq;
 
   Op qop[C::QREG ? C::NSTEP : 1];
-  const S* qrow = qb + (int64_t)(mvalid ? m : 0) * qs;
+  const S* qrow = qb + (int64_t)(mvalid ? m : 0) * qs + khalf_slot<Tag>(h);
   if constexpr (C::QREG) {
 #pragma unroll
     for (int s = 0; s < C::NSTEP; ++s)
-      qop[s] = mvalid ? load_op<Tag>(qrow + kslot<Tag>(s, h)) : zero_op<Tag>();
+      qop[s] = mvalid ? load_op<Tag>(qrow + kslot<Tag>(s)) : zero_op<Tag>();
     wait_vm_all();
   }
 
@@ -177,13 +177,13 @@ __global__ __launch_bounds__(256) void fwd_kernel(fa_fwd_params p, int num_m_blo
 #pragma unroll
       for (int kb2 = 0; kb2 < C::NKB; ++kb2) {
         sacc[kb2] = zero16();
-        const S* krow = Ks + (kb2 * 32 + l32) * C::KLD;
+        const S* krow = Ks + (kb2 * 32 + l32) * C::KLD + khalf_slot<Tag>(h);
 #pragma unroll
         for (int s = 0; s < C::NSTEP; ++s) {
-          Op a = load_op<Tag>(krow + kslot<Tag>(s, h));
+          Op a = load_op<Tag>(krow + kslot<Tag>(s));
           Op bq;
           if constexpr (C::QREG) bq = qop[s];
-          else bq = mvalid ? load_op<Tag>(qrow + kslot<Tag>(s, h)) : zero_op<Tag>();
+          else bq = mvalid ? load_op<Tag>(qrow + kslot<Tag>(s)) : zero_op<Tag>();
           sacc[kb2] = EL::mma(a, bq, sacc[kb2]);
         }
       }

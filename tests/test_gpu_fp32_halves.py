@@ -10,7 +10,7 @@ from fa_rdna3 import flash_attention
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("head_dim", [32, 64, 128])
+@pytest.mark.parametrize("head_dim", [32, 64, 128, 512])
 @pytest.mark.parametrize("heads,kv,sq,sk,opts", [
     (2, 2, 1, 1, {}), (2, 1, 31, 33, {}), (2, 2, 64, 64, {"causal": True}), (4, 2, 65, 63, {"causal": True}),
     (2, 2, 129, 31, {}), (4, 1, 200, 333, {"causal": True}), (2, 2, 300, 300, {"window": (40, 10)}),
