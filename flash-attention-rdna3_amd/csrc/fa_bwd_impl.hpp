@@ -114,13 +114,12 @@ __global__ __launch_bounds__(256) void bwd_delta_kernel(fa_bwd_params p, int hea
 // ---------------------------------------------------------------------------
 // dK / dV
 // ---------------------------------------------------------------------------
-template <typename Tag, int D>
+template <typename Tag, int D, int NH>
 struct DkdvCfg {
   using EL = Elem<Tag>;
   using S = typename EL::S;
   // fp32 up to D = 64: 64 keys and their query steps split between two halves
   // of two waves (see FwdCfg), partial sums added through LDS.
-  static constexpr int NH = (sizeof(S) == 4 && D <= 64) ? 2 : 1;
   static constexpr int NWK = 4 / NH;   // key waves per half
   static constexpr int NW = NWK * NH;
   static constexpr int NT = 64 * NW;
@@ -147,9 +146,9 @@ struct DkdvCfg {
   static constexpr int NDB = DO / 32;
 };
 
-template <typename Tag, int D, int MODE>
+template <typename Tag, int D, int MODE, int NH>
 __global__ __launch_bounds__(256) void bwd_dkdv_kernel(fa_bwd_params p, int num_n_blocks) {
-  using C = DkdvCfg<Tag, D>;
+  using C = DkdvCfg<Tag, D, NH>;
   using EL = Elem<Tag>;
   using S = typename EL::S;
   using Op = typename EL::Op;
@@ -158,8 +157,8 @@ __global__ __launch_bounds__(256) void bwd_dkdv_kernel(fa_bwd_params p, int num_
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave_all = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform (SGPR)
-  const int qhalf = wave_all / C::NWK, wave = wave_all % C::NWK;
-  const int htid = tid % C::NTH;
+  const int qhalf = NH == 1 ? 0 : wave_all / C::NWK, wave = wave_all % C::NWK;
+  const int htid = NH == 1 ? tid : tid % C::NTH;
   const int h = lane >> 5, l32 = lane & 31;
   const int ndc = D / C::DO;
   const int bhk_count = f.batch * f.heads_kv;
@@ -257,7 +256,7 @@ __global__ __launch_bounds__(256) void bwd_dkdv_kernel(fa_bwd_params p, int num_
     };
 
     // Steps [0, nh0) go to half 0, the rest to half 1; both run nh0.
-    const int nh0 = (nsteps + C::NH - 1) / C::NH;
+    const int nh0 = (nsteps + NH - 1) / NH;
     const int my_first = qhalf * nh0;
     const int my_count = qhalf == 0 ? nh0 : nsteps - nh0;
     if (my_count > 0) {
@@ -361,7 +360,7 @@ __global__ __launch_bounds__(256) void bwd_dkdv_kernel(fa_bwd_params p, int num_
   }
 
   // First query half + second query half, in that order.
-  if constexpr (C::NH == 2) {
+  if constexpr (NH == 2) {
     float* ow = reinterpret_cast<float*>(smem_raw) + wave * 2 * C::NDB * 1024;
     __syncthreads();
     if (qhalf == 1) {
@@ -417,13 +416,12 @@ __global__ __launch_bounds__(256) void bwd_dkdv_kernel(fa_bwd_params p, int num_
 // ---------------------------------------------------------------------------
 // dQ
 // ---------------------------------------------------------------------------
-template <typename Tag, int D>
+template <typename Tag, int D, int NH>
 struct DqCfg {
   using EL = Elem<Tag>;
   using S = typename EL::S;
   // fp32 up to D = 64: 64 rows, key tiles split by parity between two halves
   // of two waves (see FwdCfg).
-  static constexpr int NH = (sizeof(S) == 4 && D <= 64) ? 2 : 1;
   static constexpr int NWR = 4 / NH;
   static constexpr int NW = NWR * NH;
   static constexpr int NT = 64 * NW;
@@ -448,9 +446,9 @@ struct DqCfg {
   static constexpr int NDB = DO / 32;
 };
 
-template <typename Tag, int D, int MODE>
+template <typename Tag, int D, int MODE, int NH>
 __global__ __launch_bounds__(256) void bwd_dq_kernel(fa_bwd_params p, int num_m_blocks) {
-  using C = DqCfg<Tag, D>;
+  using C = DqCfg<Tag, D, NH>;
   using EL = Elem<Tag>;
   using S = typename EL::S;
   using Op = typename EL::Op;
@@ -460,8 +458,8 @@ __global__ __launch_bounds__(256) void bwd_dq_kernel(fa_bwd_params p, int num_m_
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave_all = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform (SGPR)
-  const int khalf = wave_all / C::NWR, wave = wave_all % C::NWR;
-  const int htid = tid % C::NTH;
+  const int khalf = NH == 1 ? 0 : wave_all / C::NWR, wave = wave_all % C::NWR;
+  const int htid = NH == 1 ? tid : tid % C::NTH;
   const int h = lane >> 5, l32 = lane & 31;
   const int ndc = D / C::DO;
   const int bh_count = f.batch * f.heads_q;
@@ -539,17 +537,17 @@ __global__ __launch_bounds__(256) void bwd_dq_kernel(fa_bwd_params p, int num_m_
     ktt.store(base + 2 * C::KTILE, C::TLD, htid);
   };
 
-  const int nh0 = (ntiles + C::NH - 1) / C::NH;
-  const int my_count = (ntiles - khalf + C::NH - 1) / C::NH;
+  const int nh0 = (ntiles + NH - 1) / NH;
+  const int my_count = (ntiles - khalf + NH - 1) / NH;
   if (my_count > 0) {
     load_stage(lo + khalf * C::BN);
     store_stage(0);
   }
   __syncthreads();
   for (int t = 0; t < nh0; ++t) {
-    const int n0 = lo + (khalf + C::NH * t) * C::BN;
+    const int n0 = lo + (khalf + NH * t) * C::BN;
     const int st = (C::NSTAGE == 2) ? (t & 1) : 0;
-    if (C::NSTAGE == 2 && t + 1 < my_count) load_stage(n0 + C::NH * C::BN);
+    if (C::NSTAGE == 2 && t + 1 < my_count) load_stage(n0 + NH * C::BN);
     const int vis = mrows > 0 && t < my_count ? rect_visibility(md, m0w, mrows, n0, C::BN) : 0;
     if (vis) {
       const S* Ks = smem + (khalf * C::NSTAGE + st) * C::STAGE;
@@ -611,7 +609,7 @@ __global__ __launch_bounds__(256) void bwd_dq_kernel(fa_bwd_params p, int num_m_
     } else {
       __syncthreads();
       if (t + 1 < my_count) {
-        load_stage(n0 + C::NH * C::BN);
+        load_stage(n0 + NH * C::BN);
         store_stage(0);
       }
       __syncthreads();
@@ -619,7 +617,7 @@ __global__ __launch_bounds__(256) void bwd_dq_kernel(fa_bwd_params p, int num_m_
   }
 
   // First key half + second key half, in that order.
-  if constexpr (C::NH == 2) {
+  if constexpr (NH == 2) {
     float* ow = reinterpret_cast<float*>(smem_raw) + wave * C::NDB * 1024;
     if (khalf == 1) {
 #pragma unroll
@@ -692,6 +690,30 @@ static hipError_t launch_dqs16(const fa_bwd_params& p, long grid, int nmb, float
   hipError_t e = allow_lds((const void*)kern, C::LDS_BYTES);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(C::NT), C::LDS_BYTES, stream, p, nmb, dq_scale, ds_nt);
+  return hipGetLastError();
+}
+
+template <typename Tag, int D, int MODE, int NH>
+static hipError_t launch_dkdv_generic(const fa_bwd_params& p, hipStream_t stream) {
+  using C = DkdvCfg<Tag, D, NH>;
+  auto kern = bwd_dkdv_kernel<Tag, D, MODE, NH>;
+  hipError_t e = allow_lds((const void*)kern, C::LDS_BYTES);
+  if (e != hipSuccess) return e;
+  const int nnb = (p.fwd.seqlen_k + C::BN - 1) / C::BN;
+  const long grid = (long)nnb * p.fwd.batch * p.fwd.heads_kv * (D / C::DO);
+  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(C::NT), C::LDS_BYTES, stream, p, nnb);
+  return hipGetLastError();
+}
+
+template <typename Tag, int D, int MODE, int NH>
+static hipError_t launch_dq_generic(const fa_bwd_params& p, hipStream_t stream) {
+  using C = DqCfg<Tag, D, NH>;
+  auto kern = bwd_dq_kernel<Tag, D, MODE, NH>;
+  hipError_t e = allow_lds((const void*)kern, C::LDS_BYTES);
+  if (e != hipSuccess) return e;
+  const int nmb = (p.fwd.seqlen_q + C::BM - 1) / C::BM;
+  const long grid = (long)nmb * p.fwd.batch * p.fwd.heads_q * (D / C::DO);
+  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(C::NT), C::LDS_BYTES, stream, p, nmb);
   return hipGetLastError();
 }
 
@@ -859,26 +881,22 @@ static hipError_t run_bwd(const fa_bwd_params& p, int phases, hipStream_t stream
   }
   constexpr int GMODE = MODE == 3 ? 1 : MODE;  // no softcap-only generic variant
   if (phases & 2) {
-    using C = DkdvCfg<Tag, D>;
-    auto kern = bwd_dkdv_kernel<Tag, D, GMODE>;
-    hipError_t e = allow_lds((const void*)kern, C::LDS_BYTES);
-    if (e != hipSuccess) return e;
-    const int nnb = (f.seqlen_k + C::BN - 1) / C::BN;
-    const long grid = (long)nnb * f.batch * f.heads_kv * (D / C::DO);
-    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(C::NT), C::LDS_BYTES, stream, p, nnb);
-    e = hipGetLastError();
+    hipError_t e;
+    if constexpr (std::is_same<Tag, f32_t>::value && D <= 64) {
+      const int64_t blocks = ((int64_t)f.seqlen_k + 127) / 128 * f.batch * f.heads_kv;
+      e = f32_halves(f, blocks, true) ? launch_dkdv_generic<Tag, D, GMODE, 2>(p, stream)
+                                : launch_dkdv_generic<Tag, D, GMODE, 1>(p, stream);
+    } else {
+      e = launch_dkdv_generic<Tag, D, GMODE, 1>(p, stream);
+    }
     if (e != hipSuccess) return e;
   }
   if (phases & 4) {
-    using C = DqCfg<Tag, D>;
-    auto kern = bwd_dq_kernel<Tag, D, GMODE>;
-    hipError_t e = allow_lds((const void*)kern, C::LDS_BYTES);
-    if (e != hipSuccess) return e;
-    const int nmb = (f.seqlen_q + C::BM - 1) / C::BM;
-    const long grid = (long)nmb * f.batch * f.heads_q * (D / C::DO);
-    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(C::NT), C::LDS_BYTES, stream, p, nmb);
-    e = hipGetLastError();
-    if (e != hipSuccess) return e;
+    if constexpr (std::is_same<Tag, f32_t>::value && D <= 64) {
+      const int64_t blocks = ((int64_t)f.seqlen_q + 127) / 128 * f.batch * f.heads_q;
+      if (f32_halves(f, blocks, true)) return launch_dq_generic<Tag, D, GMODE, 2>(p, stream);
+    }
+    return launch_dq_generic<Tag, D, GMODE, 1>(p, stream);
   }
   return hipSuccess;
 }

@@ -30,7 +30,7 @@
 namespace fa {
 
 
-template <typename Tag, int D>
+template <typename Tag, int D, int NH>
 struct FwdCfg {
   using EL = Elem<Tag>;
   using S = typename EL::S;
@@ -41,7 +41,6 @@ struct FwdCfg {
   // idle.  At D = 64 the forward takes 61 us there against 100 us, dK/dV 119
   // against 203, dQ 86 against 135 (the operands of four MFMAs in one LDS
   // read, kslot, included); 4.1 / 8.2 / 6.1 GFLOP, card 153 TFLOP/s in fp32.
-  static constexpr int NH = (sizeof(S) == 4 && D <= 128) ? 2 : 1;
   static constexpr int NWR = 4 / NH;          // row waves per half
   static constexpr int NW = NWR * NH;
   static constexpr int NT = 64 * NW;
@@ -66,9 +65,9 @@ struct FwdCfg {
   static constexpr int NDB = DO / 32;           // 32-wide output blocks
 };
 
-template <typename Tag, int D, int MODE>
+template <typename Tag, int D, int MODE, int NH>
 __global__ __launch_bounds__(256) void fwd_kernel(fa_fwd_params p, int num_m_blocks) {
-  using C = FwdCfg<Tag, D>;
+  using C = FwdCfg<Tag, D, NH>;
   using EL = Elem<Tag>;
   using S = typename EL::S;
   using Op = typename EL::Op;
@@ -77,8 +76,8 @@ __global__ __launch_bounds__(256) void fwd_kernel(fa_fwd_params p, int num_m_blo
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave_all = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform (SGPR)
-  const int khalf = wave_all / C::NWR, wave = wave_all % C::NWR;
-  const int htid = tid % C::NTH;
+  const int khalf = NH == 1 ? 0 : wave_all / C::NWR, wave = wave_all % C::NWR;
+  const int htid = NH == 1 ? tid : tid % C::NTH;
   const int h = lane >> 5, l32 = lane & 31;
 
   const int ndc = D / C::DO;
@@ -156,8 +155,8 @@ __global__ __launch_bounds__(256) void fwd_kernel(fa_fwd_params p, int num_m_blo
   };
 
   // Half 0 takes the even key tiles, half 1 the odd ones; both run nh0 steps.
-  const int nh0 = (ntiles + C::NH - 1) / C::NH;
-  const int my_count = (ntiles - khalf + C::NH - 1) / C::NH;
+  const int nh0 = (ntiles + NH - 1) / NH;
+  const int my_count = (ntiles - khalf + NH - 1) / NH;
   if (my_count > 0) {
     load_tiles(lo + khalf * C::BN);
     store_tiles(0);
@@ -165,9 +164,9 @@ __global__ __launch_bounds__(256) void fwd_kernel(fa_fwd_params p, int num_m_blo
   __syncthreads();
 
   for (int t = 0; t < nh0; ++t) {
-    const int n0 = lo + (khalf + C::NH * t) * C::BN;
+    const int n0 = lo + (khalf + NH * t) * C::BN;
     const int stage = t & 1;
-    if (t + 1 < my_count) load_tiles(n0 + C::NH * C::BN);
+    if (t + 1 < my_count) load_tiles(n0 + NH * C::BN);
 
     const int vis = mrows > 0 && t < my_count ? rect_visibility(md, m0w, mrows, n0, C::BN) : 0;
     if (vis) {
@@ -265,7 +264,7 @@ __global__ __launch_bounds__(256) void fwd_kernel(fa_fwd_params p, int num_m_blo
   }
 
   // Half 1 parks (O^T, m, l) in LDS, half 0 folds them in (as fwd16_item).
-  if constexpr (C::NH == 2) {
+  if constexpr (NH == 2) {
     float* ow = reinterpret_cast<float*>(smem_raw);
     float* mw = ow + C::NWR * C::NDB * 1024;
     float* lw = mw + C::NWR * 64;
@@ -340,6 +339,19 @@ static hipError_t launch_fwd16_split(const fa_fwd_params& p, int nmb, int nsplit
   return launch_fwd_merge(p, nmb, nsplit, ws, stream);
 }
 
+template <typename Tag, int D, int MODE, int NH>
+static hipError_t launch_fwd_generic(const fa_fwd_params& p, hipStream_t stream) {
+  using C = FwdCfg<Tag, D, NH>;
+  auto kern = fwd_kernel<Tag, D, MODE, NH>;
+  hipError_t e = allow_lds((const void*)kern, C::LDS_BYTES);
+  if (e != hipSuccess) return e;
+  const int nmb = (p.seqlen_q + C::BM - 1) / C::BM;
+  const long grid = (long)nmb * p.batch * p.heads_q * (D / C::DO);
+  if (grid <= 0) return hipSuccess;
+  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(C::NT), C::LDS_BYTES, stream, p, nmb);
+  return hipGetLastError();
+}
+
 template <typename Tag, int D, int MODE>
 static hipError_t run_fwd(const fa_fwd_params& p, const FwdScratch& scratch, hipStream_t stream) {
   if constexpr (!std::is_same<Tag, f32_t>::value && D > 128) {
@@ -408,15 +420,11 @@ static hipError_t run_fwd(const fa_fwd_params& p, const FwdScratch& scratch, hip
   }
   // The generic kernel has no softcap-only variant (MODE 3 is MODE 1 there).
   constexpr int GMODE = MODE == 3 ? 1 : MODE;
-  using C = FwdCfg<Tag, D>;
-  auto kern = fwd_kernel<Tag, D, GMODE>;
-  hipError_t e = allow_lds((const void*)kern, C::LDS_BYTES);
-  if (e != hipSuccess) return e;
-  const int nmb = (p.seqlen_q + C::BM - 1) / C::BM;
-  const long grid = (long)nmb * p.batch * p.heads_q * (D / C::DO);
-  if (grid <= 0) return hipSuccess;
-  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(C::NT), C::LDS_BYTES, stream, p, nmb);
-  return hipGetLastError();
+  if constexpr (std::is_same<Tag, f32_t>::value && D <= 128) {
+    const int64_t blocks = ((int64_t)p.seqlen_q + 127) / 128 * p.batch * p.heads_q;
+    if (f32_halves(p, blocks, false)) return launch_fwd_generic<Tag, D, GMODE, 2>(p, stream);
+  }
+  return launch_fwd_generic<Tag, D, GMODE, 1>(p, stream);
 }
 
 template <typename Tag, int MODE>

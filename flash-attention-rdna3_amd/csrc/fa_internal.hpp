@@ -115,4 +115,29 @@ inline bool equal_blocks(const fa_fwd_params& p) {
   return 3 * sum >= 2 * 5 * most;
 }
 
+// fp32 up to D = 128 (backward: 64): whether workgroups of 64 rows (or keys)
+// whose other range is split between two halves (NH = 2) beat ones of 128
+// rows, given the number of 128-row blocks.  A round of the former takes 0.56
+// (backward) to 0.66 of a round of the latter, so equal blocks take them when
+// the rounds come out shorter: mostly when a last round of whole blocks would
+// leave half of the CUs idle (16 x 1000 x 64, 128 blocks: forward 59 against
+// 95 us, step 255 against 435; 192 blocks 112 against 96, 512 blocks 224
+// against 165).  At D = 32 more workgroups fit a CU: 384 blocks 83 against
+// 96 us, 512 106 against 97.  Causal blocks even out better when they are
+// small: D = 64, 384 blocks 106 against 118 us, 512 137 against 125 (rows of
+// 1000; of 4096: 435 against 466); D = 128, 256 blocks 120 against 162 us,
+// 384 190 against 165; D = 32, 768 blocks 94 against 96.
+inline bool f32_halves(const fa_fwd_params& p, int64_t blocks, bool backward) {
+  const int64_t cus = device_cu_count();
+  const int d = p.head_dim;
+  if (!equal_blocks(p)) {
+    if (d == 32) return blocks <= 3 * cus;
+    if (d == 64) return blocks * 2 <= (p.seqlen_q >= 2048 ? 4 : 3) * cus;
+    return blocks <= cus;
+  }
+  if (d == 32) return blocks * 2 <= 3 * cus;
+  const int half_cost = backward ? 27 : d == 64 ? 32 : 30;  // of a whole round's 48
+  return (2 * blocks + cus - 1) / cus * half_cost < (blocks + cus - 1) / cus * 48;
+}
+
 }  // namespace fa

@@ -1,5 +1,6 @@
-"""fp32 forward and backward, whose key or query range is split between two
-halves of a workgroup, against 64-bit attention at tile edges."""
+"""fp32 forward and backward, with the key or query range split between two
+halves of a workgroup and, on grids that fill the chip, without, against
+64-bit attention at tile edges."""
 
 import pytest
 import torch
@@ -15,6 +16,11 @@ pytestmark = pytest.mark.gpu
     (2, 2, 1, 1, {}), (2, 1, 31, 33, {}), (2, 2, 64, 64, {"causal": True}), (4, 2, 65, 63, {"causal": True}),
     (2, 2, 129, 31, {}), (4, 1, 200, 333, {"causal": True}), (2, 2, 300, 300, {"window": (40, 10)}),
     (2, 2, 150, 150, {"softcap": 8.0, "causal": True}),
+    # 200 to 900 blocks of 128 rows, odd lengths: whole workgroups where they
+    # are the faster form (see f32_halves), halves otherwise
+    (100, 50, 131, 70, {}), (150, 150, 140, 129, {}), (260, 130, 65, 131, {}), (300, 300, 129, 31, {"softcap": 8.0}),
+    (300, 100, 150, 150, {"causal": True}), (300, 300, 257, 257, {"causal": True}),
+    (260, 260, 200, 200, {"window": (30, -1)}), (260, 260, 200, 200, {"causal": True, "window": (30, -1)}),
 ])
 def test_matches_64_bit(head_dim, heads, kv, sq, sk, opts):
     gen = torch.Generator(device="cuda").manual_seed(sq + sk)
