@@ -277,7 +277,9 @@ __global__ __launch_bounds__(512, 1) void dkdv_roles_kernel(fa_bwd_params p, int
                     tc = __builtin_fmaf(-rr, rr, rr);
                   } else {
                     const int m = m0 + acc_row(i, h), n = n0w + 32 * kb + l32;
-                    const float sc = score_m<CAP, decltype(bias_t)::value, decltype(alibi_t)::value>(md, x[kb][i], m, n, tc);
+                    float sc;
+                    if constexpr (MODE == 2) sc = score<true>(md, x[kb][i], m, n, tc);
+                    else sc = score_m<CAP, decltype(bias_t)::value, decltype(alibi_t)::value>(md, x[kb][i], m, n, tc);
                     pv = __builtin_amdgcn_exp2f(sc - l2[r]);
                   }
                   if constexpr (MASK) pv = in_span(rs, acc_row(i, 0)) ? pv : 0.f;
@@ -304,6 +306,12 @@ __global__ __launch_bounds__(512, 1) void dkdv_roles_kernel(fa_bwd_params p, int
           if constexpr (MODE == 0 || MODE == 3) {
             if (vis == 1) scores(F_{}, B0{}, F_{}, T_{});
             else scores(F_{}, B0{}, F_{}, F_{});
+          } else if constexpr (MODE == 2) {
+            // One variant that tests for each modifier (CAP: tc is 0 without
+            // a softcap) and masks: sixteen of them left 1195 reads of spilled
+            // registers and a call in the step loop (1 x 16/8 x 2048 x 256
+            // bf16, dropout: dK/dV 2673 -> 448 us).
+            scores(T_{}, B0{}, F_{}, T_{});
           } else {
             if (vis == 1) dispatch_mods(md, [&](auto a, auto b_, auto c_) { scores(a, b_, c_, T_{}); });
             else dispatch_mods(md, [&](auto a, auto b_, auto c_) { scores(a, b_, c_, F_{}); });

@@ -51,3 +51,10 @@ def test_kernels_do_not_spill(spills, kernel):
     found = {n: c for n, c in spills.items() if re.search(kernel, n)}
     assert found, sorted(spills)[:5]
     assert not any(c for c, _ in found.values()), {n: c for n, c in found.items() if c[0]}
+
+
+def test_dropout_at_256_keeps_its_step_loop_in_registers(spills):
+    """The sixteen score variants of this kernel took 576 bytes of scratch a
+    lane, most of it read back in the step loop; one variant takes 168."""
+    found = {n: c for n, c in spills.items() if "dkdv_roles_kernel<" in n and ", 256, 2>" in n}
+    assert len(found) == 2 and all(s <= 256 for _, s in found.values()), found
