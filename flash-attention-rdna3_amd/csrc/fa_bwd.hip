@@ -9,9 +9,9 @@ hipError_t bwd_by_mods(const fa_bwd_params& p, int ph, hipStream_t s);
 
 // Shares of the D = 256 dK/dV pass: a grid that would leave half the CUs
 // idle is split until it fills them (at least eight query steps of 32 rows
-// each), and a causal grid of one round at most in two, since it lasts as long
-// as its heaviest block, twice the mean (1 x 16/8 x 2048 x 256 bf16: dK/dV
-// 150 -> 108 us and 14 for the merge).  At 1 x 4 x 500 x 256, two shares of
+// each in the block that sees the most), and a causal grid of one round at
+// most in two, since it lasts as long as its heaviest block, twice the mean
+// (1 x 16/8 x 2048 x 256 bf16: dK/dV 150 -> 108 us and 14 for the merge).  At 1 x 4 x 500 x 256, two shares of
 // eight steps, it is 26.7 -> 21.2 + 4.3 us.
 int bwd_share_count(const fa_bwd_params& p) {
   const fa_fwd_params& f = p.fwd;
@@ -20,10 +20,10 @@ int bwd_share_count(const fa_bwd_params& p) {
   // (problems that may run in chunks of KV heads have none, whole or chunked)
   if (bwd_share_offset(p) >= kDsMinChunkBytes) return 1;
   const int64_t groups = ((int64_t)f.seqlen_k + 63) / 64 * f.batch * f.heads_kv;
-  const int64_t steps = ((int64_t)f.seqlen_q + 31) / 32;
+  const int64_t steps = (visible_queries(f, 64) + 31) / 32;
   const int64_t cus = device_cu_count();
   if (groups > cus) return 1;
-  if (groups * 2 > cus) return f.causal && steps >= 32 ? 2 : 1;
+  if (groups * 2 > cus) return f.causal && (f.window_left < 0 || !equal_blocks(f)) && steps >= 32 ? 2 : 1;
   return (int)std::max<int64_t>(1, std::min({cus / groups, steps / 8, (int64_t)8}));
 }
 

@@ -96,6 +96,17 @@ inline int64_t visible_keys(const fa_fwd_params& p, int rows) {
   return n;
 }
 
+// Most query rows that see a key among `keys` consecutive ones.
+inline int64_t visible_queries(const fa_fwd_params& p, int keys) {
+  const int64_t right = p.causal ? 0 : p.window_right;
+  int64_t n = p.seqlen_q;
+  if (right >= 0) {
+    n = std::min<int64_t>(n, p.seqlen_k + right);
+    if (p.window_left >= 0) n = std::min<int64_t>(n, p.window_left + right + keys);
+  }
+  return n;
+}
+
 // Whether a dense problem's row blocks cost about the same: the keys that
 // five rows, from the first to the last, see average at least two thirds of
 // the most any of them sees (a causal mask: half).

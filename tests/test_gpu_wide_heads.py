@@ -88,6 +88,7 @@ def test_key_splits_agree_with_one_workgroup(head_dim, hidden):
 def test_no_splits_without_room_to_gain():
     p = _native.FwdParams()
     p.dtype, p.head_dim, p.batch, p.heads_q, p.heads_kv, p.seqlen_q, p.seqlen_k = 0, 256, 1, 16, 16, 2048, 2048
+    p.window_left = p.window_right = -1  # none (0 would be a window of one key)
     need = _native.lib().fa_fwd_workspace_bytes
     assert need(ctypes.byref(p)) == 0  # 256 row blocks fill the CUs
     p.heads_q = p.heads_kv = 1

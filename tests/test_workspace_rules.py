@@ -13,11 +13,12 @@ if torch.cuda.is_available() and torch.cuda.get_device_properties(0).multi_proce
     pytest.skip("sizes below are for 256 compute units", allow_module_level=True)
 
 
-def _params(head_dim, heads, kv, sq, sk, causal=0, batch=1, dtype=0):
+def _params(head_dim, heads, kv, sq, sk, causal=0, batch=1, dtype=0, window=(-1, -1)):
     p = _native.BwdParams()
     f = p.fwd
     f.abi_version, f.dtype, f.head_dim, f.batch = _native.ABI_VERSION, dtype, head_dim, batch
     f.heads_q, f.heads_kv, f.seqlen_q, f.seqlen_k, f.causal = heads, kv, sq, sk, causal
+    f.window_left, f.window_right = window  # (-1: none; 0 would be a window of one key)
     return p
 
 
@@ -54,3 +55,31 @@ def test_backward_256_shares(heads, kv, sq, sk, causal, shares):
     assert _native.lib().fa_bwd_workspace_bytes(ctypes.byref(p)) == ds + part
     p.fwd.head_dim = 512
     assert _native.lib().fa_bwd_workspace_bytes(ctypes.byref(p)) == 0
+
+
+@pytest.mark.parametrize("sq,sk,causal,window,shares", [
+    (4096, 4096, 0, (64, 0), 1),       # 193 keys at most: under two shares of four 32-key tiles
+    (4096, 4096, 0, (200, 100), 3),    # 429 keys, 14 tiles
+    (4096, 4096, 1, (400, 50), 4),     # causal: 528 keys, 17 tiles
+    (4096, 4096, 0, (-1, 64), 8), (4096, 4096, 0, (64, -1), 8),  # one side: some block sees all keys
+    (100, 8000, 0, (64, -1), 1),       # the last 164 keys
+    (100, 8000, 0, (10000, 10000), 16),
+])
+def test_forward_shares_count_visible_keys(sq, sk, causal, window, shares):
+    p = _params(256, 1, 1, sq, sk, causal, window=window)
+    want = 0 if shares == 1 else -(-sq // 128) * shares * 4 * (128 * 256 + 256)
+    assert _native.lib().fa_fwd_workspace_bytes(ctypes.byref(p.fwd)) == want
+
+
+@pytest.mark.parametrize("heads,sq,sk,causal,window,shares", [
+    (1, 4096, 256, 0, (64, 0), 1),     # 128 queries at most see a block of 64 keys
+    (1, 4096, 256, 0, (300, 300), 2),  # 664 of the 4096, but 556 queries reach the 256 keys: 17 steps
+    (1, 4096, 4096, 1, (1000, -1), 4),
+    (1, 4096, 256, 1, (-1, -1), 1),    # only the last 256 queries see a key
+    (8, 2048, 2048, 1, (-1, -1), 2), (8, 2048, 2048, 1, (300, -1), 1), (8, 2048, 2048, 1, (4000, -1), 2),
+])
+def test_backward_256_shares_count_visible_queries(heads, sq, sk, causal, window, shares):
+    p = _params(256, heads, heads, sq, sk, causal, window=window)
+    ds = heads * -(-sk // 64) * -(-sq // 128) * 16384 + 1024
+    part = -(-sk // 64) * heads * shares * 2 * 64 * 256 * 4 if shares > 1 else 0
+    assert _native.lib().fa_bwd_workspace_bytes(ctypes.byref(p)) == ds + part
