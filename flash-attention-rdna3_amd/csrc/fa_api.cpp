@@ -174,7 +174,8 @@ size_t fa_bwd_workspace_min_bytes(const fa_bwd_params* params) {
   const size_t full = fa::bwd_ds_bytes(*params);
   const int per = (params->fwd.heads_kv + 1) / 2;
   const size_t half = params->fwd.heads_kv > 1 ? fa::bwd_ds_chunk_bytes(*params, per) : 0;
-  return (half > 0 && fa::bwd_ds_chunk_heads(*params, (int64_t)half) == per) ? half : full;
+  if (half > 0 && fa::bwd_ds_chunk_heads(*params, (int64_t)half) == per) return half;
+  return fa::bwd_ds_only_bytes(*params);
 }
 
 // With dS scratch, phase 2 alone reads the dS that phase 1 stored there.
@@ -209,7 +210,7 @@ DsRecord ds_record_of(const fa_bwd_params& p) {
 
 bool ds_scratch_used(const fa_bwd_params& p) {
   if (!p.ds_workspace) return false;
-  const size_t need = fa::bwd_ds_bytes(p);
+  const size_t need = fa::bwd_ds_only_bytes(p);
   return need > 0 && p.ds_workspace_bytes >= (int64_t)need;
 }
 }  // namespace

@@ -45,7 +45,7 @@ hipError_t launch_dkdv_merge(const fa_bwd_params& p, int nshare, hipStream_t s) 
   return p.fwd.dtype == FA_DTYPE_F16 ? run_dkdv_merge<f16_t>(p, nshare, s) : run_dkdv_merge<bf16_t>(p, nshare, s);
 }
 
-size_t bwd_ds_bytes(const fa_bwd_params& p) {
+size_t bwd_ds_only_bytes(const fa_bwd_params& p) {
   const fa_fwd_params& f = p.fwd;
   if (f.dtype == FA_DTYPE_F32 || f.head_dim > 256 || f.head_dim < 64) return 0;
   if (f.head_dim > 128 && f.cu_seqlens_q) return 0;
@@ -60,7 +60,13 @@ size_t bwd_ds_bytes(const fa_bwd_params& p) {
   } else {
     elems = (int64_t)f.batch * f.heads_q * ds_region_elems(f.seqlen_q, f.seqlen_k);
   }
-  size_t bytes = (size_t)elems * 2 + 1024;
+  return (size_t)elems * 2 + 1024;
+}
+
+size_t bwd_ds_bytes(const fa_bwd_params& p) {
+  const fa_fwd_params& f = p.fwd;
+  size_t bytes = bwd_ds_only_bytes(p);
+  if (bytes == 0) return 0;
   if (const int n = bwd_share_count(p); n > 1)  // 64 keys of dK and dV in fp32 per share
     bytes += ((size_t)f.seqlen_k + 63) / 64 * f.batch * f.heads_kv * n * (2 * 64 * 256 * 4);
   return bytes;

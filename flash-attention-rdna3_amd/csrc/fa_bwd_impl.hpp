@@ -664,8 +664,8 @@ static hipError_t run_bwd_dkdv16(const fa_bwd_params& p, hipStream_t stream) {
     auto kern = dkdv_roles_kernel<Tag, D, MODE>;
     hipError_t e = allow_lds((const void*)kern, C::LDS_BYTES);
     if (e != hipSuccess) return e;
-    // (ds_workspace is set only when it holds bwd_ds_bytes)
-    const int nshare = p.ds_workspace ? bwd_share_count(p) : 1;
+    // (ds_workspace is set only when it holds the dS)
+    const int nshare = p.ds_workspace && p.ds_workspace_bytes >= (int64_t)bwd_ds_bytes(p) ? bwd_share_count(p) : 1;
     float* part = nshare > 1
                       ? reinterpret_cast<float*>(static_cast<char*>(p.ds_workspace) + bwd_share_offset(p))
                       : nullptr;
@@ -733,7 +733,7 @@ static hipError_t run_bwd(const fa_bwd_params& p, int phases, hipStream_t stream
   // delta has its own kernel.
   bool use_ds = false;
   if constexpr (FAST && D >= 64) {
-    const size_t need = bwd_ds_bytes(p);
+    const size_t need = bwd_ds_only_bytes(p);
     use_ds = fast_ok && p.ds_workspace != nullptr && need > 0 && p.ds_workspace_bytes >= (int64_t)need;
   }
   // Scratch too small for every head at once: dK/dV and dQ run in two

@@ -60,6 +60,7 @@ __host__ __device__ inline int64_t ds_qblocks(int sq) { return ((int64_t)sq + kD
 __host__ __device__ inline int64_t ds_region_elems(int sq, int sk) {
   return ((int64_t)sk + kDsTileKeys - 1) / kDsTileKeys * ds_qblocks(sq) * kDsTileElems;
 }
+size_t bwd_ds_only_bytes(const fa_bwd_params& p);  // without the shares below
 size_t bwd_ds_bytes(const fa_bwd_params& p);
 // D = 256 with dS scratch: workgroups that share a key block's query steps
 // (1: none); their fp32 sums follow the dS in the scratch.

@@ -293,3 +293,35 @@ def test_chunked_ds_path_odd_kv_heads():
     chunked = _grads_at_limit(fn, (q, k, v, do), half)
     for a, b in zip(whole, chunked):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("case", range(len(CASES)))
+def test_dense_256_with_and_without_scratch(case):
+    """CASES at head dim 256: the dS path (dK/dV unshared and shared) against
+    the recomputed dQ.  delta comes from its own kernel either way."""
+    opts = dict(CASES[case])
+    torch.manual_seed(case)
+    dtype, hq, hk, sq, sk = torch.float16, 4, 2, 700, 421
+    q, do = _rand((1, hq, sq, 256), dtype), _rand((1, hq, sq, 256), dtype)
+    k, v = _rand((1, hk, sk, 256), dtype), _rand((1, hk, sk, 256), dtype)
+    if opts.pop("alibi", False):
+        opts["alibi_slopes"] = alibi_slopes(hq, device=DEVICE)
+    if opts.pop("bias", False):
+        opts["bias"] = _rand((1, hq, sq, sk), dtype)
+    state = torch.get_rng_state()
+
+    def fn(a, b, c):
+        torch.set_rng_state(state)  # the same dropout seed every time
+        return flash_attention(a, b, c, **opts)
+
+    only_ds = hq * -(-sk // 64) * -(-sq // 128) * 16384 + 1024
+    full = _grads_at_limit(fn, (q, k, v, do), 1 << 30)
+    unshared = _grads_at_limit(fn, (q, k, v, do), only_ds)
+    recompute = _grads_at_limit(fn, (q, k, v, do), 0)
+    assert torch.equal(full[0], unshared[0])  # dQ is dS K of the same dS
+    ulp = 2.0 ** -10
+    for other in (unshared, recompute):
+        for a, b in zip(full, other):
+            assert torch.isfinite(a).all()
+            assert (a.float() - b.float()).abs().max() <= 4 * ulp * b.float().abs().max()
+    assert torch.equal(unshared[1], recompute[1]) and torch.equal(unshared[2], recompute[2])

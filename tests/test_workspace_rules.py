@@ -83,3 +83,4 @@ def test_backward_256_shares_count_visible_queries(heads, sq, sk, causal, window
     ds = heads * -(-sk // 64) * -(-sq // 128) * 16384 + 1024
     part = -(-sk // 64) * heads * shares * 2 * 64 * 256 * 4 if shares > 1 else 0
     assert _native.lib().fa_bwd_workspace_bytes(ctypes.byref(p)) == ds + part
+    assert _native.lib().fa_bwd_workspace_min_bytes(ctypes.byref(p)) == ds  # the dS path without shares
