@@ -17,7 +17,8 @@ int bwd_share_count(const fa_bwd_params& p) {
   const fa_fwd_params& f = p.fwd;
   if (f.dtype == FA_DTYPE_F32 || f.head_dim != 256 || f.cu_seqlens_q) return 1;
   if (f.batch <= 0 || f.heads_q <= 0 || f.heads_kv <= 0 || f.seqlen_q <= 0 || f.seqlen_k <= 0) return 1;
-  // (problems that may run in chunks of KV heads have none, whole or chunked)
+  // (problems that may run in chunks of KV heads have none; the chunks' own
+  // launches get scratch for their dS only)
   if (bwd_share_offset(p) >= kDsMinChunkBytes) return 1;
   const int64_t groups = ((int64_t)f.seqlen_k + 63) / 64 * f.batch * f.heads_kv;
   const int64_t steps = (visible_queries(f, 64) + 31) / 32;

@@ -776,6 +776,8 @@ static hipError_t run_bwd(const fa_bwd_params& p, int phases, hipStream_t stream
           c.dv = const_cast<void*>(shift(p.dv, kv0 * p.dv_stride[1]));
           c.fwd.heads_kv = n;
           c.fwd.heads_q = n * group;
+          // (room for no shares: the chunks add up as the whole problem does)
+          if constexpr (D > 128) c.ds_workspace_bytes = (int64_t)bwd_ds_only_bytes(c);
           hipError_t e = run_bwd<Tag, D, MODE>(c, 6, stream);
           if (e != hipSuccess) return e;
         }

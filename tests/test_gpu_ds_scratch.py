@@ -295,6 +295,27 @@ def test_chunked_ds_path_odd_kv_heads():
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("opts", [dict(causal=True), dict(causal=True, softcap=30.0), dict(window_size=(4000, 3000))])
+def test_chunked_256_odd_kv_heads(opts):
+    """Head dim 256, three KV heads in chunks of 2 and 1: the second chunk is
+    small enough to share out its query steps by itself, but must add up as
+    the whole problem does."""
+    torch.manual_seed(9)
+    dtype = torch.float16
+    q, do = _rand((1, 3, 16384, 256), dtype), _rand((1, 3, 16384, 256), dtype)
+    k, v = _rand((1, 3, 16384, 256), dtype), _rand((1, 3, 16384, 256), dtype)
+
+    def fn(a, b, c):
+        return flash_attention(a, b, c, **opts)
+
+    half, full = _min_and_full(q, k, None)
+    assert (half - 1024) * 3 == (full - 1024) * 2
+    whole = _grads_at_limit(fn, (q, k, v, do), full)
+    chunked = _grads_at_limit(fn, (q, k, v, do), half)
+    for a, b in zip(whole, chunked):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("case", range(len(CASES)))
 def test_dense_256_with_and_without_scratch(case):
     """CASES at head dim 256: the dS path (dK/dV unshared and shared) against
