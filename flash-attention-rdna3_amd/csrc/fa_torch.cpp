@@ -64,6 +64,17 @@ int64_t ds_scratch_bytes(const fa_bwd_params& p, int64_t limit) {
   return (half > 0 && half < full && half <= limit) ? half : 0;
 }
 
+// Device scratch that a call is faster with but can do without: an undefined
+// tensor when the device has no room for it.
+Tensor optional_scratch(int64_t bytes, const Tensor& like) {
+  if (bytes <= 0) return Tensor();
+  try {
+    return at::empty({bytes}, like.options().dtype(at::kByte));
+  } catch (const c10::OutOfMemoryError&) {
+    return Tensor();
+  }
+}
+
 struct Options {
   bool causal;
   double scale;
@@ -195,16 +206,18 @@ std::tuple<Tensor, Tensor> forward_impl(const Tensor& query, const Tensor& key, 
   Tensor lse = at::empty({q.size(0), q.size(1), q.size(2)}, query.options().dtype(at::kFloat));
   fa_fwd_params p;
   const Extras ex = fill_fwd(p, q, k, v, out, lse, o);
-  Tensor ws;
   const size_t bytes = fa_fwd_workspace_bytes(&p);
-  if (bytes > 0) ws = at::empty({(int64_t)bytes}, query.options().dtype(at::kByte));
-  check_status(fa_fwd_ws(&p, bytes > 0 ? ws.data_ptr() : nullptr, bytes, stream_of(query)), "fa_fwd");
+  const Tensor ws = optional_scratch((int64_t)bytes, query);
+  check_status(fa_fwd_ws(&p, ws.defined() ? ws.data_ptr() : nullptr, ws.defined() ? bytes : 0, stream_of(query)),
+               "fa_fwd");
   if (kdim != head_dim) out = out.narrow(-1, 0, head_dim).contiguous();
   return {out, lse};
 }
 
 // reference interface.py:202-277 (_backward): delta, dK/dV and dQ in one
-// fa_bwd call, with the dS scratch when it fits under the limit.
+// fa_bwd call, with the dS scratch when it fits under the limit and on the
+// device: a step that fits without it must not fail for it (at head dim 256
+// the scratch is batch * heads * Sq * Sk * 2 bytes, up to the limit).
 std::tuple<Tensor, Tensor, Tensor> backward_impl(const Tensor& dout, const Tensor& query, const Tensor& key,
                                                  const Tensor& value, const Tensor& out, const Tensor& lse_in,
                                                  const Options& o) {
@@ -235,10 +248,13 @@ std::tuple<Tensor, Tensor, Tensor> backward_impl(const Tensor& dout, const Tenso
   abi_strides4(p.dk_stride, dk);
   abi_strides4(p.dv_stride, dv);
   abi_strides3(p.delta_stride, delta);
-  Tensor ds;
-  const int64_t bytes = ds_scratch_bytes(p, g_ds_limit.load(std::memory_order_relaxed));
-  if (bytes > 0) {
-    ds = at::empty({bytes}, query.options().dtype(at::kByte));
+  int64_t bytes = ds_scratch_bytes(p, g_ds_limit.load(std::memory_order_relaxed));
+  Tensor ds = optional_scratch(bytes, query);
+  if (bytes > 0 && !ds.defined()) {
+    bytes = ds_scratch_bytes(p, bytes - 1);  // the smaller form, if there is one
+    ds = optional_scratch(bytes, query);
+  }
+  if (ds.defined()) {
     p.ds_workspace = ds.data_ptr();
     p.ds_workspace_bytes = bytes;
   }

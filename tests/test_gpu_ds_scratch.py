@@ -346,3 +346,38 @@ def test_dense_256_with_and_without_scratch(case):
             assert torch.isfinite(a).all()
             assert (a.float() - b.float()).abs().max() <= 4 * ulp * b.float().abs().max()
     assert torch.equal(unshared[1], recompute[1]) and torch.equal(unshared[2], recompute[2])
+
+
+@pytest.mark.parametrize("head_dim", [128, 256])
+def test_backward_without_room_for_the_scratch(head_dim):
+    """With the device's memory used up but for what the step itself needs,
+    the backward runs without its scratch."""
+    torch.manual_seed(10)
+    dtype, n, heads = torch.float16, 4096, 16  # 512 MiB of dS, 32 MiB a tensor at most
+    q, do, k, v = (_rand((1, heads, n, head_dim), dtype) for _ in range(4))
+    fn = lambda a, b, c: flash_attention(a, b, c, causal=True)
+    want = _grads_at_limit(fn, (q, k, v, do), 0)
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    try:
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (448 << 20)) / total)
+        got = _grads_at_limit(fn, (q, k, v, do), 12 << 30)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+
+
+def test_forward_without_room_for_the_shares():
+    torch.manual_seed(11)
+    q, k, v = (_rand((1, 1, 8192, 512), torch.float16) for _ in range(3))
+    run = lambda: flash_attention(q, k, v)  # 64 MiB of shares' states
+    want = run().float()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    try:
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (40 << 20)) / total)
+        got = run().float()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert (got - want).abs().max() <= 4 * 2.0 ** -11 * want.abs().max()
