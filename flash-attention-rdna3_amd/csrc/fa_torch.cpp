@@ -387,10 +387,48 @@ Tensor decode_workspace(const Tensor& q, int64_t kdim, int64_t num_splits) {
   return at::empty({(int64_t)bytes}, q.options().dtype(at::kByte));
 }
 
-void check_with_query(const Tensor& q, std::initializer_list<const Tensor*> others) {
+// The operators may be called by themselves (torch.ops.fa_mi355x.decode), and
+// the C ABI sees bare pointers: device, type, rank and extent of everything a
+// kernel reads or writes are checked here.
+void check_query_and_caches(const Tensor& q, const Tensor& k, const Tensor& v, bool kv_fp8) {
   TORCH_CHECK(q.is_cuda() && q.dim() == 4, "fa_mi355x: query must be a 4-D GPU tensor");
-  for (const Tensor* t : others)
+  for (const Tensor* t : {&k, &v}) {
     TORCH_CHECK(t->device() == q.device(), "fa_mi355x: all tensors must be on the query's device");
+    TORCH_CHECK(t->dim() == 4 && t->sizes() == k.sizes() && t->size(3) == q.size(3),
+                "fa_mi355x: key and value caches must be 4-D, of one shape and the query's head_dim");
+    TORCH_CHECK(t->scalar_type() == (kv_fp8 ? at::kFloat8_e4m3fn : q.scalar_type()),
+                "fa_mi355x: key and value caches must have the query's dtype (kv_fp8: float8_e4m3fn)");
+  }
+}
+
+void check_int32(const Tensor& t, const Tensor& q, at::IntArrayRef sizes, const char* what) {
+  TORCH_CHECK(t.device() == q.device() && t.scalar_type() == at::kInt && t.sizes() == sizes, "fa_mi355x: ", what,
+              " must be an int32 tensor of shape ", sizes, " on the query's device");
+}
+
+void check_tickets(const OptTensor& tickets, const Tensor& q) {
+  if (!tickets.has_value()) return;
+  const int64_t need = (int64_t)fa_decode_ticket_count((int)q.size(0), (int)q.size(1), (int)q.size(2));
+  TORCH_CHECK(tickets->device() == q.device() && tickets->scalar_type() == at::kInt && tickets->is_contiguous() &&
+                  tickets->numel() >= need,
+              "fa_mi355x: tickets must be at least ", need, " contiguous int32 counters on the query's device");
+}
+
+// New rows are written in place: into the caches as they are, not a copy.
+void check_append(const Tensor& q, const Tensor& k, const Tensor& v, const OptTensor& new_key,
+                  const OptTensor& new_value, const OptTensor& lens, bool kv_fp8) {
+  TORCH_CHECK(new_key.has_value() == new_value.has_value(), "fa_mi355x: new_k and new_v must be given together");
+  if (!new_key.has_value()) return;
+  TORCH_CHECK(lens.has_value() && !kv_fp8, "fa_mi355x: appending needs lens and a 16-bit cache");
+  for (const Tensor* t : {&*new_key, &*new_value})
+    TORCH_CHECK(t->device() == q.device() && t->scalar_type() == q.scalar_type() && t->dim() == 4 &&
+                    t->sizes() == new_key->sizes() && t->size(0) == k.size(0) && t->size(1) == k.size(1) &&
+                    t->size(3) == k.size(3),
+                "fa_mi355x: new_k and new_v must be (batch, heads_kv, rows, head_dim), in the query's dtype and on "
+                "its device");
+  for (const Tensor* t : {&k, &v})
+    TORCH_CHECK(kernel_ready(*t).is_same(*t),
+                "fa_mi355x: a cache that is appended to needs a unit last stride and 16-byte aligned rows");
 }
 
 void append_rows(const Tensor& query, const Tensor& k_cache, const Tensor& v_cache, const Tensor& key,
@@ -421,7 +459,11 @@ void append_rows(const Tensor& query, const Tensor& k_cache, const Tensor& v_cac
 Tensor decode_op(const Tensor& query, const Tensor& key, const Tensor& value, const OptTensor& new_key,
                  const OptTensor& new_value, const OptTensor& lens, bool causal, double scale, int64_t num_splits,
                  bool kv_fp8, double k_scale, double v_scale, const OptTensor& tickets) {
-  check_with_query(query, {&key, &value});
+  check_query_and_caches(query, key, value, kv_fp8);
+  TORCH_CHECK(key.size(0) == query.size(0), "fa_mi355x: caches must have the query's batch");
+  if (lens.has_value()) check_int32(*lens, query, {query.size(0)}, "lens");
+  check_append(query, key, value, new_key, new_value, lens, kv_fp8);
+  check_tickets(tickets, query);
   c10::DeviceGuard guard(query.device());
   const int64_t head_dim = query.size(3), kdim = std::max(kMinKernelHeadDim, head_dim);
   int64_t added = 0;
@@ -474,7 +516,11 @@ Tensor decode_op(const Tensor& query, const Tensor& key, const Tensor& value, co
 Tensor decode_paged_op(const Tensor& query, const Tensor& k_cache, const Tensor& v_cache, const Tensor& block_table,
                        const Tensor& context_lens, bool causal, double scale, int64_t num_splits, bool kv_fp8,
                        double k_scale, double v_scale, const OptTensor& tickets) {
-  check_with_query(query, {&k_cache, &v_cache, &block_table, &context_lens});
+  check_query_and_caches(query, k_cache, v_cache, kv_fp8);
+  TORCH_CHECK(block_table.dim() == 2, "fa_mi355x: block_table must be 2-D");
+  check_int32(block_table, query, {query.size(0), block_table.size(1)}, "block_table");
+  check_int32(context_lens, query, {query.size(0)}, "context_lens");
+  check_tickets(tickets, query);
   c10::DeviceGuard guard(query.device());
   const int64_t head_dim = query.size(3), kdim = std::max(kMinKernelHeadDim, head_dim);
   const Tensor q = kernel_ready(pad_head_dim(query, kdim));
