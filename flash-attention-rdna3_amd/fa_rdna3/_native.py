@@ -207,6 +207,18 @@ def ops():
     return torch.ops.fa_mi355x
 
 
+def run_decode(op, *args):
+    """Call a decode operator.  It has no rule for torch.func transforms, and
+    their wrappers must not reach it: a jvp would come back with a silent zero
+    tangent.  Plain tensors inside a transform are not its business."""
+    if torch._C._functorch.peek_interpreter_stack() is None:
+        return op(*args)
+    if any(isinstance(t, torch.Tensor) and torch._C._functorch.is_functorch_wrapped_tensor(t) for t in args):
+        raise RuntimeError("this decode API does not support torch.func transforms of its arguments")
+    with torch._C._DisableFuncTorch():
+        return op(*args)
+
+
 def _check(rc, what):
     if rc != 0:
         msg = lib().fa_last_error_string().decode(errors="replace")

@@ -1,10 +1,10 @@
 """The decode operators called by themselves check what their kernels read and
-write."""
+write, and decode refuses torch.func transforms of its arguments."""
 
 import pytest
 import torch
 
-from fa_rdna3 import _native, flash_attention_decode_paged, flash_attention_with_kvcache
+from fa_rdna3 import _native, flash_attention_decode, flash_attention_decode_paged, flash_attention_with_kvcache
 
 pytestmark = pytest.mark.gpu
 B, HQ, HKV, ROWS, KEYS, D = 2, 8, 2, 1, 300, 64
@@ -85,3 +85,36 @@ def test_operators_run_with_what_they_ask_for():
     want = flash_attention_decode_paged(args["q"].squeeze(2), args["k_cache"], args["v_cache"], args["block_table"],
                                         args["context_lens"])
     torch.testing.assert_close(_native.ops().decode_paged(**args).squeeze(2), want, rtol=4e-3, atol=4e-3)
+
+
+def _calls():
+    a, p = _decode_args(), _paged_args()
+    return [
+        (lambda q: flash_attention_decode(q, a["k"], a["v"], cache_seqlens=a["lens"]), a["q"]),
+        (lambda q: flash_attention_with_kvcache(q, a["k"], a["v"], a["new_k"], a["new_v"], cache_seqlens=a["lens"]),
+         a["q"]),
+        (lambda q: flash_attention_decode_paged(q, p["k_cache"], p["v_cache"], p["block_table"], p["context_lens"]),
+         p["q"].squeeze(2)),
+    ]
+
+
+@pytest.mark.parametrize("which", range(3))
+def test_transforms_of_the_arguments_are_refused(which):
+    """A jvp used to come back with a zero tangent."""
+    call, q = _calls()[which]
+    with pytest.raises(RuntimeError):
+        torch.func.jvp(call, (q,), (torch.ones_like(q),))
+    with pytest.raises(RuntimeError):
+        torch.vmap(call)(q[None].clone())
+
+
+@pytest.mark.parametrize("which", range(3))
+def test_plain_tensors_inside_a_transform(which):
+    call, q = _calls()[which]
+    want = call(q)
+    if which < 2:  # (one-row paged decode reshapes its query, which jvp wraps)
+        out, tangent = torch.func.jvp(lambda x: call(q).float() * x, (torch.tensor(2.0, device="cuda"),),
+                                      (torch.tensor(1.0, device="cuda"),))
+        assert torch.equal(out, 2 * want.float()) and torch.equal(tangent, want.float())
+    out = torch.vmap(lambda x: call(q).float() * x)(torch.tensor([1.0, 3.0], device="cuda"))
+    assert torch.equal(out[1], 3 * want.float())
