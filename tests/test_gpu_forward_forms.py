@@ -12,10 +12,12 @@ pytestmark = pytest.mark.gpu
 BOUND = {torch.float16: 4 * 2.0 ** -11, torch.bfloat16: 4 * 2.0 ** -8}
 
 
-def _check(out, q, k, v, dtype, rows=slice(None), **opts):
-    ref = attention(q[:1].double(), k[:1].double(), v[:1].double(), **opts)
-    err = (out[:1].double() - ref).norm() / ref.norm()
-    assert torch.isfinite(out).all() and err <= BOUND[dtype], float(err)
+def _check(out, q, k, v, dtype, **opts):
+    ref = attention(q.double(), k.double(), v.double(), **opts)
+    assert torch.isfinite(out).all()
+    for got, want in zip(out, ref):  # each batch entry by itself: its own bias base, form and loads
+        err = (got.double() - want).norm() / want.norm()
+        assert err <= BOUND[dtype], float(err)
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
@@ -58,7 +60,7 @@ def test_bias_layouts(dtype, bias_dtype, layout, sq, sk, head_dim):
     if sk > 8:
         bias[..., -5] = float("-inf")  # one hidden key
     out = flash_attention(q, k, v, bias=bias)
-    _check(out, q, k, v, dtype, bias=bias.expand(2, 3, sq, sk)[:1].double())
+    _check(out, q, k, v, dtype, bias=bias.expand(2, 3, sq, sk).double())
 
 
 @pytest.mark.parametrize("head_dim", [64, 128])
