@@ -29,27 +29,27 @@
 
 namespace fa {
 
-// A workgroup owns BN keys (NK pairs of KB 32-key blocks) and splits their
+// A workgroup owns BN keys (NK pairs of waves, 32 keys each) and splits their
 // query steps in two halves of four waves, as dkdv16_kernel does.  The two
 // waves of a SIMD (w and w + 4) take opposite roles.
 template <int D>
 struct DkdvRolesCfg {
-  static constexpr int KB = D >= 256 ? 1 : 2;  // 32-key blocks per wave
-  static constexpr int NK = 2;                 // wave pairs per half
+  static_assert(D == 256, "dkdv16_kernel holds both sums of the narrower heads in one wave");
+  static constexpr int NK = 2;  // wave pairs per half
   static constexpr int NW = 4 * NK;
   static constexpr int NT = 64 * NW;
   static constexpr int NTH = NT / 2;
-  static constexpr int BN = 32 * KB * NK;
+  static constexpr int BN = 32 * NK;
   static constexpr int BMQ = 32;
   static constexpr int QT = BMQ * D;  // elements per Q / dO tile
   static constexpr int STAGE_BYTES = 2 * QT * 2 + 2 * BMQ * 4;
   static constexpr int HALF_BYTES = 2 * STAGE_BYTES;
-  static constexpr int XCH_FLOATS = KB * 1024;  // one pair's P of a step
+  static constexpr int XCH_FLOATS = 1024;  // one pair's P of a step
   static constexpr int LOOP_BYTES = 2 * HALF_BYTES + 2 * NK * XCH_FLOATS * 4;
   static constexpr int NSTEP = D / 16;
   static constexpr int NPV = BMQ / 16;
   static constexpr int NDB = D / 32;
-  static constexpr int PARK_WAVE_BYTES = KB * NDB * 4096;
+  static constexpr int PARK_WAVE_BYTES = NDB * 4096;
   static constexpr int MERGE_BYTES = 2 * NK * PARK_WAVE_BYTES;
   static constexpr int LDS_BYTES = LOOP_BYTES > MERGE_BYTES ? LOOP_BYTES : MERGE_BYTES;
   static_assert(LDS_BYTES <= 160 * 1024, "one workgroup per CU");
@@ -65,7 +65,6 @@ __global__ __launch_bounds__(512, 1) void dkdv_roles_kernel(fa_bwd_params p, int
   using C = DkdvRolesCfg<D>;
   using EL = Elem<Tag>;
   using S = uint16_t;
-  constexpr int KB = C::KB;
   extern __shared__ __align__(256) unsigned char smem_raw[];
   const fa_fwd_params& f = p.fwd;
 
@@ -95,37 +94,29 @@ __global__ __launch_bounds__(512, 1) void dkdv_roles_kernel(fa_bwd_params p, int
   const int n0 = nblk * C::BN;
   if (n0 >= sk || num_n_blocks <= 0) return;
 
-  const int n0w = n0 + 32 * KB * pair;
-  const int ncols = min(32 * KB, sk - n0w);
+  const int n0w = n0 + 32 * pair;
+  const int ncols = min(32, sk - n0w);
 
   // The resident operands (MFMA B layout): K rows of the V wave, V rows of
   // the K wave; rows past the last key are zero.
-  s16x8 op[KB][C::NSTEP];
+  s16x8 op[C::NSTEP];
   {
     const int64_t st = kwave ? f.v_stride[2] : f.k_stride[2];
     const S* base = kwave ? reinterpret_cast<const S*>(f.v) + b * f.v_stride[0] + hk * f.v_stride[1]
                           : reinterpret_cast<const S*>(f.k) + b * f.k_stride[0] + hk * f.k_stride[1];
+    const S* row = base + (int64_t)(k_start + min(n0w + l32, sk - 1)) * st + 8 * h;
 #pragma unroll
-    for (int kb = 0; kb < KB; ++kb) {
-      const int n = n0w + 32 * kb + l32;
-      const S* row = base + (int64_t)(k_start + min(n, sk - 1)) * st + 8 * h;
-#pragma unroll
-      for (int s = 0; s < C::NSTEP; ++s) op[kb][s] = load_op<Tag>(row + 16 * s);
-    }
+    for (int s = 0; s < C::NSTEP; ++s) op[s] = load_op<Tag>(row + 16 * s);
     wait_vm_all();
+    if (n0w + l32 >= sk) {
 #pragma unroll
-    for (int kb = 0; kb < KB; ++kb)
-      if (n0w + 32 * kb + l32 >= sk) {
-#pragma unroll
-        for (int s = 0; s < C::NSTEP; ++s) op[kb][s] = zero_op<Tag>();
-      }
+      for (int s = 0; s < C::NSTEP; ++s) op[s] = zero_op<Tag>();
+    }
   }
 
-  f32x16 acc[KB][C::NDB];  // dV (V wave) or dK (K wave)
+  f32x16 acc[C::NDB];  // dV (V wave) or dK (K wave)
 #pragma unroll
-  for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-    for (int i = 0; i < C::NDB; ++i) acc[kb][i] = zero16();
+  for (int i = 0; i < C::NDB; ++i) acc[i] = zero16();
 
   DmaLeanTile<C::BMQ, D, C::NTH> qd, gd;
   qd.init(f.q_stride[2], htid);
@@ -137,7 +128,8 @@ __global__ __launch_bounds__(512, 1) void dkdv_roles_kernel(fa_bwd_params p, int
   float* const xch = reinterpret_cast<float*>(smem_raw + 2 * C::HALF_BYTES) + (qhalf * C::NK + pair) * C::XCH_FLOATS;
   const int nlast = min(n0 + C::BN, sk) - 1;
 
-  const int64_t ds_base = p.ds_workspace != nullptr ? ds_seq_base<true>(p, b, sq, sk) : 0;
+  // (dS scratch is for dense problems only at this head dim)
+  const int64_t ds_base = (int64_t)b * f.heads_q * ds_region_elems(sq, sk);
   for (int g = 0; g < group; ++g) {
     const int hq = hk * group + g;
     const Mods md = make_mods(f, b, hq, sq, sk);
@@ -216,8 +208,8 @@ __global__ __launch_bounds__(512, 1) void dkdv_roles_kernel(fa_bwd_params p, int
       const float* L2 = reinterpret_cast<const float*>(base + 2 * C::QT * 2);
       const float* DL = L2 + C::BMQ;
 
-      f32x16 x[KB];               // S then P (V wave), dP then dS (K wave)
-      s16x8 xb[KB][C::NPV];
+      f32x16 x;  // S then P (V wave), dP then dS (K wave)
+      s16x8 xb[C::NPV];
       if (vis) {
         // Both roles: x += tile . resident operand.
         if (kwave && MODE != 2) {
@@ -225,24 +217,19 @@ __global__ __launch_bounds__(512, 1) void dkdv_roles_kernel(fa_bwd_params p, int
           for (int q4 = 0; q4 < 4; ++q4) {
             const f32x4 d = *reinterpret_cast<const f32x4*>(DL + 8 * q4 + 4 * h);
 #pragma unroll
-            for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-              for (int r = 0; r < 4; ++r) x[kb][4 * q4 + r] = d[r];
+            for (int r = 0; r < 4; ++r) x[4 * q4 + r] = d[r];
           }
         } else {
-#pragma unroll
-          for (int kb = 0; kb < KB; ++kb) x[kb] = zero16();
+          x = zero16();
         }
         const uint32_t ra = tile_lane(qtile + (kwave ? C::QT * 2u : 0u), row_off);
 #pragma unroll
         for (int i = 0; i < C::NSTEP; ++i) {
           // k-steps 8 apart share an address (row_op): taken in turn.
-          const int s = C::NSTEP <= 8 ? i : (i >> 1) + 8 * (i & 1);
-          const s16x8 a = row_op<D>(ra, s);
-#pragma unroll
-          for (int kb = 0; kb < KB; ++kb) x[kb] = EL::mma(a, op[kb][s], x[kb]);
+          const int s = (i >> 1) + 8 * (i & 1);
+          x = EL::mma(row_op<D>(ra, s), op[s], x);
         }
-        sched_reads<C::NSTEP, 2, 1, KB>();
+        sched_reads<C::NSTEP, 2, 1, 1>();
         if (!kwave) {
           // P, and what the K wave needs of it: P times the softcap's
           // derivative, negative where dropout dropped the pair.  (All of the
@@ -253,52 +240,49 @@ __global__ __launch_bounds__(512, 1) void dkdv_roles_kernel(fa_bwd_params p, int
           auto scores = [&](auto cap_t, auto bias_t, auto alibi_t, auto mask_t) {
             constexpr bool CAP = decltype(cap_t)::value;
             constexpr bool MASK = decltype(mask_t)::value;
-#pragma unroll
-            for (int kb = 0; kb < KB; ++kb) {
-              Span rs{0, 0};
-              if constexpr (MASK) {
-                int rlo, rhi;
-                row_bounds(md, n0w + 32 * kb + l32, rlo, rhi);
-                rs = make_span(rlo, rhi, m0 + 4 * h);
-              }
-              f32x16 w;
-#pragma unroll
-              for (int q4 = 0; q4 < 4; ++q4) {
-                const f32x4 l2 = *reinterpret_cast<const f32x4*>(L2 + 8 * q4 + 4 * h);
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                  const int i = 4 * q4 + r;
-                  float pv, tc = 0.f, wv;
-                  if constexpr (MODE == 0) {
-                    pv = __builtin_amdgcn_exp2f(__builtin_fmaf(x[kb][i], c, -l2[r]));
-                  } else if constexpr (MODE == 3) {
-                    const float rr = softcap_r(md, x[kb][i]);
-                    pv = __builtin_amdgcn_exp2f(__builtin_fmaf(md.cap2_m2, rr, l2[r]));
-                    tc = __builtin_fmaf(-rr, rr, rr);
-                  } else {
-                    const int m = m0 + acc_row(i, h), n = n0w + 32 * kb + l32;
-                    float sc;
-                    if constexpr (MODE == 2) sc = score<true>(md, x[kb][i], m, n, tc);
-                    else sc = score_m<CAP, decltype(bias_t)::value, decltype(alibi_t)::value>(md, x[kb][i], m, n, tc);
-                    pv = __builtin_amdgcn_exp2f(sc - l2[r]);
-                  }
-                  if constexpr (MASK) pv = in_span(rs, acc_row(i, 0)) ? pv : 0.f;
-                  wv = pv;
-                  if constexpr (MODE == 3) wv *= 4.f * tc;
-                  else if constexpr (CAP) wv *= (1.f - tc * tc);
-                  if constexpr (MODE == 2) {
-                    if (md.drop_p > 0.f) {
-                      const bool keep = dropout_keep(md, m0 + acc_row(i, h), n0w + 32 * kb + l32);
-                      pv = keep ? pv * md.drop_scale : 0.f;
-                      wv = keep ? wv : -wv;
-                    }
-                  }
-                  x[kb][i] = pv;
-                  w[i] = wv;
-                }
-              }
-              park_acc(xch + kb * 1024, lane, w);
+            Span rs{0, 0};
+            if constexpr (MASK) {
+              int rlo, rhi;
+              row_bounds(md, n0w + l32, rlo, rhi);
+              rs = make_span(rlo, rhi, m0 + 4 * h);
             }
+            f32x16 w;
+#pragma unroll
+            for (int q4 = 0; q4 < 4; ++q4) {
+              const f32x4 l2 = *reinterpret_cast<const f32x4*>(L2 + 8 * q4 + 4 * h);
+#pragma unroll
+              for (int r = 0; r < 4; ++r) {
+                const int i = 4 * q4 + r;
+                float pv, tc = 0.f, wv;
+                if constexpr (MODE == 0) {
+                  pv = __builtin_amdgcn_exp2f(__builtin_fmaf(x[i], c, -l2[r]));
+                } else if constexpr (MODE == 3) {
+                  const float rr = softcap_r(md, x[i]);
+                  pv = __builtin_amdgcn_exp2f(__builtin_fmaf(md.cap2_m2, rr, l2[r]));
+                  tc = __builtin_fmaf(-rr, rr, rr);
+                } else {
+                  const int m = m0 + acc_row(i, h), n = n0w + l32;
+                  float sc;
+                  if constexpr (MODE == 2) sc = score<true>(md, x[i], m, n, tc);
+                  else sc = score_m<CAP, decltype(bias_t)::value, decltype(alibi_t)::value>(md, x[i], m, n, tc);
+                  pv = __builtin_amdgcn_exp2f(sc - l2[r]);
+                }
+                if constexpr (MASK) pv = in_span(rs, acc_row(i, 0)) ? pv : 0.f;
+                wv = pv;
+                if constexpr (MODE == 3) wv *= 4.f * tc;
+                else if constexpr (CAP) wv *= (1.f - tc * tc);
+                if constexpr (MODE == 2) {
+                  if (md.drop_p > 0.f) {
+                    const bool keep = dropout_keep(md, m0 + acc_row(i, h), n0w + l32);
+                    pv = keep ? pv * md.drop_scale : 0.f;
+                    wv = keep ? wv : -wv;
+                  }
+                }
+                x[i] = pv;
+                w[i] = wv;
+              }
+            }
+            park_acc(xch, lane, w);
           };
           using T_ = std::true_type;
           using F_ = std::false_type;
@@ -317,47 +301,38 @@ __global__ __launch_bounds__(512, 1) void dkdv_roles_kernel(fa_bwd_params p, int
             else dispatch_mods(md, [&](auto a, auto b_, auto c_) { scores(a, b_, c_, F_{}); });
           }
 #pragma unroll
-          for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-            for (int j = 0; j < C::NPV; ++j) xb[kb][j] = pack_op<Tag>(x[kb], j);
+          for (int j = 0; j < C::NPV; ++j) xb[j] = pack_op<Tag>(x, j);
         }
       }
       __syncthreads();  // P of every pair is in LDS
       if (vis) {
         if (kwave) {
+          const f32x16 w = unpark_acc(xch, lane);
+          if constexpr (MODE == 2) {
 #pragma unroll
-          for (int kb = 0; kb < KB; ++kb) {
-            const f32x16 w = unpark_acc(xch + kb * 1024, lane);
-            if constexpr (MODE == 2) {
+            for (int q4 = 0; q4 < 4; ++q4) {
+              const f32x4 d = *reinterpret_cast<const f32x4*>(DL + 8 * q4 + 4 * h);
 #pragma unroll
-              for (int q4 = 0; q4 < 4; ++q4) {
-                const f32x4 d = *reinterpret_cast<const f32x4*>(DL + 8 * q4 + 4 * h);
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                  const int i = 4 * q4 + r;
-                  const bool keep = !(__float_as_uint(w[i]) >> 31);
-                  const float dp = keep ? x[kb][i] * md.drop_scale : 0.f;
-                  x[kb][i] = fabsf(w[i]) * (dp - d[r]);
-                }
+              for (int r = 0; r < 4; ++r) {
+                const int i = 4 * q4 + r;
+                const bool keep = !(__float_as_uint(w[i]) >> 31);
+                const float dp = keep ? x[i] * md.drop_scale : 0.f;
+                x[i] = fabsf(w[i]) * (dp - d[r]);
               }
-            } else {
-#pragma unroll
-              for (int i = 0; i < 16; ++i) x[kb][i] *= w[i];
             }
+          } else {
 #pragma unroll
-            for (int j = 0; j < C::NPV; ++j) xb[kb][j] = pack_op<Tag>(x[kb], j);
+            for (int i = 0; i < 16; ++i) x[i] *= w[i];
           }
+#pragma unroll
+          for (int j = 0; j < C::NPV; ++j) xb[j] = pack_op<Tag>(x, j);
         }
         const uint32_t ta = tile_lane(qtile + (kwave ? 0u : C::QT * 2u), tr_off);
 #pragma unroll
         for (int j = 0; j < C::NPV; ++j)
 #pragma unroll
-          for (int db = 0; db < C::NDB; ++db) {
-            const s16x8 a = tr_op<D>(ta, j, db);
-#pragma unroll
-            for (int kb = 0; kb < KB; ++kb) acc[kb][db] = EL::mma(a, xb[kb][j], acc[kb][db]);
-          }
-        sched_reads<C::NPV * C::NDB, 2, 2, KB>();
+          for (int db = 0; db < C::NDB; ++db) acc[db] = EL::mma(tr_op<D>(ta, j, db), xb[j], acc[db]);
+        sched_reads<C::NPV * C::NDB, 2, 2, 1>();
       }
       if (t + 1 < my_count) store_stage(st ^ 1, m0 + C::BMQ);
       const bool ds_store = ds_on && vis && kwave;
@@ -365,30 +340,27 @@ __global__ __launch_bounds__(512, 1) void dkdv_roles_kernel(fa_bwd_params p, int
         // As in dkdv16_kernel: one permlane32 swap per dword pair gives each
         // lane 16 consecutive queries of its key, two 16-byte stores.
         static_assert(C::NPV == 2 && C::BMQ == kDsSubQueries, "a query step is one dS sub-tile");
+        u32x4 w0 = __builtin_bit_cast(u32x4, xb[0]), w1 = __builtin_bit_cast(u32x4, xb[1]);
 #pragma unroll
-        for (int kb = 0; kb < KB; ++kb) {
-          u32x4 w0 = __builtin_bit_cast(u32x4, xb[kb][0]), w1 = __builtin_bit_cast(u32x4, xb[kb][1]);
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const auto r = __builtin_amdgcn_permlane32_swap(w0[i], w1[i], false, false);
-            w0[i] = r[0];
-            w1[i] = r[1];
-          }
-          // A buffer window over this wave's rows of the sub-tile: lanes past
-          // the last key fall outside it and store nothing, yet every wave
-          // issues the same stores (the wait below counts them).
-          const int rows = min(32, ncols - 32 * kb);
-          const S* at = dsn + kb * 32 * kDsSubQueries + (int64_t)(m0 / kDsTileQueries) * kDsTileElems +
-                        (m0 % kDsTileQueries) / kDsSubQueries * kDsSubElems;
-          const __amdgpu_buffer_rsrc_t rs = rows_rsrc<kDsSubQueries>(at, kDsSubQueries, rows);
-          const uint32_t o = (uint32_t)(l32 * kDsSubQueries * 2 + 32 * h);
-          __builtin_amdgcn_raw_buffer_store_b128(u32x4{w0[0], w0[1], w1[0], w1[1]}, rs, o, 0, 0);
-          __builtin_amdgcn_raw_buffer_store_b128(u32x4{w0[2], w0[3], w1[2], w1[3]}, rs, o + 16, 0, 0);
+        for (int i = 0; i < 4; ++i) {
+          const auto r = __builtin_amdgcn_permlane32_swap(w0[i], w1[i], false, false);
+          w0[i] = r[0];
+          w1[i] = r[1];
         }
+        // A buffer window over this wave's rows of the sub-tile: lanes past
+        // the last key fall outside it and store nothing, yet every wave
+        // issues the same stores (the wait below counts them).
+        const int rows = min(32, ncols);
+        const S* at = dsn + (int64_t)(m0 / kDsTileQueries) * kDsTileElems +
+                      (m0 % kDsTileQueries) / kDsSubQueries * kDsSubElems;
+        const __amdgpu_buffer_rsrc_t rs = rows_rsrc<kDsSubQueries>(at, kDsSubQueries, rows);
+        const uint32_t o = (uint32_t)(l32 * kDsSubQueries * 2 + 32 * h);
+        __builtin_amdgcn_raw_buffer_store_b128(u32x4{w0[0], w0[1], w1[0], w1[1]}, rs, o, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b128(u32x4{w0[2], w0[3], w1[2], w1[3]}, rs, o + 16, 0, 0);
       }
       // The next stage must have landed; this step's dS stores, issued after
       // its loads, may still be in flight.
-      if (ds_store) wait_vm<2 * KB>();
+      if (ds_store) wait_vm<2>();
       else wait_vm_all();
       __syncthreads();
     }
@@ -397,26 +369,20 @@ __global__ __launch_bounds__(512, 1) void dkdv_roles_kernel(fa_bwd_params p, int
   // First query half + second query half, in that order.
   {
     __syncthreads();
-    float* ow = reinterpret_cast<float*>(smem_raw) + slot * KB * C::NDB * 1024;
+    float* ow = reinterpret_cast<float*>(smem_raw) + slot * C::NDB * 1024;
     if (qhalf == 1) {
 #pragma unroll
-      for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-        for (int db = 0; db < C::NDB; ++db) park_acc(ow + (kb * C::NDB + db) * 1024, lane, acc[kb][db]);
+      for (int db = 0; db < C::NDB; ++db) park_acc(ow + db * 1024, lane, acc[db]);
     }
     __syncthreads();
     if (qhalf == 1) return;
 #pragma unroll
-    for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-      for (int db = 0; db < C::NDB; ++db) acc[kb][db] += unpark_acc(ow + (kb * C::NDB + db) * 1024, lane);
+    for (int db = 0; db < C::NDB; ++db) acc[db] += unpark_acc(ow + db * 1024, lane);
   }
   if (nshare > 1) {
-    float* pw = part + ((int64_t)blockIdx.x * 2 * C::NK + slot) * (KB * C::NDB * 1024);
+    float* pw = part + ((int64_t)blockIdx.x * 2 * C::NK + slot) * (C::NDB * 1024);
 #pragma unroll
-    for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-      for (int db = 0; db < C::NDB; ++db) park_acc(pw + (kb * C::NDB + db) * 1024, lane, acc[kb][db]);
+    for (int db = 0; db < C::NDB; ++db) park_acc(pw + db * 1024, lane, acc[db]);
     return;
   }
   // Whole-row stores through this wave's merge block (read back already).
@@ -425,10 +391,7 @@ __global__ __launch_bounds__(512, 1) void dkdv_roles_kernel(fa_bwd_params p, int
                    : reinterpret_cast<S*>(p.dv) + b * p.dv_stride[0] + hk * p.dv_stride[1];
   const float sc = kwave ? f.softmax_scale : 1.f;
   uint16_t* const stage = reinterpret_cast<uint16_t*>(smem_raw + slot * C::PARK_WAVE_BYTES);
-#pragma unroll
-  for (int kb = 0; kb < KB; ++kb)
-    store_rows_staged<Tag, D>(acc[kb], sc, stage, orow0 + (int64_t)(k_start + n0w + 32 * kb) * ost, ost,
-                              ncols - 32 * kb, lane);
+  store_rows_staged<Tag, D>(acc, sc, stage, orow0 + (int64_t)(k_start + n0w) * ost, ost, ncols, lane);
 }
 
 // dK / dV of the shares above, added in share order: 64 columns of one item
@@ -438,7 +401,7 @@ __global__ __launch_bounds__(256) void dkdv_merge_kernel(fa_bwd_params p, int ns
   using C = DkdvRolesCfg<D>;
   using S = uint16_t;
   constexpr int MD = 64, PER = D / MD;
-  static_assert(C::KB == 1 && 2 * C::NK == 4, "one wave per merge block");
+  static_assert(2 * C::NK == 4, "one wave per merge block");
   __shared__ __align__(16) uint16_t stage[4 * 32 * (MD + 8)];
   const fa_fwd_params& f = p.fwd;
   const int lane = threadIdx.x & 63;

@@ -482,8 +482,7 @@ __global__ __launch_bounds__(256 * NH, D > 128 ? 1 : 3 - NH) void fwd16_kernel(f
 // workgroups (blockIdx = item * nsplit + split).  The shares' states are fp32
 // and unnormalised, so the merge loses nothing against one workgroup.
 template <typename Tag, int D, int MODE>
-__global__ __launch_bounds__(256, D > 128 ? 1 : 2) void fwd16_split_kernel(fa_fwd_params p, int num_m_blocks,
-                                                                           int nsplit, float* ws) {
+__global__ __launch_bounds__(256, 1) void fwd16_split_kernel(fa_fwd_params p, int num_m_blocks, int nsplit, float* ws) {
   extern __shared__ __align__(256) unsigned char smem_raw[];
   const int item = blockIdx.x / nsplit;
   fwd16_item<Tag, D, MODE, 1, false, true>(p, num_m_blocks, item, smem_raw, false, true, blockIdx.x - item * nsplit, nsplit,
