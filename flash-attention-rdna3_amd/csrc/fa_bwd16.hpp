@@ -323,7 +323,9 @@ __global__ __launch_bounds__(512, 1) void dkdv16_kernel(fa_bwd_params p, int num
               if constexpr (MASK) pv = in_span(rs, acc_row(i, 0)) ? pv : 0.f;
             } else {
               const int m = m0 + acc_row(i, h);
-              const float x = score_m<CAP, decltype(bias_t)::value, decltype(alibi_t)::value>(md, sacc[i], m, n, tc);
+              float x;
+              if constexpr (MODE == 2) x = score<true>(md, sacc[i], m, n, tc);
+              else x = score_m<CAP, decltype(bias_t)::value, decltype(alibi_t)::value>(md, sacc[i], m, n, tc);
               // lse2 of this score's row, read here rather than held across
               // the stage (register pressure of the modifier variants).
               const float l2i = L2[8 * (i / 4) + 4 * h + (i % 4)];
@@ -351,7 +353,14 @@ __global__ __launch_bounds__(512, 1) void dkdv16_kernel(fa_bwd_params p, int num
           // softcap only
           if (vis == 1) scores(F_{}, T_{}, std::integral_constant<int, 0>{}, F_{}, T_{});
           else scores(F_{}, T_{}, std::integral_constant<int, 0>{}, F_{}, F_{});
-        } else if constexpr (MODE >= 1) {
+        } else if constexpr (MODE == 2) {
+          // One variant that tests for each modifier (CAP: tc is 0 without a
+          // softcap) and masks: of sixteen, one was a function call with its
+          // operands in scratch, whose time also moved by 8 % with where the
+          // build placed it (bf16 2 x 16 x 2048 x 128 causal step,
+          // dropout: 3118 -> 792 us).
+          scores(F_{}, T_{}, std::integral_constant<int, 0>{}, F_{}, T_{});
+        } else if constexpr (MODE == 1) {
           if (vis == 1) dispatch_mods(md, [&](auto a, auto b_, auto c_) { scores(F_{}, a, b_, c_, T_{}); });
           else dispatch_mods(md, [&](auto a, auto b_, auto c_) { scores(F_{}, a, b_, c_, F_{}); });
         } else {

@@ -53,8 +53,12 @@ def test_kernels_do_not_spill(spills, kernel):
     assert not any(c for c, _ in found.values()), {n: c for n, c in found.items() if c[0]}
 
 
-def test_dropout_at_256_keeps_its_step_loop_in_registers(spills):
-    """The sixteen score variants of this kernel took 576 bytes of scratch a
-    lane, most of it read back in the step loop; one variant takes 168."""
-    found = {n: c for n, c in spills.items() if "dkdv_roles_kernel<" in n and ", 256, 2>" in n}
-    assert len(found) == 2 and all(s <= 256 for _, s in found.values()), found
+@pytest.mark.parametrize("kernel,bytes_per_lane", [
+    (r"dkdv_roles_kernel<.*, 256, 2>", 256), (r"dkdv16_kernel<.*, 128, 2>", 400), (r"dkdv16_kernel<.*, (32|64), 2>", 0),
+])
+def test_dropout_backward_keeps_its_step_loop_in_registers(spills, kernel, bytes_per_lane):
+    """The sixteen score variants of these kernels took 512 to 576 bytes of
+    scratch a lane, most of it read back in the step loop or handed to a
+    function there; one variant takes 168 at D = 256, 328 at 128, else none."""
+    found = {n: c for n, c in spills.items() if re.search(kernel, n)}
+    assert len(found) >= 2 and all(s <= bytes_per_lane for _, s in found.values()), found
