@@ -565,6 +565,20 @@ Tensor decode_paged_op(const Tensor& query, const Tensor& k_cache, const Tensor&
   return kdim != head_dim ? out.narrow(-1, 0, head_dim) : out;
 }
 
+// Inside a torch.func transform.  Decode has no rule for any of them, and a
+// wrapped argument must not reach it: a jvp would come back with a silent zero
+// tangent.  Plain tensors are not the transform's business.
+void decode_in_transform(const c10::OperatorHandle& op, c10::DispatchKeySet, torch::jit::Stack* stack) {
+  const c10::DispatchKeySet wrapped(
+      {c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::Functionalize});
+  for (const c10::IValue& arg : torch::jit::last(*stack, op.schema().arguments().size()))
+    TORCH_CHECK(!arg.isTensor() || !arg.toTensor().key_set().has_any(wrapped), op.schema().name(),
+                " does not support torch.func transforms of its arguments");
+  const c10::impl::ExcludeDispatchKeyGuard guard(c10::DispatchKeySet(
+      {c10::DispatchKey::FuncTorchDynamicLayerFrontMode, c10::DispatchKey::FuncTorchDynamicLayerBackMode}));
+  op.callBoxed(stack);
+}
+
 int64_t set_ds_scratch_limit(int64_t bytes) {
   return g_ds_limit.exchange(bytes < 0 ? 0 : bytes);
 }
@@ -607,6 +621,11 @@ TORCH_LIBRARY_IMPL(fa_mi355x, CUDA, m) {
 TORCH_LIBRARY_IMPL(fa_mi355x, Autograd, m) {
   m.impl("decode", torch::CppFunction::makeFallthrough());
   m.impl("decode_paged", torch::CppFunction::makeFallthrough());
+}
+
+TORCH_LIBRARY_IMPL(fa_mi355x, FuncTorchDynamicLayerFrontMode, m) {
+  m.impl("decode", torch::CppFunction::makeFromBoxedFunction<&decode_in_transform>());
+  m.impl("decode_paged", torch::CppFunction::makeFromBoxedFunction<&decode_in_transform>());
 }
 
 TORCH_LIBRARY_IMPL(fa_mi355x, ADInplaceOrView, m) {

@@ -8,7 +8,6 @@ if the library is missing the import of any compute path fails loudly.
 """
 
 import ctypes
-import functools
 import os
 import threading
 
@@ -206,23 +205,6 @@ def ops():
     the differentiable ``attention``), loaded with the native library."""
     lib()
     return torch.ops.fa_mi355x
-
-
-def decode_operator(name):
-    """The decode operator ``name``.  It has no rule for torch.func transforms,
-    and their wrappers must not reach it: a jvp would come back with a silent
-    zero tangent.  Plain tensors inside a transform are not its business."""
-    op = getattr(ops(), name)
-    if torch._C._functorch.peek_interpreter_stack() is None:
-        return op
-    return functools.partial(_call_in_transform, op)
-
-
-def _call_in_transform(op, *args):
-    if any(isinstance(t, torch.Tensor) and torch._C._functorch.is_functorch_wrapped_tensor(t) for t in args):
-        raise RuntimeError("this decode API does not support torch.func transforms of its arguments")
-    with torch._C._DisableFuncTorch():
-        return op(*args)
 
 
 def _check(rc, what):

@@ -520,9 +520,9 @@ def _decode_launch(query, key, value, softmax_scale, lens, causal, new_rows=(Non
     else:
         num_splits = _decode_num_splits(batch, heads, seqlen_q, seqlen_k, 4 * _cu_count(query.device))
     k_scale, v_scale = fp8_scales if fp8_scales is not None else (1.0, 1.0)
-    decode = _native.decode_operator("decode")
-    return decode(query, key, value, new_rows[0], new_rows[1], lens, causal, softmax_scale, num_splits,
-                  fp8_scales is not None, k_scale, v_scale, _native.decode_tickets(query, batch, heads, seqlen_q))
+    return _native.ops().decode(query, key, value, new_rows[0], new_rows[1], lens, causal, softmax_scale, num_splits,
+                                fp8_scales is not None, k_scale, v_scale,
+                                _native.decode_tickets(query, batch, heads, seqlen_q))
 
 
 def _rows_vector_ready(t):
@@ -777,10 +777,9 @@ def _paged_launch(query, k_cache, v_cache, block_table, context_lens, softmax_sc
                                        2 * _cu_count(query.device), max_context_len=max_context_len,
                                        requested_splits=num_splits))
     k_scale, v_scale = fp8_scales if fp8_scales is not None else (1.0, 1.0)
-    decode_paged = _native.decode_operator("decode_paged")
-    return decode_paged(query, k_cache, v_cache, block_table, context_lens, causal, softmax_scale, splits,
-                        fp8_scales is not None, k_scale, v_scale,
-                        _native.decode_tickets(query, batch, q_heads, seqlen_q))
+    return _native.ops().decode_paged(query, k_cache, v_cache, block_table, context_lens, causal, softmax_scale,
+                                      splits, fp8_scales is not None, k_scale, v_scale,
+                                      _native.decode_tickets(query, batch, q_heads, seqlen_q))
 
 
 def flash_attention_decode_paged_multi(query, k_cache, v_cache, block_table, context_lens, softmax_scale=None,

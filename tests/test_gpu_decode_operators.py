@@ -102,10 +102,12 @@ def _calls():
 def test_transforms_of_the_arguments_are_refused(which):
     """A jvp used to come back with a zero tangent."""
     call, q = _calls()[which]
-    with pytest.raises(RuntimeError):
+    with pytest.raises(RuntimeError, match="torch.func transforms"):
         torch.func.jvp(call, (q,), (torch.ones_like(q),))
-    with pytest.raises(RuntimeError):
+    with pytest.raises(RuntimeError, match="torch.func transforms"):
         torch.vmap(call)(q[None].clone())
+    with pytest.raises(RuntimeError):
+        torch.func.functionalize(call)(q)
 
 
 @pytest.mark.parametrize("which", range(3))
