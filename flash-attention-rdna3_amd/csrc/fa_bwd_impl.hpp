@@ -118,7 +118,7 @@ template <typename Tag, int D, int NH>
 struct DkdvCfg {
   using EL = Elem<Tag>;
   using S = typename EL::S;
-  // fp32 up to D = 64: 64 keys and their query steps split between two halves
+  // NH = 2, fp32 up to D = 64: 64 keys and their query steps split between two halves
   // of two waves (see FwdCfg), partial sums added through LDS.
   static constexpr int NWK = 4 / NH;   // key waves per half
   static constexpr int NW = NWK * NH;
@@ -420,7 +420,7 @@ template <typename Tag, int D, int NH>
 struct DqCfg {
   using EL = Elem<Tag>;
   using S = typename EL::S;
-  // fp32 up to D = 64: 64 rows, key tiles split by parity between two halves
+  // NH = 2, fp32 up to D = 64: 64 rows, key tiles split by parity between two halves
   // of two waves (see FwdCfg).
   static constexpr int NWR = 4 / NH;
   static constexpr int NW = NWR * NH;

@@ -17,10 +17,15 @@
 // registers are full, so whatever lives across the step loop is kept small
 // (row_op / tr_op / DmaLeanTile addresses, LDS reads two MFMAs ahead, dS
 // stores by buffer window): a reload from scratch inside the loop waits for
-// the next stage's loads too, and cost 25 us of the figure below.
-// Measured at 1 x 16/8 x 2048 x 256 bf16 causal (69 GFLOP): 148 us with the
-// dS stores, against 920 us for bwd_dkdv_kernel; dQ from that dS 47 us against
-// 453 us for bwd_dq_kernel.
+// the next stage's loads too.  The plain form has none there; softcap, the
+// variants for bias and ALiBi and dropout keep 18, 79 and 49 registers in
+// scratch, some of them read back in the loop.
+// Measured at 1 x 16/8 x 2048 x 256 bf16 causal (69 GFLOP): 102 us with the
+// dS stores in two shares and 14 for their merge, against 920 us for
+// bwd_dkdv_kernel; dQ from that dS 47 us against 453 us for bwd_dq_kernel.
+// Without a mask (103 GFLOP), bwd_dkdv_kernel and this: plain 1012 and 157,
+// softcap 1142 and 222, ALiBi 1141 and 285, a bf16 bias 1704 and 415, dropout
+// 1534 and 448.
 #pragma once
 
 #include <type_traits>

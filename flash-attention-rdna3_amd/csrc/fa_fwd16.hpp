@@ -32,10 +32,12 @@ namespace fa {
 // a heavy causal block runs at full CU throughput instead of sharing the CU
 // with a light one and then running alone.
 //
-// D > 128 runs NH = 1 only, one workgroup per CU: O^T, Q and the scores of 32
-// rows take up to 400 registers, so a SIMD holds one wave.  What bounds it is
-// LDS operand reads, one per MFMA as in the narrower forms, and the softmax
-// that no second wave covers.
+// D > 128 runs NH = 1 only, planned for one workgroup per CU (the launch bound
+// allows 512 registers; share counts assume one).  O^T, Q and the scores of 32
+// rows take 248 to 288 registers at D = 256, so that only the forms of at most
+// 256 can share a SIMD, and 315 to 352 at D = 512.  What bounds it is LDS
+// operand reads, one per MFMA as in the narrower forms, and the softmax that
+// no second wave covers.
 //
 // NH = 1 is the same kernel with one key half: 4 waves walk all key tiles of
 // the 128 rows and no merge is needed.  Its 64 KiB of LDS and 4 waves let two
@@ -43,8 +45,8 @@ namespace fa {
 // epilogue (output store) overlap the other's steady state.  It is launched
 // for packed varlen batches, for causal grids of many rounds of workgroups,
 // where that per-workgroup cost adds up, and for blocks of equal cost that
-// outnumber the CUs; a short causal batch keeps NH = 2, whose key split lets
-// a heavy block use the whole CU.
+// outnumber the CUs (D = 32: twice); a short causal batch keeps NH = 2, whose
+// key split lets a heavy block use the whole CU (run_fwd has the lines).
 template <int D, int NH = 2>
 struct Fwd16Cfg {
   static constexpr int NQ = 4;                 // row quarters (waves per half)

@@ -34,13 +34,14 @@ template <typename Tag, int D, int NH>
 struct FwdCfg {
   using EL = Elem<Tag>;
   using S = typename EL::S;
-  // fp32 up to D = 128: 64 query rows (two waves) and their key tiles split
-  // by parity between two halves of two waves, merged through LDS.  A wave is
+  // NH = 2, fp32 up to D = 128: 64 query rows (two waves) and their key tiles
+  // split by parity between two halves of two waves, merged through LDS.  A wave is
   // MFMA-bound (64 cycles for 32x32x2), so what counts is that there are
   // enough of them: 1 x 16 x 1000 rows in blocks of 128 left half the CUs
   // idle.  At D = 64 the forward takes 61 us there against 100 us, dK/dV 119
   // against 203, dQ 86 against 135 (the operands of four MFMAs in one LDS
   // read, kslot, included); 4.1 / 8.2 / 6.1 GFLOP, card 153 TFLOP/s in fp32.
+  // f32_halves says which grids take it.
   static constexpr int NWR = 4 / NH;          // row waves per half
   static constexpr int NW = NWR * NH;
   static constexpr int NT = 64 * NW;
@@ -355,10 +356,9 @@ static hipError_t launch_fwd_generic(const fa_fwd_params& p, hipStream_t stream)
 template <typename Tag, int D, int MODE>
 static hipError_t run_fwd(const fa_fwd_params& p, const FwdScratch& scratch, hipStream_t stream) {
   if constexpr (!std::is_same<Tag, f32_t>::value && D > 128) {
-    // Wide heads: one wave per SIMD with all 512 registers (O^T of 32 rows
-    // takes 128 of them, Q 64 to 128; at two waves per SIMD the D = 256 form
-    // spilled 38), one key half.  Measured against fwd_kernel (O^T split two
-    // to four ways over the grid, scores recomputed for each):
+    // Wide heads: up to 512 registers a wave (O^T of 32 rows takes 128 of
+    // them, Q 64 to 128), one key half.  Measured against fwd_kernel (O^T
+    // split two to four ways over the grid, scores recomputed for each):
     // D = 256 bf16 causal, 1 x 16 x 2048 (34 GFLOP): 207 -> 115 us;
     // D = 512 fp16, 1 x 1 x 4096 (34 GFLOP), with key splits: 787 -> 92 us
     // (shares 79, merge 13; 52 GFLOP with the scores of both column halves).

@@ -337,8 +337,12 @@ int fa_bwd_phase(const fa_bwd_params* params, int phase, void* stream);
  * does not apply: fp32, head_dim other than 64, 128 or (dense) 256, or more
  * than 512 varlen sequences).
  * Dense: batch * heads_q * ceil(Sk / 64) * ceil(Sq / 128) * 16 KiB plus
- * 1 KiB; varlen, an upper bound from max_seqlen_k, total_q and batch.  With dS scratch, phase 2 of
- * fa_bwd_phase reads the dS that phase 1 stored. */
+ * 1 KiB; varlen, an upper bound from max_seqlen_k, total_q and batch.  At
+ * head_dim 256, where the key blocks leave compute units idle (it depends on
+ * the current device's count), 128 KiB more per 64 keys of each KV head and
+ * share of their query rows: call this function rather than compute the size.
+ * Scratch that holds the dS alone runs the dS path without shares.  With dS
+ * scratch, phase 2 of fa_bwd_phase reads the dS that phase 1 stored. */
 size_t fa_bwd_workspace_bytes(const fa_bwd_params* params);
 /* No counterpart in the reference.  The smallest ds_workspace fa_bwd uses
  * the dS path with: for a problem it chunks, the dS of ceil(heads_kv / 2)
@@ -346,8 +350,9 @@ size_t fa_bwd_workspace_bytes(const fa_bwd_params* params);
  * runs dK/dV and dQ once per half of the KV heads.  It chunks only when
  * each half holds at least 1 GiB of dS and the problem has no bias, ALiBi
  * or dropout (their head index would shift); smaller or more chunks measured
- * slower than recomputing dQ.  Otherwise equal to fa_bwd_workspace_bytes
- * (0 when the dS path does not apply).  fa_bwd_phase uses the dS path only
+ * slower than recomputing dQ.  Otherwise the dS alone, without shares: equal
+ * to fa_bwd_workspace_bytes but at head_dim 256 (0 when the dS path does not
+ * apply).  fa_bwd_phase uses the dS path only
  * with the full fa_bwd_workspace_bytes. */
 size_t fa_bwd_workspace_min_bytes(const fa_bwd_params* params);
 /* uint32 counters `tickets` needs: batch * heads_q * seqlen_q. */
