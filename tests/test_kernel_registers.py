@@ -62,3 +62,12 @@ def test_dropout_backward_keeps_its_step_loop_in_registers(spills, kernel, bytes
     function there; one variant takes 168 at D = 256, 328 at 128, else none."""
     found = {n: c for n, c in spills.items() if re.search(kernel, n)}
     assert len(found) >= 2 and all(s <= bytes_per_lane for _, s in found.values()), found
+
+
+@pytest.mark.parametrize("kernel,bytes_per_lane", [(r"dq16_kernel<.*, 128, 1>", 64), (r"dq16_kernel<.*, (32|64), 1>", 0),
+                                                   (r"dq16_kernel<.*, (32|64|128), (0|3)>", 64)])
+def test_recomputing_dq_is_part_of_its_kernel(spills, kernel, bytes_per_lane):
+    """As a function of its own the block took 628 bytes of scratch a lane at
+    D = 128 with modifiers; inlined it takes 20."""
+    found = {n: c for n, c in spills.items() if re.search(kernel, n)}
+    assert len(found) >= 2 and all(s <= bytes_per_lane for _, s in found.values()), found
