@@ -485,7 +485,7 @@ struct Dq16Cfg {
 // query head) bh; fuse_delta computes delta here. Inlined by force: as a call
 // (dq16_kernel has two) the modifier forms kept 628 bytes a lane in scratch at
 // D = 128, and a causal ALiBi step without stored dS (2 x 16 x 2048 x 128)
-// took 285 us (bf16) and 295 (fp16) against 257 and 262 inlined.
+// took 285 us (fp16) and 299 (bf16) against 250 and 255 inlined.
 template <typename Tag, int D, int MODE>
 __device__ __forceinline__ void dq16_block(const fa_bwd_params& p, int num_m_blocks, int mb_rev, int bh, int fuse_delta) {
   using C = Dq16Cfg<D>;
